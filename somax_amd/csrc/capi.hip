@@ -192,7 +192,50 @@ struct Batch {
   int any_mass = 0;
   float* homsol = nullptr;
   double* hmean = nullptr;
+  // direct FP64 inversion (null: it does not pay, or a mixed ensemble class,
+  // which only ever takes SSP-RK3 steps)
+  struct DirectDelete {
+    void operator()(Direct* d) const { direct_destroy(d); }
+  };
+  std::unique_ptr<Direct, DirectDelete> direct;
 };
+
+// What an inversion is for decides its form (`use_direct`).
+enum class Solve {
+  STEP,   // a stage of an SSP-RK3 step
+  STATE,  // psi itself, a Tsit5 stage, a projection
+  FIELD,  // derivatives of psi are the result (tendency, diagnostics)
+};
+
+// Whether an inversion of batch `p` runs in its direct form: wherever the
+// batch has one (direct_pays), except
+//   * SSP-RK3 steps of the mixed form.  Ensembles take those in merged launch
+//     groups whose phases are the split-operand transforms, and a member's
+//     step equals its single model's bit for bit, so both keep them;
+//   * results that are derivatives of psi.  They carry psi's last bits
+//     amplified (1e-5 in a tendency, 1e-3 in a vorticity at 512^2), so any
+//     other order of sums moves them by that much; they keep the arithmetic
+//     that their stored references were made with.
+inline bool use_direct(const Batch& p, Solve what) {
+  return p.direct && what != Solve::FIELD && !(what == Solve::STEP && p.precision == SOMAXHIP_PREC_MIXED);
+}
+
+// Whether the direct FP64 form is the faster inversion of P planes: the grid
+// has to fit, and its operations F (four products of the folded transforms)
+// have to stay below what the split-operand launches do in the time they take
+// at least.  Those cost 4 launches of one round of tiles each, whatever the
+// number of planes, until the tiles fill the chip; the direct form runs at the
+// FP64 rate from the start.  Measured (an SSP-RK3 step of 3-layer members, us,
+// split -> direct): FP32 64^2 x 4 265 -> 114, 128^2 x 64 634 -> 483, 256^2 x 8
+// 410 -> 330, 256^2 x 32 (F = 6.6e9) 939 -> 960, 512^2 x 2 (3.3e9) 516 -> 471,
+// 512^2 x 4 (6.5e9) 575 -> 772; six products 256^2 x 8 (1.65e9) 363 -> 332,
+// 512^2 x 1 (1.63e9) 345 -> 314, 512^2 x 2 369 -> 472.
+static bool direct_pays(int Nx, int Ny, int P, int precision) {
+  if (!direct_fits(Nx, Ny)) return false;
+  const double hx = (Nx + 1) / 2, hy = (Ny + 1) / 2;
+  const double F = 16.0 * P * hx * hy * (hx + hy);
+  return F <= (precision == SOMAXHIP_PREC_BF16X6 ? 1.8e9 : 4.0e9);
+}
 
 // Checks one model description; empty string when valid.
 static std::string check_desc(const somaxhip_qg_desc* d, bool allow_f64) {
@@ -219,7 +262,8 @@ static bool same_class(const somaxhip_qg_desc* a, const somaxhip_qg_desc* b) {
 }
 
 // Builds batch `b` from M descriptions of one class (validated by the caller).
-static hipError_t batch_build(Batch& b, const std::vector<const somaxhip_qg_desc*>& ds) {
+// `ensemble`: a class of an ensemble rather than a single model.
+static hipError_t batch_build(Batch& b, const std::vector<const somaxhip_qg_desc*>& ds, bool ensemble) {
   const somaxhip_qg_desc* d0 = ds[0];
   b.nx = d0->nx;
   b.ny = d0->ny;
@@ -292,6 +336,25 @@ static hipError_t batch_build(Batch& b, const std::vector<const somaxhip_qg_desc
       (e = b.mem.upload(&dhp, hp)) != hipSuccess || (e = b.mem.upload(&dws, wscale)) != hipSuccess ||
       (e = b.mem.upload(&b.dbeta_rows, dbeta)) != hipSuccess || (e = b.mem.upload(&b.wind_rows, wind)) != hipSuccess)
     return e;
+  if (direct_pays(b.Nx, b.Ny, P, b.precision) && !(ensemble && b.precision == SOMAXHIP_PREC_MIXED)) {
+    DirectDesc dd;
+    dd.Nx = b.Nx;
+    dd.Ny = b.Ny;
+    dd.dx = b.dx;
+    dd.dy = b.dy;
+    dd.nl = mnl;
+    dd.mask = mask;
+    dd.cl2m = cl2m;
+    dd.cm2l.assign((size_t)b.M * 64, 0.0);
+    for (int m = 0; m < b.M; ++m) {
+      const somaxhip_qg_desc* d = ds[m];
+      for (int i = 0; i < d->nl; ++i)
+        for (int k = 0; k < d->nl; ++k) dd.cm2l[(size_t)m * 64 + i * MAX_LAYERS + k] = d->cm2l[i * d->nl + k];
+      dd.lam.insert(dd.lam.end(), d->lambdas, d->lambdas + d->nl);
+    }
+    b.direct.reset(direct_create(dd, &e));
+    if (!b.direct) return e;
+  }
   b.t = Tables{dfirst, dnl, dcl2m, dcm2l, dmask, dmember, dlayer, dlam, dhp, dws, nullptr};
 
   // mass correction: homogeneous solution and its mean per plane
@@ -328,6 +391,8 @@ static hipError_t batch_build(Batch& b, const std::vector<const somaxhip_qg_desc
   b.off_OP2 = take((size_t)opl * 3 * b.wpiece * sizeof(uint16_t));
   b.off_QM = take((size_t)P * b.splane * sizeof(float));
   b.off_P0 = take((size_t)P * b.splane * sizeof(float));
+  // the direct form's scratch starts at OP1 and takes the room of these four
+  if (b.direct && off - b.off_OP1 < direct_bytes(b.Nx, b.Ny, P)) take(direct_bytes(b.Nx, b.Ny, P) - (off - b.off_OP1));
   if (b.precision == SOMAXHIP_PREC_MIXED) b.off_D = take((size_t)P * b.splane * sizeof(float));
   b.off_Q1 = take((size_t)P * b.splane * sizeof(float));
   b.off_Q2 = take((size_t)P * b.splane * sizeof(float));
@@ -497,7 +562,7 @@ int somaxhip_qg_plan_create(const somaxhip_qg_desc* d, somaxhip_qg_plan* out) {
     *out = p;
     return SOMAXHIP_OK;
   }
-  const hipError_t e = batch_build(p->b, {d});
+  const hipError_t e = batch_build(p->b, {d}, false);
   if (e != hipSuccess) {
     set_error(std::string("somaxhip_qg_plan_create: ") + hipGetErrorString(e));
     delete p;
@@ -893,7 +958,37 @@ void mass_layer_args(const Batch& p, LayerArgs& la, const PlaneSumArgs& ps, void
   la.psi_wall = wsf(ws, p.off_PWALL);
 }
 
-void invert(const Batch& p, const float* q, float* psi, void* ws, hipStream_t st, bool apply_bc = true) {
+DirectCall direct_call(const Batch& p, const float* q, float* psi, void* ws, bool apply_bc) {
+  DirectCall c{};
+  c.d = p.direct.get();
+  c.q = q;
+  c.psi = psi;
+  c.apply_bc = apply_bc;
+  c.buf = static_cast<char*>(ws) + p.off_OP1;
+  if (p.any_mass) {
+    c.homsol = p.homsol;
+    c.hmean = p.hmean;
+    c.psi_wall = wsf(ws, p.off_PWALL);
+  }
+  return c;
+}
+
+// Phases of the direct inversion as the profile names them; `folded` is the
+// number of points of all planes, mults the products of one 1-D transform.
+DirectPhase direct_phases(double points, double mults, hipStream_t st) {
+  return [=](int k, const std::function<void()>& launch) {
+    static const char* const names[3] = {"direct_forward", "direct_spectral", "direct_inverse"};
+    ProfScope ps(names[k], 2.0 * mults * (k == 1 ? 2.0 : 1.0), (k == 1 ? 16.0 : 12.0) * points, st);
+    launch();
+  };
+}
+double direct_mults(const Batch& p) { return (double)p.P * p.splane * 0.25 * (p.Nx + p.Ny); }  // mean of x and y, folded
+
+void invert(const Batch& p, Solve what, const float* q, float* psi, void* ws, hipStream_t st, bool apply_bc = true) {
+  if (use_direct(p, what)) {
+    launch_direct(direct_call(p, q, psi, ws, apply_bc), st, direct_phases((double)p.P * p.splane, direct_mults(p), st));
+    return;
+  }
   const bool mixed = p.precision == SOMAXHIP_PREC_MIXED;
   const bool x6 = p.precision == SOMAXHIP_PREC_BF16X6;
   float* P0 = wsf(ws, p.off_P0);
@@ -953,6 +1048,16 @@ void invert_group(const std::vector<GroupItem>& it, hipStream_t st) {
   const bool x6 = prec == SOMAXHIP_PREC_BF16X6;
   double bytes = 0.0;
   for (const GroupItem& g : it) bytes += (double)g.b->P * g.b->splane;
+  if (use_direct(*it[0].b, Solve::STEP)) {  // (a group is direct as a whole)
+    DirectCall c[MAX_GROUP];
+    double mults = 0.0;
+    for (int i = 0; i < n; ++i) {
+      c[i] = direct_call(*it[i].b, it[i].q, it[i].psi, it[i].ws, true);
+      mults += direct_mults(*it[i].b);
+    }
+    launch_direct_group(c, n, st, direct_phases(bytes, mults, st));
+    return;
+  }
   {
     ModalArgs ma[MAX_GROUP];
     for (int i = 0; i < n; ++i) ma[i] = modal_args(*it[i].b, it[i].q, it[i].ws, true);
@@ -1073,11 +1178,11 @@ void rk3(const Batch& p, float* q, float* psi_last, int nsteps, double dt, const
   float* q2 = wsf(ws, p.off_Q2);
   const float h = (float)dt;
   for (int n = 0; n < nsteps; ++n) {
-    invert(p, q, psi, ws, st);
+    invert(p, Solve::STEP, q, psi, ws, st);
     stage(p, q, psi, nullptr, q1, cp, 1.0f, h, true, ws, st);
-    invert(p, q1, psi, ws, st);
+    invert(p, Solve::STEP, q1, psi, ws, st);
     stage(p, q1, psi, q, q2, cp, 0.25f, 0.25f * h, true, ws, st);
-    invert(p, q2, psi, ws, st);
+    invert(p, Solve::STEP, q2, psi, ws, st);
     stage(p, q2, psi, q, q, cp, 2.0f / 3.0f, 2.0f / 3.0f * h, true, ws, st);
   }
 }
@@ -1135,7 +1240,7 @@ void tsit5(const Batch& p, float* q, int nsteps, double dt, const CallParams& cp
   float* K[7];
   for (int i = 0; i < 7; ++i) K[i] = Y + (i + 1) * n;
   auto f = [&](const float* y, float* k) {
-    invert(p, y, psi, ws, st);
+    invert(p, Solve::STATE, y, psi, ws, st);
     stage(p, y, psi, nullptr, k, cp, 0.0f, 1.0f, true, ws, st);
   };
   if (nsteps > 0) f(q, K[0]);
@@ -1214,7 +1319,7 @@ int somaxhip_qg_invert(somaxhip_qg_plan p, const float* q, float* psi, int apply
   int rc = check_call(p, q, psi, ws, "somaxhip_qg_invert");
   if (rc) return rc;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  invert(p->b, q, psi, ws, st, apply_bc != 0);
+  invert(p->b, Solve::STATE, q, psi, ws, st, apply_bc != 0);
   SOMAX_HIP_CHECK(hipGetLastError());
   return SOMAXHIP_OK;
 }
@@ -1229,7 +1334,7 @@ int somaxhip_qg_rhs(somaxhip_qg_plan p, const float* q, float* dq, float* psi_ou
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   float* psi = psi_out ? psi_out : wsf(ws, p->b.off_PSI);
-  invert(p->b, q, psi, ws, st, apply_bc != 0);
+  invert(p->b, Solve::FIELD, q, psi, ws, st, apply_bc != 0);
   stage(p->b, q, psi, nullptr, dq, uniform_params(prm), 0.0f, 1.0f, apply_bc != 0, ws, st);
   SOMAX_HIP_CHECK(hipGetLastError());
   return SOMAXHIP_OK;
@@ -1312,7 +1417,7 @@ int somaxhip_qg_project(somaxhip_qg_plan p, double f0, const double* H, const do
   }
   a.hdev = h_deviation ? 1 : 0;
   launch_project_pv(a, st);
-  invert(b, a.q, const_cast<float*>(a.psi), ws, st, false);
+  invert(b, Solve::STATE, a.q, const_cast<float*>(a.psi), ws, st, false);
   launch_project_geo(a, st);
   SOMAX_HIP_CHECK(hipGetLastError());
   return SOMAXHIP_OK;
@@ -1347,7 +1452,7 @@ int somaxhip_qg_diagnose(somaxhip_qg_plan p, const float* q, float* psi, float* 
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const Batch& b = p->b;
-  invert(b, q, psi, ws, st, false);
+  invert(b, Solve::FIELD, q, psi, ws, st, false);
   QGDiagArgs a{};
   a.q = q;
   a.psi = psi;
@@ -1457,7 +1562,7 @@ int somaxhip_ens_create(const somaxhip_qg_desc* members, const somaxhip_qg_param
       set_error("somaxhip_ens_create: out of host memory");
       return SOMAXHIP_ERR_ALLOC;
     }
-    hipError_t e = batch_build(*b, ds);
+    hipError_t e = batch_build(*b, ds, true);
     MemberParams* dp = nullptr;
     std::vector<MemberParams> hp;
     int biharm = 0;
@@ -1576,7 +1681,7 @@ int somaxhip_ens_set_stage_rows(somaxhip_ens e, int cls, int rows) {
 namespace {
 
 // Launch groups of a merged ensemble: classes in order, each joining the
-// first group with the same precision, advection, biharmonic flag and (for
+// first group with the same precision, inversion form, advection, biharmonic flag and (for
 // the Arakawa stage) tile height that still has room.
 std::vector<std::vector<int>> ens_groups(somaxhip_ens e) {
   std::vector<std::vector<int>> groups;
@@ -1584,6 +1689,7 @@ std::vector<std::vector<int>> ens_groups(somaxhip_ens e) {
     const Batch& x = *e->cls[a];
     const Batch& y = *e->cls[b];
     return x.precision == y.precision && x.advection == y.advection && e->cbiharm[a] == e->cbiharm[b] &&
+           !x.direct == !y.direct &&
            (x.advection == 1 || x.stage_rows == y.stage_rows);
   };
   for (int c = 0; c < (int)e->cls.size(); ++c) {

@@ -6,6 +6,9 @@
 // the member and plane tables below.  A single model is the one-member batch.
 #pragma once
 
+#include <functional>
+#include <vector>
+
 #include "somaxhip.h"
 #include "common.h"
 
@@ -421,5 +424,43 @@ PlaneSumArgs plane_sums_args(const float* a, const float* b, int Nx, int Ny, int
 int launch_plane_sums(const float* a, const float* b, int Nx, int Ny, int P, long plane, double* partial,
                       hipStream_t st);  // returns the partials per plane (at most 64)
 void launch_plane_sums_group(const PlaneSumArgs* a, int n, hipStream_t st);
+
+}  // namespace somax
+
+namespace somax {
+
+// Direct FP64 inversion of one batch (direct.hip): psi = Cm2l (lap_h -
+// lambda)^-1 Cl2m q with every sum and intermediate in FP64, three launches.
+// Folded extents up to DIRECT_MAX_H: the forward kernel's four parity rows
+// (64 rows of LDS, one double per folded point) end at 157 KiB of the 160.
+constexpr int DIRECT_MAX_H = 304;
+struct Direct;
+struct DirectDesc {
+  int Nx, Ny;
+  double dx, dy;
+  std::vector<int> nl;              // layers per member
+  std::vector<unsigned char> mask;  // per member: ghost ring of psi set to 0
+  std::vector<double> cl2m, cm2l;   // [M][8][8]
+  std::vector<double> lam;          // per plane
+};
+bool direct_fits(int Nx, int Ny);
+size_t direct_bytes(int Nx, int Ny, int P);  // scratch of one inversion
+Direct* direct_create(const DirectDesc& s, hipError_t* err);
+void direct_destroy(Direct* d);
+struct DirectCall {
+  const Direct* d;
+  const void* q;  // float planes (double: f64)
+  void* psi;
+  bool f64, apply_bc;
+  void* buf;           // direct_bytes()
+  const void* homsol;  // mass correction (null: none), in the state's type
+  const double* hmean;
+  float* psi_wall;     // nullable: wall psi per plane
+  double* alpha;       // nullable: multiplier per plane
+};
+// phase(k, launch) calls launch() for kernel k of the three (timing hooks).
+using DirectPhase = std::function<void(int, const std::function<void()>&)>;
+void launch_direct(const DirectCall& c, hipStream_t st, const DirectPhase& phase);
+void launch_direct_group(const DirectCall* c, int n, hipStream_t st, const DirectPhase& phase);  // n <= MAX_GROUP
 
 }  // namespace somax

@@ -7,11 +7,11 @@
 // SOMAXHIP_PREC_FP64, selects it.  Its kernels are written for exactness
 // first (this form serves the small FP64 double gyre):
 //   * layer <-> mode projections, one thread per cell and all layers;
-//   * the DST-I Helmholtz solve as four batched FP64 GEMMs per inversion
-//     (F S_x, S_y (.), S_y F S_x / (Lam_y + Lam_x - lambda), and back): on
-//     FP64 MFMA one wave per 16 x 16 tile up to 256 x 256, LDS-tiled FMAs
-//     beyond; the sine matrices built on the host with the angle reduced
-//     exactly in integers first;
+//   * the inversion in the direct form (direct.hip) up to its largest grid,
+//     beyond it the DST-I Helmholtz solve as four batched LDS-tiled FP64 GEMMs
+//     (F S_x, S_y (.), S_y F S_x / (Lam_y + Lam_x - lambda), and back), the
+//     sine matrices built on the host with the angle reduced exactly in
+//     integers first;
 //   * the mass constraint's means as fixed-order block reductions;
 //   * one stage kernel per RK stage: Arakawa Jacobian or WENO-Z flux form,
 //     wind, bottom drag, harmonic and biharmonic viscosity and the stage
@@ -40,7 +40,7 @@ struct Qg64 {
   long plane = 0;
   double dx = 0.0, dy = 0.0;
   int advection = 0, zero_psi_ghost = 0, mass = 0;
-  int direct = 0;  // one layer, identity projections, no mass constraint: the transforms read q and write psi
+  Direct* direct = nullptr;  // the inversion in three launches (null: the grid is too large for it)
   std::vector<void*> mem;
   // device tables
   double *sx = nullptr, *sy = nullptr;      // orthonormal DST-I matrices, Nx x Nx and Ny x Ny
@@ -52,6 +52,7 @@ struct Qg64 {
   size_t off_A = 0, off_B = 0, off_PSI = 0, off_Q1 = 0, off_Q2 = 0, off_ALPHA = 0, ws_bytes = 0;
   ~Qg64() {
     for (void* p : mem) (void)hipFree(p);
+    if (direct) direct_destroy(direct);
   }
   template <class T>
   hipError_t upload(T** out, const std::vector<T>& v) {
@@ -87,8 +88,6 @@ struct Gemm64 {
   const double* ly;
   const double* lx;
   const double* lam;
-  int a_ring;  // read the outer ring of A (rows 0, M-1; columns 0, K-1) as 0
-  int c_ring;  // write 0 on the outer ring of C (rows 0, M-1; columns 0, N-1)
 };
 
 // 64 x 64 output tile per workgroup of 256 threads, each thread 4 x 4
@@ -111,8 +110,7 @@ __global__ __launch_bounds__(256) void gemm64_kernel(Gemm64 g) {
     for (int e = threadIdx.x; e < TILE * KT; e += 256) {
       const int r = e / KT, k = e % KT;
       const int gr = row0 + r, gk = k0 + k;
-      const bool ring = g.a_ring && (gr == 0 || gr == g.M - 1 || gk == 0 || gk == g.K - 1);
-      As[k][r] = (gr < g.M && gk < g.K && !ring) ? A[(long)gr * g.lda + gk] : 0.0;
+      As[k][r] = (gr < g.M && gk < g.K) ? A[(long)gr * g.lda + gk] : 0.0;
     }
     for (int e = threadIdx.x; e < KT * TILE; e += 256) {
       const int k = e / TILE, c = e % TILE;
@@ -145,64 +143,8 @@ __global__ __launch_bounds__(256) void gemm64_kernel(Gemm64 g) {
       if (col >= g.N) continue;
       double v = acc[i][j];
       if (g.ly) v = v / ((g.ly[row] + g.lx[col]) - g.lam[b]);
-      if (g.c_ring && (row == 0 || row == g.M - 1 || col == 0 || col == g.N - 1)) v = 0.0;
       C[(long)row * g.ldc + col] = v;
     }
-  }
-}
-
-typedef double double4m __attribute__((ext_vector_type(4)));
-
-// Small transforms (M, N <= 256): one wave per 16 x 16 output tile on FP64
-// MFMA (v_mfma_f64_16x16x4f64, lane l holds A[l % 16][l / 16] and
-// B[l / 16][l % 16] of each k-step of 4; the result row l / 16 + 4 r, column
-// l % 16), the operands read from global memory (they stay in L2 at these
-// sizes) GK k-steps ahead of the MFMAs.
-constexpr int GK = 8;
-constexpr int GEMM64_MFMA_MAX = 256;
-__global__ __launch_bounds__(256) void gemm64_mfma_kernel(Gemm64 g) {
-  const int tn = (g.N + 15) / 16, tiles = ((g.M + 15) / 16) * tn;
-  const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wave >= tiles) return;
-  const int lane = threadIdx.x & 63, b = blockIdx.y;
-  const int i0 = (wave / tn) * 16, j0 = (wave % tn) * 16;
-  const double* A = g.A + b * g.sA;
-  const double* B = g.B + b * g.sB;
-  const int ai = i0 + (lane & 15), bj = j0 + (lane & 15), kq = lane >> 4;
-  const bool arow = ai < g.M, bcol = bj < g.N;
-  const int nks = (g.K + 3) / 4;  // k-steps
-  double xa[GK], xb[GK], ya[GK], yb[GK];
-  auto load = [&](int s0, double (&pa)[GK], double (&pb)[GK]) {
-#pragma unroll
-    for (int t = 0; t < GK; ++t) {
-      const int k = (s0 + t) * 4 + kq;
-      const bool ring = g.a_ring && (ai == 0 || ai == g.M - 1 || k == 0 || k == g.K - 1);
-      pa[t] = (arow && k < g.K && !ring) ? A[(long)ai * g.lda + k] : 0.0;
-      pb[t] = (bcol && k < g.K) ? B[(long)k * g.ldb + bj] : 0.0;
-    }
-  };
-  double4m acc = {0.0, 0.0, 0.0, 0.0};
-  load(0, xa, xb);
-  for (int s0 = 0; s0 < nks; s0 += GK) {
-    if (s0 + GK < nks) load(s0 + GK, ya, yb);
-#pragma unroll
-    for (int t = 0; t < GK; ++t) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[t], xb[t], acc, 0, 0, 0);
-#pragma unroll
-    for (int t = 0; t < GK; ++t) {
-      xa[t] = ya[t];
-      xb[t] = yb[t];
-    }
-  }
-  if (!bcol) return;
-  double* C = g.C + b * g.sC;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = i0 + kq + 4 * r;
-    if (row >= g.M) continue;
-    double v = acc[r];
-    if (g.ly) v = v / ((g.ly[row] + g.lx[bj]) - g.lam[b]);
-    if (g.c_ring && (row == 0 || row == g.M - 1 || bj == 0 || bj == g.N - 1)) v = 0.0;
-    C[(long)row * g.ldc + bj] = v;
   }
 }
 
@@ -518,11 +460,6 @@ inline unsigned blocks(long n) { return (unsigned)((n + 255) / 256); }
 inline double* wsd(void* ws, size_t off) { return reinterpret_cast<double*>(static_cast<char*>(ws) + off); }
 
 void gemm(const Gemm64& g, int batch, hipStream_t st) {
-  if (g.M <= GEMM64_MFMA_MAX && g.N <= GEMM64_MFMA_MAX) {
-    const int tiles = ((g.M + 15) / 16) * ((g.N + 15) / 16);
-    gemm64_mfma_kernel<<<dim3((tiles + 3) / 4, batch), 256, 0, st>>>(g);
-    return;
-  }
   const dim3 grid((g.N + TILE - 1) / TILE, (g.M + TILE - 1) / TILE, batch);
   gemm64_kernel<<<grid, 256, 0, st>>>(g);
 }
@@ -549,16 +486,19 @@ void invert(const Qg64& p, const double* q, double* psi, void* ws, bool apply_bc
   double* B = wsd(ws, p.off_B);
   double* alpha = wsd(ws, p.off_ALPHA);
   if (p.direct) {
-    // the projections are identities: bc(q) enters the first transform (its
-    // ring read as 0) and the last one writes psi (its ring 0 when masked)
-    const int Nx = p.Nx, Ny = p.Ny;
-    const long pl = p.plane;
-    gemm(Gemm64{q, pl, Nx, p.sx, 0, Nx, B, pl, Nx, Ny, Nx, Nx, nullptr, nullptr, nullptr, apply_bc ? 1 : 0, 0}, 1,
-         st);
-    gemm(Gemm64{p.sy, 0, Ny, B, pl, Nx, A, pl, Nx, Ny, Nx, Ny, p.lamy, p.lamx, p.lambdas, 0, 0}, 1, st);
-    gemm(Gemm64{A, pl, Nx, p.sx, 0, Nx, B, pl, Nx, Ny, Nx, Nx, nullptr, nullptr, nullptr, 0, 0}, 1, st);
-    gemm(Gemm64{p.sy, 0, Ny, B, pl, Nx, psi, pl, Nx, Ny, Nx, Ny, nullptr, nullptr, nullptr, 0, p.zero_psi_ghost}, 1,
-         st);
+    DirectCall c{};
+    c.d = p.direct;
+    c.q = q;
+    c.psi = psi;
+    c.f64 = true;
+    c.apply_bc = apply_bc;
+    c.buf = A;
+    if (p.mass) {
+      c.homsol = p.homsol;
+      c.hmean = p.hmean;
+      c.alpha = alpha;
+    }
+    launch_direct(c, st, [](int, const std::function<void()>& launch) { launch(); });
     return;
   }
   const unsigned nb = blocks(p.plane);
@@ -709,8 +649,11 @@ Qg64* qg64_create(const somaxhip_qg_desc* d, std::string* err) {
   std::vector<double> lam(d->lambdas, d->lambdas + nl), ws(d->wind_scale, d->wind_scale + nl);
   std::vector<double> beta(d->beta_y_row, d->beta_y_row + p->Ny), wind(d->wind_row, d->wind_row + p->Ny);
   hipError_t e;
-  if ((e = p->upload(&p->sx, sine_matrix(p->Nx))) != hipSuccess ||
-      (e = p->upload(&p->sy, sine_matrix(p->Ny))) != hipSuccess ||
+  // the dense sine matrices serve the grids without the direct form, and the
+  // homogeneous solutions below
+  const bool dense = p->mass || !direct_fits(p->Nx, p->Ny);
+  if ((dense && (e = p->upload(&p->sx, sine_matrix(p->Nx))) != hipSuccess) ||
+      (dense && (e = p->upload(&p->sy, sine_matrix(p->Ny))) != hipSuccess) ||
       (e = p->upload(&p->lamx, sine_eigenvalues(p->Nx, p->dx))) != hipSuccess ||
       (e = p->upload(&p->lamy, sine_eigenvalues(p->Ny, p->dy))) != hipSuccess ||
       (e = p->upload(&p->cl2m, cl2m)) != hipSuccess || (e = p->upload(&p->cm2l, cm2l)) != hipSuccess ||
@@ -726,14 +669,37 @@ Qg64* qg64_create(const somaxhip_qg_desc* d, std::string* err) {
     off += (size_t)round_up((long)bytes, 256);
     return o;
   };
+  if (direct_fits(p->Nx, p->Ny)) {
+    DirectDesc dd;
+    dd.Nx = p->Nx;
+    dd.Ny = p->Ny;
+    dd.dx = p->dx;
+    dd.dy = p->dy;
+    dd.nl = {nl};
+    dd.mask = {(unsigned char)p->zero_psi_ghost};
+    dd.cl2m.assign(64, 0.0);
+    dd.cm2l.assign(64, 0.0);
+    for (int i = 0; i < nl; ++i)
+      for (int k = 0; k < nl; ++k) {
+        dd.cl2m[i * MAX_LAYERS + k] = cl2m[i * nl + k];
+        dd.cm2l[i * MAX_LAYERS + k] = cm2l[i * nl + k];
+      }
+    dd.lam = lam;
+    p->direct = direct_create(dd, &e);
+    if (!p->direct) {
+      *err = hipGetErrorString(e);
+      return nullptr;
+    }
+  }
   p->off_A = take(fields);
   p->off_B = take(fields);
+  // the direct form's scratch takes the room of A and B
+  if (p->direct && off < direct_bytes(p->Nx, p->Ny, nl)) take(direct_bytes(p->Nx, p->Ny, nl) - off);
   p->off_PSI = take(fields);
   p->off_Q1 = take(fields);
   p->off_Q2 = take(fields);
   p->off_ALPHA = take((size_t)MAX_LAYERS * sizeof(double));
   p->ws_bytes = off;
-  p->direct = nl == 1 && !p->mass && cl2m[0] == 1.0 && cm2l[0] == 1.0;
   if (p->mass) {
     // homogeneous solutions h_m = 1 + (nabla^2 - lambda_m)^-1 [lambda_m], solved
     // here by the same FP64 transforms; their means come from the description

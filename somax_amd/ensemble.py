@@ -7,7 +7,8 @@ counts and parameters -- steps as one ensemble: members sharing a grid,
 advection and precision form a class whose planes every kernel of the step
 covers in one launch; classes run concurrently on their own streams, and the
 step is captured as a hipGraph and replayed.  The arithmetic per member is
-that of ``model.step``.
+that of ``model.step`` (FP32 and six-product classes of so many planes that
+their inversion leaves the direct FP64 form round differently, at 1e-8).
 
 With ``merged=True`` the classes are packed into launch groups (those
 sharing precision, advection, biharmonic flag and stage tile height, up to
