@@ -188,6 +188,7 @@ struct Batch {
   size_t off_PWALL = 0;  // per-plane wall psi
   size_t ws_bytes = 0;
   int stage_rows = 16;  // Arakawa stage tile height (8 or 16), chosen per class
+  bool alone = true;    // false: a class of a concurrent ensemble, whose launches share the chip
   // mass correction: homogeneous solutions (P planes) and their means (0: none)
   int any_mass = 0;
   float* homsol = nullptr;
@@ -672,6 +673,7 @@ void dst_solve_folded(const Batch& p, bool interior_input, int np_fwd, int np_in
     const long var = s.frows * s.fld;
     g.ldx = p.wpitch;
     g.xrows = xrows;
+    g.alone = p.alone ? 1 : 0;
     g.K = K;
     if (f32) {
       g.Xf = reinterpret_cast<const float*>(X);
@@ -789,6 +791,7 @@ void dst_solve(const Batch& p, bool interior_input, int np_fwd, int np_inv_lo, i
                   int np_hi) {
     g.ldx = p.wpitch;
     g.xrows = xrows;
+    g.alone = p.alone ? 1 : 0;
     g.K = K;
     if (f32) {
       g.Xf = reinterpret_cast<const float*>(X);
@@ -1563,6 +1566,7 @@ int somaxhip_ens_create(const somaxhip_qg_desc* members, const somaxhip_qg_param
       return SOMAXHIP_ERR_ALLOC;
     }
     hipError_t e = batch_build(*b, ds, true);
+    b->alone = C == 1 || !(flags & SOMAXHIP_ENS_CONCURRENT) || (flags & SOMAXHIP_ENS_MERGED);
     MemberParams* dp = nullptr;
     std::vector<MemberParams> hp;
     int biharm = 0;

@@ -20,10 +20,12 @@
 //
 // Block tile 128x128 of 32x32 MFMA tiles: 16 waves (4x4) of 32x32 for the
 // x1 / x3 instances, 8 waves (2x4) of 64x32 for x6, 4 waves (2x2) of 64x64
-// for FP32.  Grids are 1-D
-// and remapped so that each XCD works on a contiguous run of tiles (shared
+// for FP32; 64x64 of four 32x32 waves for launches of few tiles, 128x64 for
+// launches of more than a round (pick_tiles), every output's chain of products
+// the same in all of them.  Grids are 1-D and remapped so that each XCD works on a contiguous run of tiles (shared
 // operand rows in its L2).
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -97,12 +99,12 @@ __device__ inline float prefetch_spectral(const GemmArgs& a, const Spectral& sp,
   return 0.0f;
 }
 
-// WN: waves along N; BW: columns of the tile (128, or 64 for the pair tiles).
-template <bool SUM64, int TM, int TN, int WN = 4 / TN, int BW = 128>
+// WN: waves along N; BW, BH: columns and rows of the tile (64 or 128).
+template <bool SUM64, int TM, int TN, int WN = 4 / TN, int BW = 128, int BH = 128>
 __device__ inline void store_tile(const GemmArgs& a, long z, int a0, int b0, const floatx16 (&acc)[TM][TN],
                                   const double (&sum)[TM][TN][16], int opieces, float* stage, const Spectral& sp,
                                   const float* lam = nullptr) {
-  constexpr int WM = 4 / TM, NT = 64 * WM * WN;  // waves along M, threads
+  constexpr int WM = BH / 32 / TM, NT = 64 * WM * WN;  // waves along M, threads
   constexpr int TPR = BW / 8;                    // threads per row of 8-column vectors
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -110,7 +112,7 @@ __device__ inline void store_tile(const GemmArgs& a, long z, int a0, int b0, con
   const int wm = wave / WN, wn = wave % WN;
   const float lamz = sp.lamz;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < BH / 64; ++h) {
     __syncthreads();  // the LDS is free (pipeline drained / previous half stored)
     if ((wm * 32 * TM) / 64 == h) {  // this wave's rows lie in half h
       const int lr0 = (wm * 32 * TM) & 63;
@@ -296,6 +298,64 @@ __device__ void gemm_fringe(const GemmArgs& a, long z, int part, const GemmCut& 
     }
   };
 
+  const int per = (dots + fpw - 1) / fpw;
+  const int d0 = part * per;
+  const int d1 = d0 + per < dots ? d0 + per : dots;
+  // this lane group's two dots of the pass from `base`
+  const char* vrow[2];
+  long vpiece[2];
+  int fixi[2], rr[2], cc[2];
+  bool live[2];
+  auto choose = [&](int base) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int d = base + G * h + g;
+      live[h] = d < d1;
+      int r = 0, c = 0, f = 0;
+      bool var_is_b = true;
+      if (live[h]) {
+        if (d < nrow) {
+          const int q = (unsigned)d / (unsigned)a.RB;
+          r = cut.am + q;
+          c = d - q * a.RB;
+          f = r - cut.am;
+        } else {
+          const int e = d - nrow;
+          const int q = fb == 1 ? e : e >> 1;  // fb is 1 or 2
+          r = q;
+          c = cut.bm + (e - q * fb);
+          f = fa + c - cut.bm;
+          var_is_b = false;
+        }
+      }
+      rr[h] = r;
+      cc[h] = c;
+      fixi[h] = f;
+      vrow[h] = var_is_b ? row_of(false, c, vpiece[h]) : row_of(true, r, vpiece[h]);
+    }
+  };
+  u32x4 raw[2][KB][NV];  // KB chunks of both variable rows
+  auto fetch = [&](int kb) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < KB; ++j) {
+        const int k0 = kb + 64 * j + l8 * 8;
+#pragma unroll
+        for (int w = 0; w < NV; ++w) {
+          const char* src = vrow[h] + (long)k0 * esz + (F32 ? 16 * w : w * vpiece[h] * esz);
+          raw[h][j][w] = (live[h] && k0 < a.K) ? *reinterpret_cast<const u32x4*>(src) : u32x4{0u, 0u, 0u, 0u};
+        }
+      }
+  };
+  // the first variable rows, before anything waits (the kernels of more waves
+  // have no registers to hold them through the staging)
+  constexpr bool EARLY = NT == 256;
+  if constexpr (EARLY) {
+    choose(d0);
+    fetch(0);
+  }
+
   // zero padding first (stores need no wait): rows [am, RA), and every row
   // when the columns have a fringe; 32 lanes per row, columns RB + lane
   {
@@ -333,54 +393,11 @@ __device__ void gemm_fringe(const GemmArgs& a, long z, int part, const GemmCut& 
   }
   __syncthreads();
 
-  const int per = (dots + fpw - 1) / fpw;
-  const int d0 = part * per;
-  const int d1 = d0 + per < dots ? d0 + per : dots;
   for (int base = d0; base < d1; base += 2 * G) {
-    const char* vrow[2];
-    long vpiece[2];
-    int fixi[2], rr[2], cc[2];
-    bool live[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int d = base + G * h + g;
-      live[h] = d < d1;
-      int r = 0, c = 0, f = 0;
-      bool var_is_b = true;
-      if (live[h]) {
-        if (d < nrow) {
-          const int q = (unsigned)d / (unsigned)a.RB;
-          r = cut.am + q;
-          c = d - q * a.RB;
-          f = r - cut.am;
-        } else {
-          const int e = d - nrow;
-          const int q = fb == 1 ? e : e >> 1;  // fb is 1 or 2
-          r = q;
-          c = cut.bm + (e - q * fb);
-          f = fa + c - cut.bm;
-          var_is_b = false;
-        }
-      }
-      rr[h] = r;
-      cc[h] = c;
-      fixi[h] = f;
-      vrow[h] = var_is_b ? row_of(false, c, vpiece[h]) : row_of(true, r, vpiece[h]);
-    }
+    if (!EARLY || base != d0) choose(base);
     acc_t acc[2] = {(acc_t)0, (acc_t)0};
     for (int kb = 0; kb < a.K; kb += 64 * KB) {
-      u32x4 raw[2][KB][NV];
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < KB; ++j) {
-          const int k0 = kb + 64 * j + l8 * 8;
-#pragma unroll
-          for (int w = 0; w < NV; ++w) {
-            const char* src = vrow[h] + (long)k0 * esz + (F32 ? 16 * w : w * vpiece[h] * esz);
-            raw[h][j][w] = (live[h] && k0 < a.K) ? *reinterpret_cast<const u32x4*>(src) : u32x4{0u, 0u, 0u, 0u};
-          }
-        }
+      if (!EARLY || base != d0 || kb != 0) fetch(kb);
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -396,16 +413,18 @@ __device__ void gemm_fringe(const GemmArgs& a, long z, int part, const GemmCut& 
               v[4 + e] = (acc_t)__builtin_bit_cast(float, u1);
             }
           } else {
+            auto lo = [](uint32_t u) { return __builtin_bit_cast(float, u << 16); };
+            auto hi = [](uint32_t u) { return __builtin_bit_cast(float, u & 0xffff0000u); };
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = (acc_t)0;
+            for (int e = 0; e < 4; ++e) {
+              v[2 * e] = (acc_t)lo(raw[h][j][0][e]);
+              v[2 * e + 1] = (acc_t)hi(raw[h][j][0][e]);
 #pragma unroll
-            for (int w = 0; w < NV; ++w)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const uint32_t u = raw[h][j][w][e];
-                v[2 * e] += (acc_t)__builtin_bit_cast(float, u << 16);
-                v[2 * e + 1] += (acc_t)__builtin_bit_cast(float, u & 0xffff0000u);
+              for (int w = 1; w < NV; ++w) {
+                v[2 * e] += (acc_t)lo(raw[h][j][w][e]);
+                v[2 * e + 1] += (acc_t)hi(raw[h][j][w][e]);
               }
+            }
           }
           const acc_t* fx = fix + fixi[h] * K8 + k0;
 #pragma unroll
@@ -456,17 +475,21 @@ __device__ inline int swz(int r) { return ((r >> 1) ^ (r >> 2)) & 3; }
 
 // k-tile stages in LDS per operand piece count (1, 2 or 3 bf16 pieces).  Five
 // stages for two pieces (160 KiB) and eight for one were measured no faster.
-__host__ __device__ constexpr int bf16_nstage(int npc) { return npc == 3 ? 3 : 4; }
+// The 64 x 64 tiles have half the bytes a stage; they take 64, 64 and 72 KiB, so
+// that two workgroups share a CU.
+__host__ __device__ constexpr int bf16_nstage(int npc, int bt) {
+  return bt == 64 ? (npc == 1 ? 8 : (npc == 2 ? 4 : 3)) : (npc == 3 ? 3 : 4);
+}
 
-template <int NPROD, int TM, int TN>
+template <int NPROD, int TM, int TN, int BT>
 struct Bf16Cfg {
   static constexpr int NPC = NPROD == 1 ? 1 : (NPROD == 3 ? 2 : 3);
-  static constexpr int NSTAGE = bf16_nstage(NPC);
-  static constexpr int TILE = 128 * 32;         // bf16 elements per operand piece
+  static constexpr int NSTAGE = bf16_nstage(NPC, BT);
+  static constexpr int TILE = BT * 32;          // bf16 elements per operand piece
   static constexpr int STAGE = 2 * NPC * TILE;  // A pieces then B pieces
-  static constexpr int NWAVES = (4 / TM) * (4 / TN);
+  static constexpr int NWAVES = (BT / 32 / TM) * (BT / 32 / TN);
   static constexpr int OPW = NWAVES >= 16 ? 1 : 2;           // operands each wave loads
-  static constexpr int RPT = 16 / (NWAVES * OPW);            // 16-row blocks per operand piece
+  static constexpr int RPT = BT / 8 / (NWAVES * OPW);        // 16-row blocks per operand piece
   static constexpr int LPT = OPW * NPC * RPT;                // global_load_lds per thread per k-tile
   static constexpr int FLUSH = 2;               // k-tiles between FP64 flushes
 };
@@ -490,14 +513,14 @@ __device__ inline void wait_later(int later) {
   }
 }
 
-template <int NPROD, bool ACC64, int TM, int TN>
+template <int NPROD, bool ACC64, int TM, int TN, int BT>
 __device__ inline void bf16_mainloop(const GemmArgs& a, const uint16_t* S, uint16_t* lds, long z, int a0, int b0,
                                      bool x_in_a, floatx16 (&acc)[TM][TN], double (&sum)[TM][TN][16]) {
-  using C = Bf16Cfg<NPROD, TM, TN>;
+  using C = Bf16Cfg<NPROD, TM, TN, BT>;
   constexpr int NPC = C::NPC;
   constexpr int RPT = C::RPT;
   constexpr int OPW = C::OPW;
-  constexpr int WN = 4 / TN;
+  constexpr int WN = BT / 32 / TN;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -590,7 +613,7 @@ __device__ inline void bf16_mainloop(const GemmArgs& a, const uint16_t* S, uint1
   // until the MFMA starts and serialise LDS latency with MFMA execution).
   // (Two sets when two waves share a SIMD and three-piece fragments would not
   // fit: the other wave covers the read-after-MFMA wait.)
-  constexpr int NS = (TN == 1 && NPC == 3) ? 2 : 4;
+  constexpr int NS = (BT == 128 && TN == 1 && NPC == 3) ? 2 : 4;
   bf16x8 fsa[NS][3][TM], fsb[NS][3][TN];
   auto& fa0 = fsa[0];
   auto& fb0 = fsb[0];
@@ -787,9 +810,9 @@ __device__ inline void bf16_mainloop_pair(const GemmArgs& a, const uint16_t* S, 
 
 }  // namespace
 
-size_t dst_gemm_lds_bytes(int max_np) {
+size_t dst_gemm_lds_bytes(int max_np, int bt) {
   const int npc = max_np == 1 ? 1 : (max_np == 3 ? 2 : 3);
-  return (size_t)bf16_nstage(npc) * 2 * npc * 128 * 32 * sizeof(uint16_t);
+  return (size_t)bf16_nstage(npc, bt) * 2 * npc * bt * 32 * sizeof(uint16_t);
 }
 size_t dst_gemm_pair_lds_bytes(int max_np) {
   const int npc = max_np == 1 ? 1 : 2;
@@ -801,20 +824,20 @@ size_t dst_gemm_pair_lds_bytes(int max_np) {
 // registers).  Several waves per SIMD let one wave's MFMAs overlap another's
 // LDS traffic: 8 waves are 23-33% faster than 4 at the same tile, and 16 a
 // further 12-20% on the many small tiles of ensemble grids.
-template <int NPMAX>
+template <int NPMAX, int BT>
 struct KernelShape {
-  static constexpr int TM = NPMAX == 6 ? 2 : 1;
+  static constexpr int TM = BT == 128 && NPMAX == 6 ? 2 : 1;
   static constexpr int TN = 1;
-  static constexpr int NT = 64 * (4 / TM) * (4 / TN);
-  static constexpr int WPE = NT / 256;  // waves per SIMD
+  static constexpr int NT = 64 * (BT / 32 / TM) * (BT / 32 / TN);
+  static constexpr int WPE = BT == 64 ? 2 : NT / 256;  // waves per SIMD
 };
 
 // One instantiation per largest product count of a launch (x1, x3, x6), so
 // each is a kernel symbol of its own; planes may use fewer products.
-// The tile count of a transform (its fringe workgroups follow).
-__device__ inline int gemm_tiles(const GemmArgs& a) {
-  const GemmCut cut = gemm_cut(a.RA, a.RB, a.K);
-  return ((cut.am + BM - 1) / BM) * ((cut.bm + BN - 1) / BN) * a.nplanes;
+// The tile count of a transform on bm x bn tiles (its fringe workgroups follow).
+__device__ inline int gemm_tiles(const GemmArgs& a, int bm, int bn) {
+  const GemmCut cut = a.cut;
+  return ((cut.am + bm - 1) / bm) * ((cut.bm + bn - 1) / bn) * a.nplanes;
 }
 
 // Transforms of one launch: G == 1 for a single transform, else up to
@@ -827,32 +850,32 @@ struct GemmTable {
   BlockTable t;
   GemmArgs a[G];
 };
-template <int G>
+template <int G, int BMT, int BNT>
 __device__ inline int gemm_block(const GemmTable<G>& g, int& c) {
   if (G == 1) {
     c = 0;
-    const int T = gemm_tiles(g.a[0]);
+    const int T = gemm_tiles(g.a[0], BMT, BNT);
     const int b = blockIdx.x;
     return b < T ? remap_tiles(b, T) : b;
   }
   int l;
   if (!table_class(g.t, blockIdx.x, c, l)) return -1;  // padding between transforms
-  const int T = gemm_tiles(g.a[c]);
+  const int T = gemm_tiles(g.a[c], BMT, BNT);
   return l < T ? remap_tiles(l, T) : l;
 }
 
-template <int NPMAX, int G>
-__global__ __launch_bounds__(KernelShape<NPMAX>::NT)
-__attribute__((amdgpu_waves_per_eu(KernelShape<NPMAX>::WPE, KernelShape<NPMAX>::WPE)))
+template <int NPMAX, int G, int BT>
+__global__ __launch_bounds__((KernelShape<NPMAX, BT>::NT))
+__attribute__((amdgpu_waves_per_eu(KernelShape<NPMAX, BT>::WPE, KernelShape<NPMAX, BT>::WPE)))
 void dst_gemm_bf16_kernel(GemmTable<G> g) {
-  constexpr int TM = KernelShape<NPMAX>::TM, TN = KernelShape<NPMAX>::TN, NT = KernelShape<NPMAX>::NT;
+  constexpr int TM = KernelShape<NPMAX, BT>::TM, TN = KernelShape<NPMAX, BT>::TN, NT = KernelShape<NPMAX, BT>::NT;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds16[];
   int c;
-  const int lb = gemm_block<G>(g, c);
+  const int lb = gemm_block<G, BT, BT>(g, c);
   if (lb < 0) return;
   const GemmArgs& a = g.a[c];
-  const GemmCut cut = gemm_cut(a.RA, a.RB, a.K);
-  const int GA = (cut.am + BM - 1) / BM, GB = (cut.bm + BN - 1) / BN;
+  const GemmCut cut = a.cut;
+  const int GA = (cut.am + BT - 1) / BT, GB = (cut.bm + BT - 1) / BT;
   const int T = GA * GB * a.nplanes;
   const bool fringe = lb >= T;
   int zi, ta = 0, tb = 0, part = 0;
@@ -868,13 +891,13 @@ void dst_gemm_bf16_kernel(GemmTable<G> g) {
   const int np = lo ? a.np_lo : a.np_hi;
   const int opieces = lo ? a.op_lo : a.op_hi;
   if (fringe) {
-    if (NPMAX == 1 || np == 1) gemm_fringe<false, 1, NT>(a, z, part, cut, ps, opieces, lds16);
-    else if (NPMAX == 3 || np == 3) gemm_fringe<false, 2, NT>(a, z, part, cut, ps, opieces, lds16);
-    else gemm_fringe<false, 3, NT>(a, z, part, cut, ps, opieces, lds16);
+    if (NPMAX == 1 || np == 1) gemm_fringe<false, 1, NT, BT == 64 ? 9 : 0>(a, z, part, cut, ps, opieces, lds16);
+    else if (NPMAX == 3 || np == 3) gemm_fringe<false, 2, NT, BT == 64 ? 9 : 0>(a, z, part, cut, ps, opieces, lds16);
+    else gemm_fringe<false, 3, NT, BT == 64 ? 5 : 0>(a, z, part, cut, ps, opieces, lds16);
     return;
   }
-  const int a0 = ta * BM;
-  const int b0 = tb * BN;
+  const int a0 = ta * BT;
+  const int b0 = tb * BT;
   const bool x_in_a = !a.trans;
   const uint16_t* S = a.Sb + ps.s_off;
 
@@ -887,49 +910,31 @@ void dst_gemm_bf16_kernel(GemmTable<G> g) {
   zero_acc<TM, TN>(acc, sum);
   // FP32 accumulation over K ~ 1e3 costs ~2e-7 relative, far below the
   // 3-product split error (~1e-5): only 6-product planes accumulate in FP64.
-  if (NPMAX == 1 || np == 1) bf16_mainloop<1, false, TM, TN>(a, S, lds16, z, a0, b0, x_in_a, acc, sum);
-  else if (NPMAX == 3 || np == 3) bf16_mainloop<3, false, TM, TN>(a, S, lds16, z, a0, b0, x_in_a, acc, sum);
-  else if (a.acc64) bf16_mainloop<6, true, TM, TN>(a, S, lds16, z, a0, b0, x_in_a, acc, sum);
-  else bf16_mainloop<6, false, TM, TN>(a, S, lds16, z, a0, b0, x_in_a, acc, sum);
+  if (NPMAX == 1 || np == 1) bf16_mainloop<1, false, TM, TN, BT>(a, S, lds16, z, a0, b0, x_in_a, acc, sum);
+  else if (NPMAX == 3 || np == 3) bf16_mainloop<3, false, TM, TN, BT>(a, S, lds16, z, a0, b0, x_in_a, acc, sum);
+  else if (a.acc64) bf16_mainloop<6, true, TM, TN, BT>(a, S, lds16, z, a0, b0, x_in_a, acc, sum);
+  else bf16_mainloop<6, false, TM, TN, BT>(a, S, lds16, z, a0, b0, x_in_a, acc, sum);
   float* stage = reinterpret_cast<float*>(lds16);
   if (spectral && threadIdx.x < 256) lam_tile[threadIdx.x] = lam_pre;  // read after store_tile's first barrier
   const float* lam = spectral ? lam_tile : nullptr;
-  if (NPMAX == 6 && np == 6 && a.acc64) store_tile<true, TM, TN>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam);
-  else store_tile<false, TM, TN>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam);
+  if (NPMAX == 6 && np == 6 && a.acc64) store_tile<true, TM, TN, BT / 32 / TN, BT, BT>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam);
+  else store_tile<false, TM, TN, BT / 32 / TN, BT, BT>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam);
 }
 
 
 // Pair-tile instance of the x1 / x3 transforms: tiles of 128 x 64, two
 // workgroups per CU (see bf16_mainloop_pair); the fringe as in the other
 // instances.
-__device__ inline int gemm_tiles_pair(const GemmArgs& a) {
-  const GemmCut cut = gemm_cut(a.RA, a.RB, a.K);
-  return ((cut.am + BM - 1) / BM) * ((cut.bm + BNP - 1) / BNP) * a.nplanes;
-}
-template <int G>
-__device__ inline int gemm_block_pair(const GemmTable<G>& g, int& c) {
-  if (G == 1) {
-    c = 0;
-    const int T = gemm_tiles_pair(g.a[0]);
-    const int b = blockIdx.x;
-    return b < T ? remap_tiles(b, T) : b;
-  }
-  int l;
-  if (!table_class(g.t, blockIdx.x, c, l)) return -1;  // padding between transforms
-  const int T = gemm_tiles_pair(g.a[c]);
-  return l < T ? remap_tiles(l, T) : l;
-}
-
 template <int NPMAX, int G>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void dst_gemm_bf16_pair_kernel(GemmTable<G> g) {
   static_assert(NPMAX == 1 || NPMAX == 3, "pair tiles serve the x1 and x3 transforms");
   extern __shared__ __attribute__((aligned(16))) uint16_t lds16[];
   int c;
-  const int lb = gemm_block_pair<G>(g, c);
+  const int lb = gemm_block<G, BM, BNP>(g, c);
   if (lb < 0) return;
   const GemmArgs& a = g.a[c];
-  const GemmCut cut = gemm_cut(a.RA, a.RB, a.K);
+  const GemmCut cut = a.cut;
   const int GA = (cut.am + BM - 1) / BM, GB = (cut.bm + BNP - 1) / BNP;
   const int T = GA * GB * a.nplanes;
   const bool fringe = lb >= T;
@@ -977,10 +982,10 @@ template <int G>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void dst_gemm_f32_kernel(GemmTable<G> g) {
   __shared__ __attribute__((aligned(16))) float lds[2 * 2 * TILE32];
   int c;
-  const int lb = gemm_block<G>(g, c);
+  const int lb = gemm_block<G, BM, BN>(g, c);
   if (lb < 0) return;
   const GemmArgs& a = g.a[c];
-  const GemmCut cut = gemm_cut(a.RA, a.RB, a.K);
+  const GemmCut cut = a.cut;
   const int GA = (cut.am + BM - 1) / BM, GB = (cut.bm + BN - 1) / BN;
   const int T = GA * GB * a.nplanes;
   if (lb >= T) {
@@ -1092,63 +1097,153 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   else store_tile<false, 2, 2>(a, z, a0, b0, acc, sum, 0, lds, ps.sp);
 }
 
+// 64 x 64 tiles of four 32 x 32 waves for launches of few tiles: k-tiles of 16
+// in the bf16 kernels' LDS layout (64-byte rows, swizzled 16-byte chunks, filled
+// by global_load_lds), F32_STAGES of them, so that seven are in flight under
+// the 512 matrix cycles of one.  Per output the chain of products and the FP64
+// windows of the 128 x 128 tiles.
+constexpr int F32_STAGES = 8;
+constexpr size_t F32_SMALL_LDS = (size_t)F32_STAGES * 2 * 64 * 64;
+template <int G>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
+void dst_gemm_f32_small_kernel(GemmTable<G> g) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds16[];
+  int c;
+  const int lb = gemm_block<G, 64, 64>(g, c);
+  if (lb < 0) return;
+  const GemmArgs& a = g.a[c];
+  const GemmCut cut = a.cut;
+  const int GA = (cut.am + 63) / 64, GB = (cut.bm + 63) / 64;
+  const int T = GA * GB * a.nplanes;
+  if (lb >= T) {
+    const int zf = (lb - T) / cut.fpw;
+    gemm_fringe<true, 1, 256>(a, zf, (lb - T) - zf * cut.fpw, cut, select_plane(a, zf), 0, lds16);
+    return;
+  }
+  int zi, ta, tb;
+  tile_of(lb, GA, GB, zi, ta, tb);
+  const long z = zi;
+  const PlaneSel ps = select_plane(a, z);
+  const int a0 = ta * 64, b0 = tb * 64;
+  const bool x_in_a = !a.trans;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  constexpr int TILE = 64 * 16;  // floats per operand tile
+  float* const lds = reinterpret_cast<float*>(lds16);
+  // each wave fills 16 rows of both operands' tiles
+  const int row = wave * 16 + (lane >> 2);
+  const int chunk = (lane & 3) ^ swz(row);
+  const int x0 = x_in_a ? a0 : b0, s0 = x_in_a ? b0 : a0;
+  const int xr = x0 + row < a.xrows ? x0 + row : a.xrows - 1;  // rows past R are never stored
+  const float* xsrc = a.Xf + z * a.x_batch + (long)xr * a.ldx + chunk * 4;
+  const float* ssrc = a.Sf + ps.s_off + (long)(s0 + row) * a.lds + chunk * 4;
+  const int xdst = (x_in_a ? 0 : TILE) + wave * 256, sdst = (x_in_a ? TILE : 0) + wave * 256;
+  auto issue = [&](int kt) {
+    float* sb = lds + (kt % F32_STAGES) * 2 * TILE;
+    __builtin_amdgcn_global_load_lds(xsrc + kt * BK32, sb + xdst, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds(ssrc + kt * BK32, sb + sdst, 16, 0, 0);
+  };
+  const int nk = (a.K + BK32 - 1) / BK32;
+#pragma unroll
+  for (int s = 0; s < F32_STAGES - 1; ++s)
+    if (s < nk) issue(s);
+  const int ra = wm * 32 + (lane & 31), rb = wn * 32 + (lane & 31);
+  const bool odd = lane >= 32;  // lanes 32-63 hold the odd k of each pair
+  auto ktile = [&](int kt, floatx16& w) {
+    // tile kt has landed once at most the later tiles' loads are outstanding;
+    // after the barrier every wave has read tile kt-1, whose stage is refilled
+    const int later = (nk - 1 - kt) < (F32_STAGES - 2) ? (nk - 1 - kt) : (F32_STAGES - 2);
+    wait_later<2, F32_STAGES - 2>(later);
+    __builtin_amdgcn_s_waitcnt((0xF) | (0x7 << 4) | (0x0 << 8) | (0x3 << 14));  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (kt + F32_STAGES - 1 < nk) issue(kt + F32_STAGES - 1);
+    const float* tA = lds + (kt % F32_STAGES) * 2 * TILE;
+    const float* tB = tA + TILE;
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) {
+      const floatx4 fa = *reinterpret_cast<const floatx4*>(tA + ra * 16 + ((ch ^ swz(ra)) << 2));
+      const floatx4 fb = *reinterpret_cast<const floatx4*>(tB + rb * 16 + ((ch ^ swz(rb)) << 2));
+      w = __builtin_amdgcn_mfma_f32_32x32x2f32(odd ? fa[1] : fa[0], odd ? fb[1] : fb[0], w, 0, 0, 0);
+      w = __builtin_amdgcn_mfma_f32_32x32x2f32(odd ? fa[3] : fa[2], odd ? fb[3] : fb[2], w, 0, 0, 0);
+    }
+  };
+  floatx16 acc[1][1];
+  double sum[1][1][16];
+  zero_acc<1, 1>(acc, sum);
+  int kt = 0;
+  for (; kt + 4 <= nk; kt += 4) {
+    floatx16 w = {};
+    for (int f = 0; f < 4; ++f) ktile(kt + f, w);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sum[0][0][r] += (double)w[r];
+  }
+  for (; kt < nk; ++kt) ktile(kt, acc[0][0]);
+  store_tile<true, 1, 1, 2, 64, 64>(a, z, a0, b0, acc, sum, 0, lds, ps.sp);
+}
 
-template __global__ void dst_gemm_bf16_kernel<1, 1>(GemmTable<1>);
-template __global__ void dst_gemm_bf16_kernel<3, 1>(GemmTable<1>);
-template __global__ void dst_gemm_bf16_kernel<6, 1>(GemmTable<1>);
-template __global__ void dst_gemm_bf16_kernel<1, MAX_GROUP>(GemmTable<MAX_GROUP>);
-template __global__ void dst_gemm_bf16_kernel<3, MAX_GROUP>(GemmTable<MAX_GROUP>);
-template __global__ void dst_gemm_bf16_kernel<6, MAX_GROUP>(GemmTable<MAX_GROUP>);
+template __global__ void dst_gemm_f32_small_kernel<1>(GemmTable<1>);
+template __global__ void dst_gemm_f32_small_kernel<MAX_GROUP>(GemmTable<MAX_GROUP>);
+template __global__ void dst_gemm_bf16_kernel<1, 1, 128>(GemmTable<1>);
+template __global__ void dst_gemm_bf16_kernel<1, 1, 64>(GemmTable<1>);
+template __global__ void dst_gemm_bf16_kernel<3, 1, 128>(GemmTable<1>);
+template __global__ void dst_gemm_bf16_kernel<3, 1, 64>(GemmTable<1>);
+template __global__ void dst_gemm_bf16_kernel<6, 1, 128>(GemmTable<1>);
+template __global__ void dst_gemm_bf16_kernel<6, 1, 64>(GemmTable<1>);
 template __global__ void dst_gemm_bf16_pair_kernel<1, 1>(GemmTable<1>);
 template __global__ void dst_gemm_bf16_pair_kernel<3, 1>(GemmTable<1>);
+template __global__ void dst_gemm_bf16_kernel<1, MAX_GROUP, 128>(GemmTable<MAX_GROUP>);
+template __global__ void dst_gemm_bf16_kernel<1, MAX_GROUP, 64>(GemmTable<MAX_GROUP>);
+template __global__ void dst_gemm_bf16_kernel<3, MAX_GROUP, 128>(GemmTable<MAX_GROUP>);
+template __global__ void dst_gemm_bf16_kernel<3, MAX_GROUP, 64>(GemmTable<MAX_GROUP>);
+template __global__ void dst_gemm_bf16_kernel<6, MAX_GROUP, 128>(GemmTable<MAX_GROUP>);
+template __global__ void dst_gemm_bf16_kernel<6, MAX_GROUP, 64>(GemmTable<MAX_GROUP>);
 template __global__ void dst_gemm_bf16_pair_kernel<1, MAX_GROUP>(GemmTable<MAX_GROUP>);
 template __global__ void dst_gemm_bf16_pair_kernel<3, MAX_GROUP>(GemmTable<MAX_GROUP>);
 
+namespace {
+hipError_t raise(const void* k, size_t bytes) {
+  return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+template <int NPMAX, int G>
+hipError_t prepare_np() {
+  hipError_t e =
+      raise(reinterpret_cast<const void*>(dst_gemm_bf16_kernel<NPMAX, G, 128>), dst_gemm_lds_bytes(NPMAX, 128));
+  if (e == hipSuccess)
+    e = raise(reinterpret_cast<const void*>(dst_gemm_bf16_kernel<NPMAX, G, 64>), dst_gemm_lds_bytes(NPMAX, 64));
+  if constexpr (NPMAX != 6)
+    if (e == hipSuccess)
+      e = raise(reinterpret_cast<const void*>(dst_gemm_bf16_pair_kernel<NPMAX, G>), dst_gemm_pair_lds_bytes(NPMAX));
+  return e;
+}
+}  // namespace
+
 hipError_t prepare_dst_gemm() {
-  // up to 144 KiB of the 160 KiB LDS of a gfx950 CU (3 pieces, 3 stages);
-  // set outside any stream capture, before the first launch
+  // up to 144 KiB of the 160 KiB LDS of a gfx950 CU; set outside any stream
+  // capture, before the first launch
   static hipError_t status = [] {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_kernel<1, 1>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_lds_bytes(1));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_kernel<3, 1>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_lds_bytes(3));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_kernel<6, 1>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_lds_bytes(6));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_kernel<1, MAX_GROUP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_lds_bytes(1));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_kernel<3, MAX_GROUP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_lds_bytes(3));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_kernel<6, MAX_GROUP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_lds_bytes(6));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_pair_kernel<1, 1>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_pair_lds_bytes(1));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_pair_kernel<3, 1>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_pair_lds_bytes(3));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_pair_kernel<1, MAX_GROUP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_pair_lds_bytes(1));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(dst_gemm_bf16_pair_kernel<3, MAX_GROUP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dst_gemm_pair_lds_bytes(3));
+    hipError_t e = prepare_np<1, 1>();
+    if (e == hipSuccess) e = prepare_np<3, 1>();
+    if (e == hipSuccess) e = prepare_np<6, 1>();
+    if (e == hipSuccess) e = prepare_np<1, MAX_GROUP>();
+    if (e == hipSuccess) e = prepare_np<3, MAX_GROUP>();
+    if (e == hipSuccess) e = prepare_np<6, MAX_GROUP>();
+    if (e == hipSuccess) e = raise(reinterpret_cast<const void*>(dst_gemm_f32_small_kernel<1>), F32_SMALL_LDS);
+    if (e == hipSuccess) e = raise(reinterpret_cast<const void*>(dst_gemm_f32_small_kernel<MAX_GROUP>), F32_SMALL_LDS);
     return e;
   }();
   return status;
 }
 
 namespace {
-// Blocks of one transform: tiles of 128 x 128 (or 128 x 64 with pair tiles)
-// and the fringe workgroups.
-int gemm_blocks(const GemmArgs& a, bool pair = false) {
-  const GemmCut cut = gemm_cut(a.RA, a.RB, a.K);
-  const int bn = pair ? BNP : BN;
-  const int tiles = ((cut.bm + bn - 1) / bn) * ((cut.am + BM - 1) / BM) * a.nplanes;
+// Tile shapes of a launch.
+enum class Tiles { WHOLE, PAIR, SMALL };  // 128 x 128, 128 x 64, 64 x 64
+// Blocks of one transform: its tiles and the fringe workgroups.
+int gemm_blocks(const GemmArgs& a, Tiles t) {
+  const GemmCut cut = a.cut;
+  const int bm = t == Tiles::SMALL ? 64 : BM, bn = t == Tiles::WHOLE ? BN : 64;
+  const int tiles = ((cut.bm + bn - 1) / bn) * ((cut.am + bm - 1) / bm) * a.nplanes;
   return tiles + cut.fpw * a.nplanes;
 }
 int max_products(const GemmArgs& a) { return a.np_lo > a.np_hi ? a.np_lo : a.np_hi; }
@@ -1166,78 +1261,94 @@ int cu_count() {
   }
   return c;
 }
+// Tile shape and fringe share (dots per fringe workgroup) of a launch.
+//
+// 64 x 64 tiles (two workgroups share a CU) while they and the fringe fit the
+// chip at once: the 128 x 128 tiles of such a launch leave most of the CUs
+// idle, and one CU takes four times as long for its tile.  Their fringe
+// workgroups have 64 dots in flight, so they take as few dots each as fits; a
+// bf16 fringe of 256 dots each would be the launch's tail (3 x 768^2: 0.8x), an
+// FP32 one is not.  Measured, a right-hand side (us, 128 x 128 -> 64 x 64): FP32
+// 64^2 x 3 74 -> 43, 301^2 x 3 152 -> 74, 512^2 x 3 152 -> 80, 640^2 x 3 175 ->
+// 117; six products 301^2 x 3 96 -> 56, 512^2 x 3 102 -> 76; mixed 256^2 x 3
+// 105 -> 85, 512^2 x 3 140 -> 114.  Launches that share the chip with others
+// (classes of a concurrent ensemble) keep the denser tiles: a 32-member
+// ensemble's step took 743 against 654 us on small ones.
+//
 // The x1 / x3 transforms run on pair tiles when their 128 x 128 workgroups
-// (tiles and fringe, `blocks`) would take more than one round of the CUs:
-// measured, the 256-member ensemble's step 3.41 -> 3.23 ms, while the 1024^2
-// model's transforms, one round of 252 workgroups, are faster whole
-// (22.2 against 25.5 us for a x3 launch).
-bool use_pair(const GemmArgs& a, int max_np, long blocks) { return !a.Xf && max_np <= 3 && blocks > cu_count(); }
+// (tiles and fringe) would take more than one round of the CUs: measured, the
+// 256-member ensemble's step 3.41 -> 3.23 ms, while the 1024^2 model's
+// transforms, one round of 252 workgroups, are faster whole (22.2 against
+// 25.5 us for a x3 launch).
+Tiles pick_tiles(GemmArgs* a, int n, int max_np) {
+  const int cus = cu_count();
+  const bool f32 = a[0].Xf != nullptr;
+  auto total = [&](Tiles t, int fdots) {
+    long b = 0;
+    for (int i = 0; i < n; ++i) {
+      a[i].cut = gemm_cut(a[i].RA, a[i].RB, a[i].K, fdots);
+      b += gemm_blocks(a[i], t);
+    }
+    return b;
+  };
+  // (the FP32 small kernel always sums its windows in FP64)
+  if (a[0].alone && (!f32 || a[0].acc64))
+    for (int fdots = 64; fdots <= (f32 ? 256 : 128); fdots *= 2)
+      if (total(Tiles::SMALL, fdots) <= 2 * cus) return Tiles::SMALL;
+  return total(Tiles::WHOLE, 256) > cus && !f32 && max_np <= 3 ? Tiles::PAIR : Tiles::WHOLE;
+}
+
+template <int NPMAX, int G>
+void launch_bf16(const GemmTable<G>& g, Tiles t, int blocks, hipStream_t st) {
+  if (t == Tiles::SMALL) {
+    hipLaunchKernelGGL((dst_gemm_bf16_kernel<NPMAX, G, 64>), dim3(blocks), dim3(KernelShape<NPMAX, 64>::NT),
+                       dst_gemm_lds_bytes(NPMAX, 64), st, g);
+    return;
+  }
+  if constexpr (NPMAX != 6)
+    if (t == Tiles::PAIR) {
+      hipLaunchKernelGGL((dst_gemm_bf16_pair_kernel<NPMAX, G>), dim3(blocks), dim3(512),
+                         dst_gemm_pair_lds_bytes(NPMAX), st, g);
+      return;
+    }
+  hipLaunchKernelGGL((dst_gemm_bf16_kernel<NPMAX, G, 128>), dim3(blocks), dim3(KernelShape<NPMAX, 128>::NT),
+                     dst_gemm_lds_bytes(NPMAX, 128), st, g);
+}
+template <int G>
+void launch_table(const GemmTable<G>& g, Tiles t, int max_np, int blocks, hipStream_t st) {
+  if (g.a[0].Xf) {
+    if (t == Tiles::SMALL)
+      hipLaunchKernelGGL(dst_gemm_f32_small_kernel<G>, dim3(blocks), dim3(256), F32_SMALL_LDS, st, g);
+    else
+      hipLaunchKernelGGL(dst_gemm_f32_kernel<G>, dim3(blocks), dim3(256), 0, st, g);
+    return;
+  }
+  if (max_np == 1) launch_bf16<1, G>(g, t, blocks, st);
+  else if (max_np == 3) launch_bf16<3, G>(g, t, blocks, st);
+  else launch_bf16<6, G>(g, t, blocks, st);
+}
 }  // namespace
 
 void launch_dst_gemm_group(const GemmArgs* args, const int* batch, int n, hipStream_t st) {
   GemmTable<MAX_GROUP> g{};
   int max_np = 0;
   for (int i = 0; i < n; ++i) {
-    const int np = max_products(args[i]);
-    max_np = np > max_np ? np : max_np;
-  }
-  long whole = 0;  // workgroups with 128 x 128 tiles
-  for (int i = 0; i < n; ++i) {
-    GemmArgs t = args[i];
-    t.nplanes = batch[i];
-    whole += gemm_blocks(t);
-  }
-  const bool pair = use_pair(args[0], max_np, whole);
-  for (int i = 0; i < n; ++i) {
     g.a[i] = args[i];
     g.a[i].nplanes = batch[i];
-    table_add(g.t, gemm_blocks(g.a[i], pair), 1, 1);
+    max_np = std::max(max_np, max_products(args[i]));
   }
-  const dim3 grid(g.t.start[g.t.n]);
-  if (args[0].Xf) {
-    hipLaunchKernelGGL(dst_gemm_f32_kernel<MAX_GROUP>, grid, dim3(256), 0, st, g);
-    return;
-  }
-  if (pair) {
-    const size_t lp = dst_gemm_pair_lds_bytes(max_np);
-    if (max_np == 1) hipLaunchKernelGGL((dst_gemm_bf16_pair_kernel<1, MAX_GROUP>), grid, dim3(512), lp, st, g);
-    else hipLaunchKernelGGL((dst_gemm_bf16_pair_kernel<3, MAX_GROUP>), grid, dim3(512), lp, st, g);
-    return;
-  }
-  const size_t lds = dst_gemm_lds_bytes(max_np);
-  if (max_np == 1)
-    hipLaunchKernelGGL((dst_gemm_bf16_kernel<1, MAX_GROUP>), grid, dim3(KernelShape<1>::NT), lds, st, g);
-  else if (max_np == 3)
-    hipLaunchKernelGGL((dst_gemm_bf16_kernel<3, MAX_GROUP>), grid, dim3(KernelShape<3>::NT), lds, st, g);
-  else
-    hipLaunchKernelGGL((dst_gemm_bf16_kernel<6, MAX_GROUP>), grid, dim3(KernelShape<6>::NT), lds, st, g);
+  const Tiles t = pick_tiles(g.a, n, max_np);
+  for (int i = 0; i < n; ++i) table_add(g.t, gemm_blocks(g.a[i], t), 1, 1);
+  launch_table(g, t, max_np, g.t.start[g.t.n], st);
 }
 
 void launch_dst_gemm(const GemmArgs& args, int batch, hipStream_t st) {
   GemmTable<1> g{};
   g.a[0] = args;
   g.a[0].nplanes = batch;
-  const GemmArgs& a = g.a[0];
-  const int max_np = max_products(a);
-  const bool pair = use_pair(a, max_np, gemm_blocks(a));
-  const int blocks = gemm_blocks(a, pair);
-  if (a.Xf) {
-    hipLaunchKernelGGL(dst_gemm_f32_kernel<1>, dim3(blocks), dim3(256), 0, st, g);
-    return;
-  }
-  if (pair) {
-    const size_t lp = dst_gemm_pair_lds_bytes(max_np);
-    if (max_np == 1) hipLaunchKernelGGL((dst_gemm_bf16_pair_kernel<1, 1>), dim3(blocks), dim3(512), lp, st, g);
-    else hipLaunchKernelGGL((dst_gemm_bf16_pair_kernel<3, 1>), dim3(blocks), dim3(512), lp, st, g);
-    return;
-  }
-  const size_t lds = dst_gemm_lds_bytes(max_np);
-  if (max_np == 1)
-    hipLaunchKernelGGL((dst_gemm_bf16_kernel<1, 1>), dim3(blocks), dim3(KernelShape<1>::NT), lds, st, g);
-  else if (max_np == 3)
-    hipLaunchKernelGGL((dst_gemm_bf16_kernel<3, 1>), dim3(blocks), dim3(KernelShape<3>::NT), lds, st, g);
-  else
-    hipLaunchKernelGGL((dst_gemm_bf16_kernel<6, 1>), dim3(blocks), dim3(KernelShape<6>::NT), lds, st, g);
+  const int max_np = max_products(args);
+  const Tiles t = pick_tiles(g.a, 1, max_np);
+  launch_table(g, t, max_np, gemm_blocks(g.a[0], t), st);
 }
 
 }  // namespace somax

@@ -127,6 +127,12 @@ struct MemberParams {
   float nu, nu4, kappa, tau0;
 };
 
+// Tile cut of a launch: rows (columns) covered by full tiles, am (bm), and
+// fringe workgroups per plane, fpw.
+struct GemmCut {
+  int am, bm, fpw;
+};
+
 // O[a][b] = sum_k A[a][k] B[b][k] with the data plane X in the A slot
 // (trans == 0: O = X S) or in the B slot (trans == 1: O = (X S)^T), S a sine
 // matrix (rows = outputs, k contiguous).  FP32 operands when Xf != null, else
@@ -175,18 +181,16 @@ struct GemmArgs {
   long s_var;   // elements between the sine operand's parity variants
   int lam_var;   // floats between the parity variants of lamA (x parity)
   int lamB_var;  // floats between the parity variants of lamB (y parity)
+  int alone;     // no other launches are meant to run beside this one
   int nplanes;   // batch planes of the launch (set by launch_dst_gemm)
+  GemmCut cut;   // its tile cut (set by launch_dst_gemm)
 };
 
-// Tile cut of a launch: rows (columns) covered by full tiles, am (bm), and
-// fringe workgroups per plane, fpw.  A dimension exceeding a multiple of 128
-// by 1 or 2 leaves that fringe to the fringe workgroups, whose fixed operand
-// rows (at most 4, FP64) are staged in 40 KiB of LDS; otherwise tiles cover
-// the whole dimension (fpw = 0).
-struct GemmCut {
-  int am, bm, fpw;
-};
-__host__ __device__ inline GemmCut gemm_cut(int RA, int RB, int K) {
+// The cut of an RA x RB x K transform with fdots dots per fringe workgroup.  A
+// dimension exceeding a multiple of 128 by 1 or 2 leaves that fringe to the
+// fringe workgroups, whose fixed operand rows (at most 4, FP64) are staged in
+// 40 KiB of LDS; otherwise tiles cover the whole dimension (fpw = 0).
+inline GemmCut gemm_cut(int RA, int RB, int K, int fdots) {
   auto cut = [](int R) {
     const int r = R & 127;
     return (R > 128 && (r == 1 || r == 2)) ? R - r : R;
@@ -198,7 +202,7 @@ __host__ __device__ inline GemmCut gemm_cut(int RA, int RB, int K) {
     c.bm = RB;
   }
   const long dots = (long)(RA - c.am) * RB + (long)c.am * (RB - c.bm);
-  c.fpw = dots > 0 ? (int)((dots + 255) / 256) : 0;
+  c.fpw = (int)((dots + fdots - 1) / fdots);
   return c;
 }
 
