@@ -174,23 +174,6 @@ __device__ __forceinline__ void product(Ring& v, const double* p, const double* 
       [&](int i, int b) { ring_load(v, i, p, b); });
 }
 
-// The same with both operands streamed.
-__device__ __forceinline__ void product(Ring& v, const double* p, Ring& w, const double* q, int ns, double4m& acc) {
-  ring_run(
-      (ns + 3) >> 2,
-      [&](int b, int i, auto whole) {
-        acc = mfma64(v[i][0], w[i][0], acc);
-        if (decltype(whole)::value || 4 * b + 1 < ns) {
-#pragma unroll
-          for (int t = 1; t < 4; ++t) acc = mfma64(v[i][t], w[i][t], acc);
-        }
-      },
-      [&](int i, int b) {
-        ring_load(v, i, p, b);
-        ring_load(w, i, q, b);
-      });
-}
-
 __host__ __device__ inline int direct_k(int h, int apply_bc) { return apply_bc ? h - 1 : h; }
 // LDS pitch (doubles) of the forward kernel's data rows: = 2 mod 4, so the 16
 // rows of a fragment read fall on distinct banks; a whole number of batches of
@@ -234,49 +217,66 @@ __global__ __launch_bounds__(512) void direct_forward_kernel(DirectTable<G> g) {
   const R* q = static_cast<const R*>(a.q) + (long)first * a.plane;
   const int Nx = a.Nx, Ny = a.Ny;
   const bool bc = a.apply_bc != 0;
-  for (int e = tid; e < 16 * kpad; e += 512) {
-    const int yy = e / kpad, j = e - yy * kpad;
-    const int jy = yt * 16 + yy;
-    double s00 = 0.0, s01 = 0.0, s10 = 0.0, s11 = 0.0;  // [py][px]
-    const bool ring_y = bc && jy == a.hy - 1;
-    if (j < K && jy < a.hy && !ring_y) {
-      const int x = fold_phys(j, a.hx), xm = Nx - 1 - x;
-      const int y = fold_phys(jy, a.hy), ym = Ny - 1 - y;
-      const int at[4] = {y * Nx + x, y * Nx + xm, ym * Nx + x, ym * Nx + xm};
-      double u[4] = {0.0, 0.0, 0.0, 0.0};
+  // EB points of a thread at a time, all their loads before the first sum
+  auto project = [&](auto eb) {
+    constexpr int EB = decltype(eb)::value;
+    for (int e0 = tid; e0 < 16 * kpad; e0 += 512 * EB) {
+      int yy[EB], jj[EB], x[EB], y[EB];
+      bool live[EB];
+      double u[EB][4];
+#pragma unroll
+      for (int b = 0; b < EB; ++b) {
+        const int e = e0 + 512 * b;
+        yy[b] = e / kpad;
+        jj[b] = e - yy[b] * kpad;
+        const int jy = yt * 16 + yy[b];
+        live[b] = yy[b] < 16 && jj[b] < K && jy < a.hy && !(bc && jy == a.hy - 1);
+        x[b] = live[b] ? fold_phys(jj[b], a.hx) : 0;
+        y[b] = live[b] ? fold_phys(jy, a.hy) : 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[b][i] = 0.0;
+      }
       for (int k0 = 0; k0 < nl; k0 += NL) {
-        // all loads of a point before the first sum (layers past the last
-        // read it again with weight 0)
-        R r[NL][4];
+        // (layers past the last read it again and are left out of the sum)
+        R r[EB][NL][4];
 #pragma unroll
-        for (int k = 0; k < NL; ++k) {
-          const R* p = q + (k0 + k < nl ? k0 + k : nl - 1) * a.plane;
+        for (int b = 0; b < EB; ++b)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) r[k][i] = p[at[i]];
-        }
+          for (int k = 0; k < NL; ++k) {
+            const R* p = q + (k0 + k < nl ? k0 + k : nl - 1) * a.plane;
+            const int r0 = y[b] * Nx, r1 = (Ny - 1 - y[b]) * Nx, xm = Nx - 1 - x[b];
+            r[b][k][0] = p[r0 + x[b]];
+            r[b][k][1] = p[r0 + xm];
+            r[b][k][2] = p[r1 + x[b]];
+            r[b][k][3] = p[r1 + xm];
+          }
 #pragma unroll
-        for (int k = 0; k < NL; ++k) {
+        for (int k = 0; k < NL; ++k)
           if (k0 + k < nl) {
             const double w = cl[k0 + k];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) u[i] += w * (double)r[k][i];
+            for (int b = 0; b < EB; ++b)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) u[b][i] += w * (double)r[b][k][i];
           }
-        }
       }
-      if (x == xm) u[1] = u[3] = 0.0;  // the middle of an odd line counts once
-      if (y == ym) u[2] = u[3] = 0.0;
-      const double p0 = u[0] + u[1], m0 = u[0] - u[1], p1 = u[2] + u[3], m1 = u[2] - u[3];
-      s00 = p0 + p1;
-      s01 = m0 + m1;
-      s10 = p0 - p1;
-      s11 = m0 - m1;
+#pragma unroll
+      for (int b = 0; b < EB; ++b) {
+        if (yy[b] >= 16) continue;
+        double* v = u[b];
+        if (2 * x[b] == Nx - 1) v[1] = v[3] = 0.0;  // the middle of an odd line counts once
+        if (2 * y[b] == Ny - 1) v[2] = v[3] = 0.0;
+        const double p0 = v[0] + v[1], m0 = v[0] - v[1], p1 = v[2] + v[3], m1 = v[2] - v[3];
+        double* o = sd + yy[b] * pitch + jj[b];
+        o[0] = live[b] ? p0 + p1 : 0.0;  // [py][px]
+        o[16 * pitch] = live[b] ? m0 + m1 : 0.0;
+        o[32 * pitch] = live[b] ? p0 - p1 : 0.0;
+        o[48 * pitch] = live[b] ? m0 - m1 : 0.0;
+      }
     }
-    double* o = sd + yy * pitch + j;
-    o[0] = s00;
-    o[16 * pitch] = s01;
-    o[32 * pitch] = s10;
-    o[48 * pitch] = s11;
-  }
+  };
+  if (16 * kpad <= 512) project(std::integral_constant<int, 1>{});
+  else project(std::integral_constant<int, (NL <= 2 ? 4 : 2)>{});
   __syncthreads();
   const double* A = sd + par * 16 * pitch + (lane & 15) * pitch + (lane >> 4);
   double* T = a.T + ((long)(z * 4 + par) * a.ntx) * (256L * a.nty) + yt * 256 + lane;
@@ -328,7 +328,9 @@ __global__ __launch_bounds__(64 * NW) void direct_spectral_kernel(DirectTable<G>
   const double* ly = a.lamy + py * 16 * a.nty + (lane >> 4);
   const bool sums = a.homsol && px == 0 && py == 0;
   const double cxv = sums ? a.cx[xt * 16 + (lane & 15)] : 0.0;
-  for (int e = tid; e < 256 * a.nty; e += 64 * NW) Ts[e] = T[e];
+  // straight into LDS, 1 KiB a wave and instruction
+  for (int e = wave; e < 2 * a.nty; e += NW)
+    __builtin_amdgcn_global_load_lds(T + e * 128 + lane * 2, Ts + e * 128, 16, 0, 0);
   double total = 0.0;
   __syncthreads();
   for (int t = wave; t < a.nty; t += NW) {
@@ -375,21 +377,24 @@ __global__ __launch_bounds__(64 * NW) void direct_spectral_kernel(DirectTable<G>
   }
 }
 
-// Inverse: workgroup = 16 x 16 folded points (four mirror images of each) of
+// Inverse: workgroup = 16 x 16 XT folded points (four mirror images of each) of
 // one member.  Wave (mode, py, px) computes one parity block of one mode; the
 // blocks meet in LDS, where they are unfolded, corrected and mixed to layers.
-template <class R, int NMODE, int G>
+// XT = 2 halves what a wave streams per product (the data of 16 rows serves two
+// tiles of columns).
+template <class R, int NMODE, int XT, int G>
 __global__ __launch_bounds__(256 * NMODE) void direct_inverse_kernel(DirectTable<G> g) {
-  extern __shared__ __attribute__((aligned(16))) double sd[];  // [mode][py px][16][17]
+  extern __shared__ __attribute__((aligned(16))) double sd[];  // [mode][py px][16][CP]
   __shared__ double salpha[MAX_LAYERS];
   __shared__ double scm[64];
-  constexpr int CP = 17;
+  constexpr int CP = 16 * XT + 1;
   int c;
   const int l = direct_block<G>(g, c);
   if (l < 0) return;
   const DirectArgs& a = g.a[c];
-  const int xt = l % a.ntx;
-  const int rest = l / a.ntx;
+  const int nbx = (a.ntx + XT - 1) / XT;
+  const int xt = (l % nbx) * XT;
+  const int rest = l / nbx;
   const int yt = rest % a.nty, m = rest / a.nty;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int first = 0, nl = a.P;
@@ -401,30 +406,49 @@ __global__ __launch_bounds__(256 * NMODE) void direct_inverse_kernel(DirectTable
   }
   const int par = wave & 3, px = par & 1;
   const long blk = 256L * a.ntx * a.nty;
-  const double* B = a.gx + px * 256L * a.ntx * a.ntx + (long)xt * 256 * a.ntx + lane;
+  const double* B[XT];  // (a tile past the last streams it again)
+#pragma unroll
+  for (int j = 0; j < XT; ++j)
+    B[j] = a.gx + px * 256L * a.ntx * a.ntx + (long)(xt + j < a.ntx ? xt + j : a.ntx - 1) * 256 * a.ntx + lane;
   const double* A = a.V + (long)(first * 4 + par) * blk + (long)yt * (256L * a.ntx) + lane;
   const int ns = (a.hx + 3) / 4;
   int k = wave >> 2;
   A += (k < nl ? k : nl - 1) * 4 * blk;
-  Ring va, vb;
-  ring_start(va, A, (ns + 3) >> 2);
-  ring_start(vb, B, (ns + 3) >> 2);
+  const int nb = (ns + 3) >> 2;
+  Ring va, vb[XT];
+  auto start = [&] {
+    ring_start(va, A, nb);
+#pragma unroll
+    for (int j = 0; j < XT; ++j) ring_start(vb[j], B[j], nb);
+  };
+  start();
   if (tid < 64) scm[tid] = a.cm2l[m * 64 + tid];
-  // this thread's points of the unfolding and the first modes' homogeneous solutions there
+  // this thread's points of the unfolding (column j * 16 + xx of each tile) and
+  // the first modes' homogeneous solutions there
   const int Nx = a.Nx, Ny = a.Ny;
   const int yy = (tid >> 4) & 15, xx = tid & 15;
-  const int jy = yt * 16 + yy, jx = xt * 16 + xx;
-  const bool live = jy < a.hy && jx < a.hx;
-  const int x = live ? fold_phys(jx, a.hx) : 0, xm = Nx - 1 - x;
-  const int y = live ? fold_phys(jy, a.hy) : 0, ym = Ny - 1 - y;
-  const int at[4] = {y * Nx + x, y * Nx + xm, ym * Nx + x, ym * Nx + xm};  // a plane is below 2^31 points
+  const int jy = yt * 16 + yy;
+  const int y = jy < a.hy ? fold_phys(jy, a.hy) : 0, ym = Ny - 1 - y;
+  bool live[XT];
+  int at[XT][4];  // a plane is below 2^31 points
+#pragma unroll
+  for (int j = 0; j < XT; ++j) {
+    const int jx = (xt + j) * 16 + xx;
+    live[j] = jy < a.hy && jx < a.hx;
+    const int x = live[j] ? fold_phys(jx, a.hx) : 0, xm = Nx - 1 - x;
+    at[j][0] = y * Nx + x;
+    at[j][1] = y * Nx + xm;
+    at[j][2] = ym * Nx + x;
+    at[j][3] = ym * Nx + xm;
+  }
   const R* hom = static_cast<const R*>(a.homsol) + (long)first * a.plane;
-  R hv[NMODE][4];
+  constexpr int NH = XT == 1 && NMODE * sizeof(R) <= 24 ? NMODE : 0;  // modes fetched early (registers)
+  R hv[NH ? NH : 1][4];
   if (a.homsol) {
 #pragma unroll
-    for (int p = 0; p < NMODE; ++p)
+    for (int p = 0; p < NH; ++p)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) hv[p][i] = hom[(p < nl ? p : nl - 1) * a.plane + at[i]];
+      for (int i = 0; i < 4; ++i) hv[p][i] = hom[(p < nl ? p : nl - 1) * a.plane + at[0][i]];
     if (tid < nl) {
       const double* p = a.partial + (long)(first + tid) * a.ntx;
       double s = 0.0;
@@ -435,63 +459,89 @@ __global__ __launch_bounds__(256 * NMODE) void direct_inverse_kernel(DirectTable
     }
   }
   for (; k < nl; k += NMODE) {
-    double4m acc = {0.0, 0.0, 0.0, 0.0};
-    product(va, A, vb, B, ns, acc);
+    double4m acc[XT];
+#pragma unroll
+    for (int j = 0; j < XT; ++j) acc[j] = double4m{0.0, 0.0, 0.0, 0.0};
+    ring_run(
+        nb,
+        [&](int b, int i, auto whole) {
+#pragma unroll
+          for (int j = 0; j < XT; ++j) acc[j] = mfma64(va[i][0], vb[j][i][0], acc[j]);
+          if (decltype(whole)::value || 4 * b + 1 < ns) {
+#pragma unroll
+            for (int t = 1; t < 4; ++t)
+#pragma unroll
+              for (int j = 0; j < XT; ++j) acc[j] = mfma64(va[i][t], vb[j][i][t], acc[j]);
+          }
+        },
+        [&](int i, int b) {
+          ring_load(va, i, A, b);
+#pragma unroll
+          for (int j = 0; j < XT; ++j) ring_load(vb[j], i, B[j], b);
+        });
     if (k + NMODE < nl) {
       A += NMODE * 4 * blk;
-      ring_start(va, A, (ns + 3) >> 2);
-      ring_start(vb, B, (ns + 3) >> 2);
+      start();
     }
     double* o = sd + ((k * 4 + par) * 16 + (lane >> 4)) * CP + (lane & 15);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o[4 * r * CP] = acc[r];
+    for (int j = 0; j < XT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[4 * r * CP + 16 * j] = acc[j][r];
   }
   __syncthreads();
-  if (a.homsol && l == m * a.ntx * a.nty && tid < nl) {
+  if (a.homsol && l == m * nbx * a.nty && tid < nl) {
     double w = 0.0;
     for (int p = 0; p < nl; ++p) w += scm[tid * MAX_LAYERS + p] * salpha[p];
     if (a.psi_wall) a.psi_wall[first + tid] = (float)w;
     if (a.alpha) a.alpha[first + tid] = salpha[tid];
   }
-  if (!live) return;
   R* psi = static_cast<R*>(a.psi) + (long)first * a.plane;
-  const bool zero = mask && (y == 0 || x == 0);  // the ghost pair of either axis
-  for (int kl = tid >> 8; kl < nl; kl += NMODE) {
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
-    auto add = [&](int p, const R* h) {
-      const double w = scm[kl * MAX_LAYERS + p];
-      const double* e = sd + (p * 4 * 16 + yy) * CP + xx;
-      const double e00 = e[0], e01 = e[16 * CP], e10 = e[32 * CP], e11 = e[48 * CP];  // [py][px]
-      const double sp = e00 + e01, sm = e00 - e01, tp = e10 + e11, tm = e10 - e11;
-      double u[4] = {sp + tp, sm + tm, sp - tp, sm - tm};
-      if (a.homsol) {
+  for (int kl = tid >> 8; kl < nl; kl += NMODE)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) u[i] += salpha[p] * (double)h[i];
+    for (int j = 0; j < XT; ++j) {
+      if (!live[j]) continue;
+      double v[4] = {0.0, 0.0, 0.0, 0.0};
+      auto add = [&](int p, const R* h) {
+        const double w = scm[kl * MAX_LAYERS + p];
+        const double* e = sd + (p * 4 * 16 + yy) * CP + 16 * j + xx;
+        const double e00 = e[0], e01 = e[16 * CP], e10 = e[32 * CP], e11 = e[48 * CP];  // [py][px]
+        const double sp = e00 + e01, sm = e00 - e01, tp = e10 + e11, tm = e10 - e11;
+        double u[4] = {sp + tp, sm + tm, sp - tp, sm - tm};
+        if (a.homsol) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) u[i] += salpha[p] * (double)h[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += w * u[i];
+      };
+#pragma unroll
+      for (int p = 0; p < NH; ++p)
+        if (p < nl) add(p, hv[p]);
+      for (int p = NH; p < nl; ++p) {
+        R h[4] = {};
+        if (a.homsol) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) h[i] = hom[p * a.plane + at[j][i]];
+        }
+        add(p, h);
       }
+      // the ghost pair of either axis
+      const bool zero = mask && (y == 0 || at[j][0] == y * Nx);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] += w * u[i];
-    };
-#pragma unroll
-    for (int p = 0; p < NMODE; ++p)
-      if (p < nl) add(p, hv[p]);
-    for (int p = NMODE; p < nl; ++p) {
-      R h[4] = {};
-      if (a.homsol) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) h[i] = hom[p * a.plane + at[i]];
-      }
-      add(p, h);
+      for (int i = 0; i < 4; ++i) psi[kl * a.plane + at[j][i]] = zero ? (R)0 : (R)v[i];
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) psi[kl * a.plane + at[i]] = zero ? (R)0 : (R)v[i];
-  }
 }
 
 size_t forward_lds(const DirectArgs& a) {
   return (size_t)64 * direct_pitch(direct_k(a.hx, a.apply_bc)) * sizeof(double);
 }
 size_t spectral_lds(const DirectArgs& a) { return (size_t)512 * a.nty * sizeof(double); }
-size_t inverse_lds(const DirectArgs& a) { return (size_t)a.nlmax * 4 * 16 * 17 * sizeof(double); }
+// Column tiles per workgroup of the inverse kernel: two where a fold has more
+// than eight tiles (measured at 512^2 x 3: 30 -> 23 us) and the registers of a
+// workgroup of up to three modes hold the second stream.
+int inverse_xt(int ntx, int nlmax) { return ntx > 8 && nlmax <= 3 ? 2 : 1; }
+size_t inverse_lds(const DirectArgs& a, int xt) { return (size_t)a.nlmax * 4 * 16 * (16 * xt + 1) * sizeof(double); }
 
 template <class K>
 hipError_t raise_lds(K kernel, int bytes) {
@@ -506,10 +556,13 @@ hipError_t prepare_kernels() {
   if (e == hipSuccess) e = raise_lds(direct_forward_kernel<R, 4, G>, DIRECT_LDS);
   if (e == hipSuccess) e = raise_lds(direct_spectral_kernel<4, G>, DIRECT_LDS);
   if (e == hipSuccess) e = raise_lds(direct_spectral_kernel<8, G>, DIRECT_LDS);
-  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 1, G>, DIRECT_LDS);
-  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 2, G>, DIRECT_LDS);
-  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 3, G>, DIRECT_LDS);
-  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 4, G>, DIRECT_LDS);
+  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 1, 1, G>, DIRECT_LDS);
+  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 2, 1, G>, DIRECT_LDS);
+  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 3, 1, G>, DIRECT_LDS);
+  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 4, 1, G>, DIRECT_LDS);
+  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 1, 2, G>, DIRECT_LDS);
+  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 2, 2, G>, DIRECT_LDS);
+  if (e == hipSuccess) e = raise_lds(direct_inverse_kernel<R, 3, 2, G>, DIRECT_LDS);
   return e;
 }
 hipError_t prepare_direct() {
@@ -534,12 +587,12 @@ void launch_spectral(DirectTable<G>& g, int blocks, size_t lds, int nty, hipStre
   if (nty > 4) hipLaunchKernelGGL((direct_spectral_kernel<8, G>), dim3(blocks), dim3(512), lds, st, g);
   else hipLaunchKernelGGL((direct_spectral_kernel<4, G>), dim3(blocks), dim3(256), lds, st, g);
 }
-template <class R, int G>
+template <class R, int XT, int G>
 void launch_inverse(DirectTable<G>& g, int blocks, size_t lds, int nlmax, hipStream_t st) {
-  if (nlmax == 1) hipLaunchKernelGGL((direct_inverse_kernel<R, 1, G>), dim3(blocks), dim3(256), lds, st, g);
-  else if (nlmax == 2) hipLaunchKernelGGL((direct_inverse_kernel<R, 2, G>), dim3(blocks), dim3(512), lds, st, g);
-  else if (nlmax == 3) hipLaunchKernelGGL((direct_inverse_kernel<R, 3, G>), dim3(blocks), dim3(768), lds, st, g);
-  else hipLaunchKernelGGL((direct_inverse_kernel<R, 4, G>), dim3(blocks), dim3(1024), lds, st, g);
+  if (nlmax == 1) hipLaunchKernelGGL((direct_inverse_kernel<R, 1, XT, G>), dim3(blocks), dim3(256), lds, st, g);
+  else if (nlmax == 2) hipLaunchKernelGGL((direct_inverse_kernel<R, 2, XT, G>), dim3(blocks), dim3(512), lds, st, g);
+  else if (nlmax == 3) hipLaunchKernelGGL((direct_inverse_kernel<R, 3, XT, G>), dim3(blocks), dim3(768), lds, st, g);
+  else hipLaunchKernelGGL((direct_inverse_kernel<R, 4, 1, G>), dim3(blocks), dim3(1024), lds, st, g);
 }
 
 // One axis on the host: operators in fragment order, eigenvalues, column sums.
@@ -703,20 +756,24 @@ DirectArgs call_args(const DirectCall& c) {
 template <class R, int G>
 void run(const DirectCall* c, int n, hipStream_t st, const DirectPhase& phase) {
   DirectTable<G> g{};
-  int blocks[3] = {0, 0, 0}, nty = 0, nlmax = 0;
+  int blocks[3] = {0, 0, 0}, nty = 0, ntx = 0, nlmax = 0;
+  for (int i = 0; i < n; ++i) {
+    nty = std::max(nty, c[i].d->a.nty);
+    ntx = std::max(ntx, c[i].d->a.ntx);
+    nlmax = std::max(nlmax, c[i].d->a.nlmax);
+  }
+  const int xt = inverse_xt(ntx, nlmax);
   size_t lds[3] = {0, 0, 0};
   BlockTable t[3] = {};
   for (int i = 0; i < n; ++i) {
     const DirectArgs& a = g.a[i] = call_args(c[i]);
-    const int count[3] = {a.P * a.nty * a.split, a.P * 4 * a.ntx, a.M * a.ntx * a.nty};
-    const size_t need[3] = {forward_lds(a), spectral_lds(a), inverse_lds(a)};
+    const int count[3] = {a.P * a.nty * a.split, a.P * 4 * a.ntx, a.M * ((a.ntx + xt - 1) / xt) * a.nty};
+    const size_t need[3] = {forward_lds(a), spectral_lds(a), inverse_lds(a, xt)};
     for (int k = 0; k < 3; ++k) {
       table_add(t[k], count[k], 1, 1);
       blocks[k] = G == 1 ? count[k] : t[k].start[t[k].n];
       lds[k] = std::max(lds[k], need[k]);
     }
-    nty = std::max(nty, a.nty);
-    nlmax = std::max(nlmax, a.nlmax);
   }
   phase(0, [&] {
     g.t = t[0];
@@ -728,7 +785,8 @@ void run(const DirectCall* c, int n, hipStream_t st, const DirectPhase& phase) {
   });
   phase(2, [&] {
     g.t = t[2];
-    launch_inverse<R, G>(g, blocks[2], lds[2], nlmax, st);
+    if (xt == 2) launch_inverse<R, 2, G>(g, blocks[2], lds[2], nlmax, st);
+    else launch_inverse<R, 1, G>(g, blocks[2], lds[2], nlmax, st);
   });
 }
 }  // namespace
