@@ -1230,38 +1230,34 @@ void rk3_group(const std::vector<RkItem>& it, int nsteps, double dt, hipStream_t
   }
 }
 
-// Tsit5 (FSAL): k0 = f(y) once, then per step six more evaluations
-// k_i = f(y + dt sum_j a_ij k_j), i = 1..6, the last at the new state
-// y + dt sum_j b_j k_j, which becomes k0 of the next step.  f = the RHS with
-// the boundary condition applied first (SomaxModel.build_terms).
-// tws: Y (stage state) then K0..K6, each P planes.
+// Tsit5: per step six evaluations k_i = f(y + dt sum_j a_ij k_j), f the RHS with
+// the boundary condition applied first (SomaxModel.build_terms).  The stage
+// kernel that computes k_i also forms the next stage state from it, the last one
+// the new state y + dt sum_j b_j k_j in place (first same as last: the seventh
+// evaluation of a step is the next step's first, and the last step needs none).
+// tws: K0..K4 and two stage states, each P planes.
 void tsit5(const Batch& p, float* q, int nsteps, double dt, const CallParams& cp, void* ws, void* tws,
            hipStream_t st) {
   const long n = (long)p.P * p.splane;
   float* psi = wsf(ws, p.off_PSI);
-  float* Y = static_cast<float*>(tws);
-  float* K[7];
-  for (int i = 0; i < 7; ++i) K[i] = Y + (i + 1) * n;
-  auto f = [&](const float* y, float* k) {
-    invert(p, Solve::STATE, y, psi, ws, st);
-    stage(p, y, psi, nullptr, k, cp, 0.0f, 1.0f, true, ws, st);
-  };
-  if (nsteps > 0) f(q, K[0]);
+  float* K = static_cast<float*>(tws);
+  float* Y[2] = {K + 5 * n, K + 6 * n};
   for (int s = 0; s < nsteps; ++s) {
-    for (int i = 1; i <= 6; ++i) {
-      LinComb c{};
-      c.y = q;
-      c.nk = i;
+    for (int i = 0; i < 6; ++i) {
+      const float* in = i ? Y[(i - 1) & 1] : q;
+      invert(p, Solve::STATE, in, psi, ws, st);
+      StageArgs a = stage_args(p, in, psi, nullptr, i < 5 ? K + i * n : nullptr, cp, 0.0f, 1.0f, true, ws);
+      a.next.y = q;
+      a.next.nk = i;
       for (int j = 0; j < i; ++j) {
-        c.k[j] = K[j];
-        c.w[j] = dt * TSIT5_A[i][j];
+        a.next.k[j] = K + j * n;
+        a.next.w[j] = dt * TSIT5_A[i + 1][j];
       }
-      c.n = n;
-      c.out = i < 6 ? Y : q;  // row 6 = b: the new state, in place
-      launch_lincomb(c, st);
-      f(c.out, K[i]);
+      a.next.wl = dt * TSIT5_A[i + 1][i];
+      a.next.out = i < 5 ? Y[i & 1] : q;
+      ProfScope ps("qg_stage", 0.0, 4.0 * p.P * (double)p.nx * p.ny * (4.0 + i + (i < 5 ? 1.0 : 0.0)), st);
+      launch_qg_stage(a, st);
     }
-    std::swap(K[0], K[6]);  // first same as last
   }
 }
 

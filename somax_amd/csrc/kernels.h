@@ -300,6 +300,19 @@ struct LayerArgs {
 void launch_to_layer(const LayerArgs& a, hipStream_t st);
 void launch_to_layer_group(const LayerArgs* a, int n, hipStream_t st);
 
+// The next stage state of a Tsit5 step, formed by the stage kernel that computes
+// the derivative k it needs last: out = y + sum_{j < nk} w[j] k_j + wl k,
+// accumulated in FP64 in that order (k in FP32, as stored).  `out` may be `y`
+// (the step's last combination), never the array whose stencils are read.
+template <class T>
+struct NextState {
+  const T* y;
+  const T* k[5];
+  double w[5], wl;
+  int nk;
+  T* out;  // null: no next state
+};
+
 // One QG RHS evaluation fused with the RK stage combination:
 //   out = qn + c1*(qs - qn) + c2*rhs(BC(qs), psi)   (qn given)
 //   out = c1*qs + c2*rhs                           (qn null)
@@ -322,6 +335,7 @@ struct StageArgs {
   int advection;
   int apply_bc;  // 1: ghost ring of qs read as 0 in the RHS (SomaxModel.build_terms)
   int tile_rows;  // Arakawa stage tile height: 8 or 16 (0: 16)
+  NextState<float> next;  // (out is then nullable: the derivative is not stored)
 };
 void launch_qg_stage(const StageArgs& a, hipStream_t st);
 // n batches sharing advection, biharm and (Arakawa) tile_rows

@@ -229,6 +229,9 @@ struct Stage64 {
   double dx, dy;
   int advection, apply_bc, rhs_only;
   double a, adiv, b, h;
+  // Tsit5: next stage state next.y + nh (sum_j next.w[j] k_j + next.wl rhs)
+  NextState<double> next;
+  double nh;
 };
 
 constexpr double WENO_EPS = 1e-20;
@@ -370,26 +373,20 @@ __global__ __launch_bounds__(256) void stage64_kernel(Stage64 s) {
     return g ? 0.0 : lap64(s, Q, jj, ii);
   };
   const double r = rhs_point(s, Q, P, QT, L, l, j, i, pw);
-  s.out[l * s.plane + c] = combine(s, in[c], s.qn ? s.qn[l * s.plane + c] : 0.0, r);
-}
-
-// out = y + h * sum_j w[j] k[j] (sum in j order)
-struct Lin64 {
-  const double* y;
-  const double* k[LINCOMB_MAX];
-  double w[LINCOMB_MAX];
-  int nk;
-  double h;
-  long n;
-  double* out;
-};
-
-__global__ __launch_bounds__(256) void lincomb64_kernel(Lin64 c) {
-  const long e = blockIdx.x * 256L + threadIdx.x;
-  if (e >= c.n) return;
-  double s = c.w[0] * c.k[0][e];
-  for (int j = 1; j < c.nk; ++j) s = s + c.w[j] * c.k[j][e];
-  c.out[e] = c.y[e] + c.h * s;
+  const long e = l * s.plane + c;
+  const double o = combine(s, in[c], s.qn ? s.qn[e] : 0.0, r);
+  if (s.out) s.out[e] = o;
+  if (s.next.out) {
+    double t = 0.0;
+    if (s.next.nk == 0) {
+      t = s.next.wl * o;
+    } else {
+      t = s.next.w[0] * s.next.k[0][e];
+      for (int j = 1; j < s.next.nk; ++j) t = t + s.next.w[j] * s.next.k[j][e];
+      t = t + s.next.wl * o;
+    }
+    s.next.out[e] = s.next.y[e] + s.nh * t;
+  }
 }
 
 // diagnose: u = -(psi[j+1] - psi[j]) / dy on rows 0..Ny-2, v = (psi[i+1] -
@@ -574,31 +571,31 @@ void rk3(const Qg64& p, double* q, double* psi_out, int nsteps, double dt, const
   }
 }
 
-// Tsit5 with first-same-as-last: tws holds Y and K0..K6, each nl planes.
+// Tsit5, as the FP32 form's: six evaluations per step, each stage kernel
+// forming the next stage state.  tws: K0..K4 and two stage states.
 void tsit5(const Qg64& p, double* q, int nsteps, double dt, const somaxhip_qg_params& prm, void* ws, void* tws,
            hipStream_t st) {
   const long n = (long)p.nl * p.plane;
   double* psi = wsd(ws, p.off_PSI);
-  double* Y = static_cast<double*>(tws);
-  double* K[7];
-  for (int i = 0; i < 7; ++i) K[i] = Y + (i + 1) * n;
-  if (nsteps > 0) rhs(p, q, K[0], psi, prm, ws, true, st);
+  double* K = static_cast<double*>(tws);
+  double* Y[2] = {K + 5 * n, K + 6 * n};
   for (int s = 0; s < nsteps; ++s) {
-    for (int i = 1; i <= 6; ++i) {
-      Lin64 c{};
-      c.y = q;
-      c.nk = i;
+    for (int i = 0; i < 6; ++i) {
+      const double* in = i ? Y[(i - 1) & 1] : q;
+      invert(p, in, psi, ws, true, st);
+      Stage64 a = stage_args(p, in, psi, nullptr, i < 5 ? K + i * n : nullptr, prm, ws, true);
+      a.rhs_only = 1;
+      a.next.y = q;
+      a.next.nk = i;
       for (int j = 0; j < i; ++j) {
-        c.k[j] = K[j];
-        c.w[j] = TSIT5_A[i][j];
+        a.next.k[j] = K + j * n;
+        a.next.w[j] = TSIT5_A[i + 1][j];
       }
-      c.h = dt;
-      c.n = n;
-      c.out = i < 6 ? Y : q;  // row 6 = the solution weights: the new state, in place
-      lincomb64_kernel<<<blocks(n), 256, 0, st>>>(c);
-      rhs(p, c.out, K[i], psi, prm, ws, true, st);
+      a.next.wl = TSIT5_A[i + 1][i];
+      a.nh = dt;
+      a.next.out = i < 5 ? Y[i & 1] : q;
+      launch_stage(p, a, st);
     }
-    std::swap(K[0], K[6]);
   }
 }
 

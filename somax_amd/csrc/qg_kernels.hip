@@ -15,12 +15,93 @@ namespace somax {
 namespace {
 constexpr int TX = 64;
 constexpr int TY_DEFAULT = 16;  // tile rows unless a batch chooses 8
+constexpr long CUS = 256;       // compute units of an MI355X
 constexpr int QW = TX + 4;  // q tile pitch (halo 2)
 constexpr int PW = TX + 2;  // psi / lap tile pitch (halo 1)
 }  // namespace
 
+// A stage on a small grid is one chain: load, LDS, store.  So every load of a block
+// is issued at once, the ghost ring's with the tile's (it was a second trip to memory
+// at the block's end), and the next stage state of Tsit5 is formed here, not by a
+// launch of its own that reads the derivatives again.  One evaluation of 64^2 x 1,
+// stage and combination: 9.0 -> 5.1 us; 128^2 x 3: 9.4 -> 5.0 (4-row tiles).
+//
+// What one output point needs beside the tile: the step-start value, the wind
+// row and, with NEXT, the terms of the next stage state.  Fetched before the tile
+// is waited for; the addresses are clamped instead of tested, so the loads issue
+// back to back.
+struct PointIn {
+  float qn, wind;
+  float y, k[5];
+};
+template <bool NEXT>
+__device__ __forceinline__ void point_fetch(const StageArgs& a, long idx, PointIn& f) {
+  f.qn = a.qn ? a.qn[idx] : 0.0f;
+  if constexpr (NEXT) {
+    f.y = a.next.y[idx];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) f.k[j] = j < a.next.nk ? a.next.k[j][idx] : 0.0f;
+  }
+}
+// Stage combination qn + c1 (qs - qn) + c2 rhs: the FP32 weights of the Shu-Osher
+// form (1/3 + 2/3 != 1 in FP32) would otherwise scale q by 1 + 3e-8 per step.
+// Without qn: c1 qs + c2 rhs.  Stored at idx, with the next stage state (NEXT).
+template <bool NEXT>
+__device__ __forceinline__ void point_store(const StageArgs& a, long idx, float qraw, float rhs, const PointIn& f) {
+  float o;
+  if (a.qn) {
+    o = f.qn + a.c1 * (qraw - f.qn) + a.c2 * rhs;
+  } else {
+    o = a.c2 * rhs;
+    if (a.c1 != 0.0f) o += a.c1 * qraw;
+  }
+  if (!NEXT || a.out) a.out[idx] = o;
+  if constexpr (NEXT) {
+    double v = (double)f.y;
+#pragma unroll
+    for (int j = 0; j < 5; ++j)
+      if (j < a.next.nk) v += a.next.w[j] * (double)f.k[j];
+    v += a.next.wl * (double)o;
+    a.next.out[idx] = (float)v;
+  }
+}
+
+// The ghost-ring point of a thread of an edge tile (rows y0 .. y0 + TY - 1 of the
+// interior block; ry < 0: none), one per thread.  Wave 0: row 0 under the first
+// tile row; wave 1: row Ny-1 under the last; wave 2: column 0 (lanes 0..TY-1,
+// first tile column) and column Nx-1 (lanes 32..32+TY-1, last tile column);
+// wave 3: the four corners.
+template <int TY>
+__device__ __forceinline__ void ring_point(const StageArgs& a, int wv, int tx, int gx, int y0, int bx, int by, int nbx,
+                                           int nby, int& ry, int& rx) {
+  static_assert(TY <= 32, "the two columns share one wave");
+  const int Nx = a.Nx, Ny = a.Ny;
+  const bool first_x = bx == 0, last_x = bx == nbx - 1;
+  const bool first_y = by == 0, last_y = by == nby - 1;
+  ry = rx = -1;
+  if (wv == 0 && first_y && gx <= Nx - 2) {
+    ry = 0;
+    rx = gx;
+  } else if (wv == 1 && last_y && gx <= Nx - 2) {
+    ry = Ny - 1;
+    rx = gx;
+  } else if (wv == 2 && tx < TY && first_x && y0 + tx <= Ny - 2) {
+    ry = y0 + tx;
+    rx = 0;
+  } else if (wv == 2 && tx >= 32 && tx < 32 + TY && last_x && y0 + tx - 32 <= Ny - 2) {
+    ry = y0 + tx - 32;
+    rx = Nx - 1;
+  } else if (wv == 3 && tx < 4) {
+    const bool top = tx < 2, left = (tx & 1) == 0;
+    if ((top ? first_y : last_y) && (left ? first_x : last_x)) {
+      ry = top ? 0 : Ny - 1;
+      rx = left ? 0 : Nx - 1;
+    }
+  }
+}
+
 // Tile (bx, by) of plane z, of a grid of nbx x nby tiles per plane.
-template <bool BIHARM, int TY>
+template <bool BIHARM, int TY, bool NEXT = false>
 __device__ __forceinline__ void qg_stage_arakawa(const StageArgs& a, int bx, int by, int z, int nbx, int nby) {
   __shared__ float sq[(TY + 4) * QW];
   __shared__ float sp[(TY + 2) * PW];
@@ -36,29 +117,18 @@ __device__ __forceinline__ void qg_stage_arakawa(const StageArgs& a, int bx, int
   const long off = (long)z * a.plane;
   const float* qs = a.qs + off;
   const float* psi = a.psi + off;
-  const int m = a.t.member[z];
+  const int m = a.mp ? a.t.member[z] : 0;  // (one model: member 0, no lookup before its rows)
   const MemberParams pr = a.mp ? a.mp[m] : a.u;
   const float* dbeta_row = a.dbeta_rows + (long)m * Ny;
   const float* wind_row = a.wind_rows + (long)m * Ny;
 
-  // This thread's outputs (column tx, rows tyb + 4 r): the previous stage
-  // value q_n and the wind row are fetched first, so their latency overlaps
-  // the tile loads instead of following the last barrier.
+  // Every load of the block is issued before the first LDS store, so that one
+  // memory latency covers them: the tile, then what the outputs of this thread
+  // (column tx, rows tyb + 4 r, and its ghost-ring point) need, then the member's
+  // rows, whose address may wait for the member table.  Tile: q with the boundary
+  // condition (ghost ring and outside the array read 0), halo 2; psi, halo 1.
   const int tx = tid & 63;
   const int tyb = tid >> 6;
-  float qn_r[TY / 4], wind_r[TY / 4];
-#pragma unroll
-  for (int r = 0; r < TY / 4; ++r) {
-    const int gy = y0 + tyb + 4 * r, gx = x0 + tx;
-    const bool ok = gy <= Ny - 2 && gx <= Nx - 2;
-    const int idx = gy * Nx + gx;
-    qn_r[r] = (ok && a.qn) ? a.qn[off + idx] : 0.0f;
-    wind_r[r] = ok ? wind_row[gy] : 0.0f;
-  }
-
-  // Tile loads: a fixed number per thread, all issued before the first LDS
-  // store, so one memory latency covers them.  q with the boundary condition
-  // (ghost ring and outside the array read 0); psi with a 1-cell halo.
   constexpr int NQ = ((TY + 4) * QW + 255) / 256;
   constexpr int NPS = ((TY + 2) * PW + 255) / 256;
   float vq[NQ], vp[NPS];
@@ -79,11 +149,26 @@ __device__ __forceinline__ void qg_stage_arakawa(const StageArgs& a, int bx, int
     const bool inside = i < (TY + 2) * PW && gy >= 0 && gy < Ny && gx >= 0 && gx < Nx;
     vp[k] = inside ? psi[gy * Nx + gx] : 0.0f;
   }
+  PointIn in[TY / 4], rin;
+  const int cgx = min(x0 + tx, Nx - 1);
+#pragma unroll
+  for (int r = 0; r < TY / 4; ++r) point_fetch<NEXT>(a, off + (long)min(y0 + tyb + 4 * r, Ny - 1) * Nx + cgx, in[r]);
+  int ry, rx;
+  ring_point<TY>(a, __builtin_amdgcn_readfirstlane(tyb), tx, x0 + tx, y0, bx, by, nbx, nby, ry, rx);
+  const long ridx = off + (long)ry * Nx + rx;
+  float rq = 0.0f;
+  if (ry >= 0) {
+    rq = a.qs[ridx];
+    point_fetch<NEXT>(a, ridx, rin);
+  }
   float vdb = 0.0f;
   if (tid < TY + 4) {
     const int gy = y0 - 2 + tid;
     vdb = (gy >= 0 && gy < Ny) ? dbeta_row[gy] : 0.0f;
   }
+#pragma unroll
+  for (int r = 0; r < TY / 4; ++r) in[r].wind = wind_row[min(y0 + tyb + 4 * r, Ny - 1)];
+  rin.wind = wind_row[max(ry, 0)];
 #pragma unroll
   for (int k = 0; k < NQ; ++k)
     if (tid + 256 * k < (TY + 4) * QW) sq[tid + 256 * k] = vq[k];
@@ -110,19 +195,6 @@ __device__ __forceinline__ void qg_stage_arakawa(const StageArgs& a, int bx, int
 
   const float wc = pr.tau0 * a.t.wind_scale[z];
   const bool bottom = (a.t.layer[z] == a.t.mnl[m] - 1) && (pr.kappa != 0.0f);
-  // Stage combination qn + c1 (qs - qn) + c2 rhs: the FP32 weights of the
-  // Shu-Osher form (1/3 + 2/3 != 1 in FP32) would otherwise scale q by
-  // 1 + 3e-8 per step.  Without qn: c1 qs + c2 rhs.
-  auto combine = [&](float qn, float qraw, float rhs) {
-    float o;
-    if (a.qn) {
-      o = qn + a.c1 * (qraw - qn) + a.c2 * rhs;
-    } else {
-      o = a.c2 * rhs;
-      if (a.c1 != 0.0f) o += a.c1 * qraw;
-    }
-    return o;
-  };
 #pragma unroll
   for (int r = 0; r < TY / 4; ++r) {
     const int ly = tyb + 4 * r;
@@ -154,45 +226,12 @@ __device__ __forceinline__ void qg_stage_arakawa(const StageArgs& a, int bx, int
       }
       if (bottom) rhs -= pr.kappa * ((pE - 2.0f * p[0] + pW) * a.idx2 + (pN - 2.0f * p[0] + pS) * a.idy2);
     }
-    rhs += wc * wind_r[r];
-    const long idx = off + (long)gy * Nx + gx;
-    a.out[idx] = combine(qn_r[r], sq[(ly + 2) * QW + tx + 2], rhs);
+    rhs += wc * in[r].wind;
+    point_store<NEXT>(a, off + (long)gy * Nx + gx, sq[(ly + 2) * QW + tx + 2], rhs, in[r]);
   }
-
   // Ghost ring: no Jacobian or viscous terms, only the wind row, and the raw
   // stage value (the tile holds 0 there under the boundary condition).
-  // Wave 0: row 0 under the first tile row; wave 1: row Ny-1 under the last;
-  // wave 2: column 0 (lanes 0..TY-1, first tile column) and column Nx-1
-  // (lanes 32..32+TY-1, last tile column); wave 3: the four corners.
-  const int wv = __builtin_amdgcn_readfirstlane(tyb);
-  const int gx = x0 + tx;
-  const bool first_x = bx == 0, last_x = bx == nbx - 1;
-  const bool first_y = by == 0, last_y = by == nby - 1;
-  int ry = -1, rx = -1;
-  if (wv == 0 && first_y && gx <= Nx - 2) {
-    ry = 0;
-    rx = gx;
-  } else if (wv == 1 && last_y && gx <= Nx - 2) {
-    ry = Ny - 1;
-    rx = gx;
-  } else if (wv == 2 && tx < TY && first_x && y0 + tx <= Ny - 2) {
-    ry = y0 + tx;
-    rx = 0;
-  } else if (wv == 2 && tx >= 32 && tx < 32 + TY && last_x && y0 + tx - 32 <= Ny - 2) {
-    ry = y0 + tx - 32;
-    rx = Nx - 1;
-  } else if (wv == 3 && tx < 4) {
-    const bool top = tx < 2, left = (tx & 1) == 0;
-    if ((top ? first_y : last_y) && (left ? first_x : last_x)) {
-      ry = top ? 0 : Ny - 1;
-      rx = left ? 0 : Nx - 1;
-    }
-  }
-  if (ry >= 0) {
-    const long idx = off + (long)ry * Nx + rx;
-    const float qn = a.qn ? a.qn[idx] : 0.0f;
-    a.out[idx] = combine(qn, a.qs[idx], wc * wind_row[ry]);
-  }
+  if (ry >= 0) point_store<NEXT>(a, ridx, rq, wc * rin.wind, rin);
 }
 
 // ---------------------------------------------------------------------------
@@ -211,7 +250,7 @@ __device__ __forceinline__ void qg_stage_arakawa(const StageArgs& a, int bx, int
 // ---------------------------------------------------------------------------
 namespace {
 constexpr int WX = 64;
-constexpr int WY = 16;
+constexpr int WY_DEFAULT = 16;
 constexpr int WQ = WX + 6;  // q tile pitch (halo 3)
 constexpr float WENO_EPS = 1e-20f;
 
@@ -280,7 +319,7 @@ __device__ inline float face_corr(int f, int n, float vel, const float* dm) {
 }  // namespace
 
 // Tile (bx, by) of plane z, of a grid of nbx x nby tiles per plane.
-template <bool BIHARM>
+template <bool BIHARM, int WY, bool NEXT = false>
 __device__ __forceinline__ void qg_stage_weno(const StageArgs& a, int bx, int by, int z, int nbx, int nby) {
   constexpr int QH = WY + 6;    // q tile rows (halo 3)
   constexpr int PH = WY + 2;    // psi / Laplacian tile rows (halo 1)
@@ -303,7 +342,7 @@ __device__ __forceinline__ void qg_stage_weno(const StageArgs& a, int bx, int by
   const long off = (long)z * a.plane;
   const float* qs = a.qs + off;
   const float* psi = a.psi + off;
-  const int m = a.t.member[z];
+  const int m = a.mp ? a.t.member[z] : 0;  // (one model: member 0, no lookup before its rows)
   const MemberParams pr = a.mp ? a.mp[m] : a.u;
   const float* dbeta_row = a.dbeta_rows + (long)m * Ny;
   const float* wind_row = a.wind_rows + (long)m * Ny;
@@ -319,17 +358,6 @@ __device__ __forceinline__ void qg_stage_weno(const StageArgs& a, int bx, int by
   const bool gx_ring = gx == Nx - 1;  // (gx >= 1)
   const bool bc = a.apply_bc != 0;
 
-  // This thread's outputs (rows wv + 4 r): the step-start value and the wind
-  // row are fetched first, so their latency overlaps the tile loads.
-  float qn_r[WY / 4], wind_r[WY / 4];
-#pragma unroll
-  for (int r = 0; r < WY / 4; ++r) {
-    const int gy = y0 + wv + 4 * r;
-    const bool ok = gy <= Ny - 2 && gx_out;
-    const int idx = gy * Nx + gx;  // plane < 2^31 cells
-    qn_r[r] = (ok && a.qn) ? a.qn[off + idx] : 0.0f;
-    wind_r[r] = ok ? wind_row[gy] : 0.0f;
-  }
   // Tile loads, all issued before the first LDS store so that one memory
   // latency covers them.  q with the boundary condition (ghost ring and
   // outside the array read 0), halo 3: the lane's own column for the wave's
@@ -370,10 +398,27 @@ __device__ __forceinline__ void qg_stage_weno(const StageArgs& a, int bx, int by
     vpe = inside ? psi[gy * Nx + hx] : 0.0f;
     pe_at = ly * PW2 + lx;
   }
+  // What the outputs of this thread (rows wv + 4 r of its column, and its
+  // ghost-ring point) need, then the member's rows.
+  PointIn pin[WY / 4], rin;
+  const int cgx = min(gx, Nx - 1);
+#pragma unroll
+  for (int r = 0; r < WY / 4; ++r) point_fetch<NEXT>(a, off + (long)min(y0 + wv + 4 * r, Ny - 1) * Nx + cgx, pin[r]);
+  int ry, rx;
+  ring_point<WY>(a, wv, tx, gx, y0, bx, by, nbx, nby, ry, rx);
+  const long ridx = off + (long)ry * Nx + rx;
+  float rq = 0.0f;
+  if (ry >= 0) {
+    rq = a.qs[ridx];
+    point_fetch<NEXT>(a, ridx, rin);
+  }
   if (tid < QH) {
     const int gy = y0 - 3 + tid;
     vdb = (gy >= 0 && gy < Ny) ? dbeta_row[gy] : 0.0f;
   }
+#pragma unroll
+  for (int r = 0; r < WY / 4; ++r) pin[r].wind = wind_row[min(y0 + wv + 4 * r, Ny - 1)];
+  rin.wind = wind_row[max(ry, 0)];
 #pragma unroll
   for (int k = 0; k < NQM; ++k)
     if (wv + 4 * k < QH) sq[(wv + 4 * k) * WQ + tx + 3] = vq[k];
@@ -482,18 +527,6 @@ __device__ __forceinline__ void qg_stage_weno(const StageArgs& a, int bx, int by
 
   const float wc = pr.tau0 * a.t.wind_scale[z];
   const bool bottom = (a.t.layer[z] == a.t.mnl[m] - 1) && (pr.kappa != 0.0f);
-  // Stage combination qn + c1 (qs - qn) + c2 rhs (the FP32 weights of the
-  // Shu-Osher form would otherwise not sum to 1); without qn: c1 qs + c2 rhs.
-  auto combine = [&](float qn, float qraw, float rhs) {
-    float o;
-    if (a.qn) {
-      o = qn + a.c1 * (qraw - qn) + a.c2 * rhs;
-    } else {
-      o = a.c2 * rhs;
-      if (a.c1 != 0.0f) o += a.c1 * qraw;
-    }
-    return o;
-  };
 #pragma unroll
   for (int r = 0; r < WY / 4; ++r) {
     const int ly = wv + 4 * r;
@@ -514,56 +547,25 @@ __device__ __forceinline__ void qg_stage_weno(const StageArgs& a, int bx, int by
       }
       if (bottom) rhs -= pr.kappa * ((p[1] - 2.0f * p[0] + p[-1]) * a.idx2 + (p[PW2] - 2.0f * p[0] + p[-PW2]) * a.idy2);
     }
-    rhs += wc * wind_r[r];
-    const long idx = off + (long)gy * Nx + gx;
-    a.out[idx] = combine(qn_r[r], sq[(ly + 3) * WQ + tx + 3], rhs);
+    rhs += wc * pin[r].wind;
+    point_store<NEXT>(a, off + (long)gy * Nx + gx, sq[(ly + 3) * WQ + tx + 3], rhs, pin[r]);
   }
-
-  // Ghost ring: no flux or viscous terms, only the wind row, and the raw
-  // stage value (the tile holds 0 there under the boundary condition).
-  // Wave 0: row 0 under the first tile row; wave 1: row Ny-1 under the last;
-  // wave 2: column 0 (lanes 0..WY-1, first tile column) and column Nx-1
-  // (lanes 32..32+WY-1, last tile column); wave 3: the four corners.
-  const bool first_x = bx == 0, last_x = bx == nbx - 1;
-  const bool first_y = by == 0, last_y = by == nby - 1;
-  int ry = -1, rx = -1;
-  if (wv == 0 && first_y && gx_out) {
-    ry = 0;
-    rx = gx;
-  } else if (wv == 1 && last_y && gx_out) {
-    ry = Ny - 1;
-    rx = gx;
-  } else if (wv == 2 && tx < WY && first_x && y0 + tx <= Ny - 2) {
-    ry = y0 + tx;
-    rx = 0;
-  } else if (wv == 2 && tx >= 32 && tx < 32 + WY && last_x && y0 + tx - 32 <= Ny - 2) {
-    ry = y0 + tx - 32;
-    rx = Nx - 1;
-  } else if (wv == 3 && tx < 4) {
-    const bool top = tx < 2, left = (tx & 1) == 0;
-    if ((top ? first_y : last_y) && (left ? first_x : last_x)) {
-      ry = top ? 0 : Ny - 1;
-      rx = left ? 0 : Nx - 1;
-    }
-  }
-  if (ry >= 0) {
-    const long idx = off + (long)ry * Nx + rx;
-    const float qn = a.qn ? a.qn[idx] : 0.0f;
-    a.out[idx] = combine(qn, a.qs[idx], wc * wind_row[ry]);
-  }
+  // Ghost ring: no flux or viscous terms, only the wind row, and the raw stage
+  // value (the tile holds 0 there under the boundary condition).
+  if (ry >= 0) point_store<NEXT>(a, ridx, rq, wc * rin.wind, rin);
 }
 
-template <bool BIHARM, int TY>
+template <bool BIHARM, int TY, bool NEXT>
 __global__ __launch_bounds__(256) void qg_stage_arakawa_kernel(StageArgs a) {
   int bx, by, z;
   xcd_tile3(bx, by, z);
-  qg_stage_arakawa<BIHARM, TY>(a, bx, by, z, gridDim.x, gridDim.y);
+  qg_stage_arakawa<BIHARM, TY, NEXT>(a, bx, by, z, gridDim.x, gridDim.y);
 }
-template <bool BIHARM>
+template <bool BIHARM, int WY, bool NEXT>
 __global__ __launch_bounds__(256) void qg_stage_weno_kernel(StageArgs a) {
   int bx, by, z;
   xcd_tile3(bx, by, z);
-  qg_stage_weno<BIHARM>(a, bx, by, z, gridDim.x, gridDim.y);
+  qg_stage_weno<BIHARM, WY, NEXT>(a, bx, by, z, gridDim.x, gridDim.y);
 }
 
 // Merged launch over the batches of a group: the tiles of all batches in one
@@ -584,39 +586,63 @@ __global__ __launch_bounds__(256) void qg_stage_weno_group_kernel(StageGroup g) 
   int c, l, bx, by, z;
   if (!table_class(g.t, blockIdx.x, c, l)) return;
   class_block(g.t, c, xcd_order(l, g.t.count[c]), bx, by, z);
-  qg_stage_weno<BIHARM>(g.a[c], bx, by, z, g.t.gx[c], g.t.gy[c]);
+  qg_stage_weno<BIHARM, WY_DEFAULT>(g.a[c], bx, by, z, g.t.gx[c], g.t.gy[c]);
 }
 
 namespace {
-dim3 stage_grid(const StageArgs& a) {
+// tiles of th rows over the interior
+dim3 stage_grid(const StageArgs& a, int th) {
   const int tw = a.advection == 1 ? WX : TX;
-  const int th = a.advection == 1 ? WY : (a.tile_rows ? a.tile_rows : TY_DEFAULT);
-  return dim3((a.Nx - 2 + tw - 1) / tw, (a.Ny - 2 + th - 1) / th, a.P);  // interior tiles
+  return dim3((a.Nx - 2 + tw - 1) / tw, (a.Ny - 2 + th - 1) / th, a.P);
+}
+int class_rows(const StageArgs& a) {
+  return a.advection == 1 ? WY_DEFAULT : (a.tile_rows ? a.tile_rows : TY_DEFAULT);
+}
+// Rows of a tile for one model: as many as leave the chip full.  Fewer rows per
+// thread make the block's chain of loads, LDS passes and stores shorter, more rows
+// read fewer halo rows.  Counted in tiles of 16 rows: up to one a CU, 4 rows
+// (128^2 x 3: 4.4 us against 5.2 with 8 and 7.2 with 16; WENO 256^2 x 3: 6.7, 7.9,
+// 9.9); up to four a CU, 8 (320^2 x 3: 6.1, 5.2, 7.8; 512^2 x 3: 10.0, 8.5, 8.9;
+// WENO 14.9, 12.4, 13.4); beyond, 16 (1024^2 x 3: 30.1, 21.4, 20.2; WENO 43.0,
+// 32.9, 31.7).  All heights give the same bits.  The classes of an ensemble keep
+// the height they report and let their caller set.
+int stage_rows(const StageArgs& a) {
+  if (a.mp) return class_rows(a);
+  const dim3 g = stage_grid(a, 16);
+  const long tiles = (long)g.x * g.y * g.z;
+  return tiles <= CUS ? 4 : (tiles <= 4 * CUS ? 8 : 16);
+}
+
+template <int TY, bool NEXT>
+void launch_stage(const StageArgs& a, hipStream_t st) {
+  const dim3 g = stage_grid(a, TY);
+  if (a.advection == 1) {
+    if (a.biharm) hipLaunchKernelGGL((qg_stage_weno_kernel<true, TY, NEXT>), g, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((qg_stage_weno_kernel<false, TY, NEXT>), g, dim3(256), 0, st, a);
+  } else {
+    if (a.biharm) hipLaunchKernelGGL((qg_stage_arakawa_kernel<true, TY, NEXT>), g, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((qg_stage_arakawa_kernel<false, TY, NEXT>), g, dim3(256), 0, st, a);
+  }
+}
+template <bool NEXT>
+void launch_stage(const StageArgs& a, hipStream_t st) {
+  const int th = stage_rows(a);
+  if (th == 4) launch_stage<4, NEXT>(a, st);
+  else if (th == 8) launch_stage<8, NEXT>(a, st);
+  else launch_stage<16, NEXT>(a, st);
 }
 }  // namespace
 
 void launch_qg_stage(const StageArgs& a, hipStream_t st) {
-  const dim3 g = stage_grid(a);
-  if (a.advection == 1) {
-    if (a.biharm) hipLaunchKernelGGL(qg_stage_weno_kernel<true>, g, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(qg_stage_weno_kernel<false>, g, dim3(256), 0, st, a);
-    return;
-  }
-  const int ty = a.tile_rows ? a.tile_rows : TY_DEFAULT;
-  if (ty == 8) {
-    if (a.biharm) hipLaunchKernelGGL((qg_stage_arakawa_kernel<true, 8>), g, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((qg_stage_arakawa_kernel<false, 8>), g, dim3(256), 0, st, a);
-  } else {
-    if (a.biharm) hipLaunchKernelGGL((qg_stage_arakawa_kernel<true, 16>), g, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((qg_stage_arakawa_kernel<false, 16>), g, dim3(256), 0, st, a);
-  }
+  if (a.next.out) launch_stage<true>(a, st);
+  else launch_stage<false>(a, st);
 }
 
 void launch_qg_stage_group(const StageArgs* a, int n, hipStream_t st) {
   StageGroup g{};
   for (int i = 0; i < n; ++i) {
     g.a[i] = a[i];
-    const dim3 d = stage_grid(a[i]);
+    const dim3 d = stage_grid(a[i], class_rows(a[i]));
     table_add(g.t, (int)d.x, (int)d.y, (int)d.z);
   }
   const dim3 grid(g.t.start[g.t.n]);
