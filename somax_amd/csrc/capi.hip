@@ -187,6 +187,7 @@ struct Batch {
   size_t off_DIAG = 0;  // FP64 partial sums of the diagnostics and the mass constraint
   size_t off_PWALL = 0;  // per-plane wall psi
   size_t ws_bytes = 0;
+  uint64_t hp_bits = 0;  // Poisson-like modes among the first 64 (t.hp)
   int stage_rows = 16;  // Arakawa stage tile height (8 or 16), chosen per class
   bool alone = true;    // false: a class of a concurrent ensemble, whose launches share the chip
   // mass correction: homogeneous solutions (P planes) and their means (0: none)
@@ -324,6 +325,7 @@ static hipError_t batch_build(Batch& b, const std::vector<const somaxhip_qg_desc
     P += nl;
   }
   b.P = P;
+  for (int m = 0; m < P && m < 64; ++m) b.hp_bits |= (uint64_t)hp[m] << m;
   b.first = mfirst;
   b.nl = mnl;
   int *dfirst, *dnl, *dmember, *dlayer;
@@ -689,7 +691,8 @@ void dst_solve_folded(const Batch& p, bool interior_input, int np_fwd, int np_in
       g.s_var = 3 * var;
     }
     g.lds = s.fld;
-    g.hp = p.t.hp;
+    g.hp = p.P <= 64 ? nullptr : p.t.hp;
+    g.hp_bits = p.hp_bits;
     g.np_lo = np_lo;
     g.np_hi = np_hi;
     g.fold_P = P;
@@ -805,7 +808,8 @@ void dst_solve(const Batch& p, bool interior_input, int np_fwd, int np_inv_lo, i
       g.s_piece = s.rows * s.ld;
     }
     g.lds = s.ld;
-    g.hp = p.t.hp;
+    g.hp = p.P <= 64 ? nullptr : p.t.hp;
+    g.hp_bits = p.hp_bits;
     g.np_lo = np_lo;
     g.np_hi = np_hi;
   };

@@ -74,18 +74,20 @@ __device__ inline void tile_of(int t, int GA, int GB, int& z, int& ta, int& tb) 
   tb = rem - ta * GB;
 }
 
-// Epilogue.  The 128 x 128 tile leaves through LDS in two halves of 64 rows
-// (the waves holding that half write their accumulators, FP64 running sum
-// added when SUM64), so global stores are wide and coalesced: FP32 outputs
-// with lanes along a row, bf16 pieces as 16-byte vectors of 8 columns.
-// `stage` needs 64 * EPI_PITCH floats of LDS; the caller's pipeline is done.
-constexpr int EPI_PITCH = 132;
+// Epilogue.  The tile leaves through LDS (the waves write their accumulators,
+// FP64 running sum added when SUM64), so global stores are wide and coalesced:
+// FP32 outputs with lanes along a row, bf16 pieces as 16-byte vectors of 8
+// columns.  SR rows at a time: all of them where the LDS allows, since every pass
+// is a chain of barrier, LDS write, barrier, LDS read and store (a x3 tile's
+// epilogue took 5 of 22 us at 1024^2 x 3 in two passes).  `stage` needs SR *
+// epi_pitch(BW) floats of LDS; the caller's pipeline is done.
+__host__ __device__ constexpr int epi_pitch(int bw) { return bw + 4; }
 
 // Eigenvalue rows of the spectral epilogue for one batch plane (null: none).
 struct Spectral {
   const float* lamA;
   const float* lamB;
-  float lamz;
+  const float* lamz;  // the mode's eigenvalue
 };
 
 // The spectral epilogue's eigenvalues of one tile (lamA of its 128 rows, then
@@ -100,22 +102,23 @@ __device__ inline float prefetch_spectral(const GemmArgs& a, const Spectral& sp,
 }
 
 // WN: waves along N; BW, BH: columns and rows of the tile (64 or 128).
-template <bool SUM64, int TM, int TN, int WN = 4 / TN, int BW = 128, int BH = 128>
+template <bool SUM64, int TM, int TN, int WN = 4 / TN, int BW = 128, int BH = 128, int SR = BH>
 __device__ inline void store_tile(const GemmArgs& a, long z, int a0, int b0, const floatx16 (&acc)[TM][TN],
                                   const double (&sum)[TM][TN][16], int opieces, float* stage, const Spectral& sp,
-                                  const float* lam = nullptr) {
+                                  const float* lam = nullptr, float lam_z = 0.0f) {
   constexpr int WM = BH / 32 / TM, NT = 64 * WM * WN;  // waves along M, threads
   constexpr int TPR = BW / 8;                    // threads per row of 8-column vectors
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
-  const float lamz = sp.lamz;
+  constexpr int PITCH = epi_pitch(BW);
+  const float lamz = lam ? lam_z : (sp.lamA ? *sp.lamz : 0.0f);
 #pragma unroll
-  for (int h = 0; h < BH / 64; ++h) {
-    __syncthreads();  // the LDS is free (pipeline drained / previous half stored)
-    if ((wm * 32 * TM) / 64 == h) {  // this wave's rows lie in half h
-      const int lr0 = (wm * 32 * TM) & 63;
+  for (int h = 0; h < BH / SR; ++h) {
+    __syncthreads();  // the LDS is free (pipeline drained / previous rows stored)
+    if ((wm * 32 * TM) / SR == h) {  // this wave's rows lie in pass h
+      const int lr0 = (wm * 32 * TM) % SR;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -124,18 +127,18 @@ __device__ inline void store_tile(const GemmArgs& a, long z, int a0, int b0, con
           for (int r = 0; r < 16; ++r) {
             const int lr = lr0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
             const int lc = wn * 32 * TN + j * 32 + (lane & 31);
-            stage[lr * EPI_PITCH + lc] = SUM64 ? (float)(sum[i][j][r] + (double)acc[i][j][r]) : acc[i][j][r];
+            stage[lr * PITCH + lc] = SUM64 ? (float)(sum[i][j][r] + (double)acc[i][j][r]) : acc[i][j][r];
           }
     }
     __syncthreads();
-    const int r0 = a0 + h * 64;
+    const int r0 = a0 + h * SR;
     if (opieces == 0) {
       // FP32 (any pitch): 64 lanes on 64 consecutive columns
-      for (int e = tid; e < 64 * BW; e += NT) {
+      for (int e = tid; e < SR * BW; e += NT) {
         const int lr = e / BW, lc = e % BW;
         const int ro = r0 + lr, co = b0 + lc;
         if (ro >= a.RA || co >= a.RBpad) continue;
-        float v = stage[lr * EPI_PITCH + lc];
+        float v = stage[lr * PITCH + lc];
         if (sp.lamA) v = v / (sp.lamA[ro] + sp.lamB[co < a.RB ? co : a.RB - 1] - lamz);
         a.Of[z * a.o_batch + (long)ro * a.ldo + co] = co < a.RB ? v : 0.0f;
       }
@@ -145,16 +148,16 @@ __device__ inline void store_tile(const GemmArgs& a, long z, int a0, int b0, con
       const int lc = (tid % TPR) * 8;
       const int co = b0 + lc;
 #pragma unroll
-      for (int k = 0; k < 64 / (NT / TPR); ++k) {
+      for (int k = 0; k < SR / (NT / TPR); ++k) {
         const int lr = tid / TPR + (NT / TPR) * k;
         const int ro = r0 + lr;
         if (ro >= a.RA || co >= a.RBpad) continue;
-        const floatx4 va = *reinterpret_cast<const floatx4*>(stage + lr * EPI_PITCH + lc);
-        const floatx4 vb = *reinterpret_cast<const floatx4*>(stage + lr * EPI_PITCH + lc + 4);
+        const floatx4 va = *reinterpret_cast<const floatx4*>(stage + lr * PITCH + lc);
+        const floatx4 vb = *reinterpret_cast<const floatx4*>(stage + lr * PITCH + lc + 4);
         float v[8] = {va[0], va[1], va[2], va[3], vb[0], vb[1], vb[2], vb[3]};
         // branch free per element (columns past RB are zero padding)
         if (sp.lamA) {
-          const float la = (lam ? lam[h * 64 + lr] : sp.lamA[ro]) - lamz;
+          const float la = (lam ? lam[h * SR + lr] : sp.lamA[ro]) - lamz;
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             const int c = co + e < a.RB ? co + e : a.RB - 1;
@@ -212,13 +215,13 @@ __device__ inline PlaneSel select_plane(const GemmArgs& a, long z) {
   s.s_off = a.fold_P ? (long)(a.s_par ? py : px) * a.s_var : 0;
   s.sp.lamA = a.lamA ? a.lamA + px * a.lam_var : nullptr;
   s.sp.lamB = a.lamB ? a.lamB + py * a.lamB_var : nullptr;
-  s.sp.lamz = a.lamA ? a.lam[s.m] : 0.0f;
+  s.sp.lamz = a.lam + s.m;
   return s;
 }
 
 // One output element of a launch: spectral division, then FP32 or bf16 pieces.
 __device__ inline void store_one(const GemmArgs& a, long z, int r, int c, float v, int opieces, const Spectral& sp) {
-  if (sp.lamA) v = v / (sp.lamA[r] + sp.lamB[c] - sp.lamz);
+  if (sp.lamA) v = v / (sp.lamA[r] + sp.lamB[c] - *sp.lamz);
   const long o = z * a.o_batch + (long)r * a.ldo + c;
   if (opieces == 0) {
     a.Of[o] = v;
@@ -812,11 +815,13 @@ __device__ inline void bf16_mainloop_pair(const GemmArgs& a, const uint16_t* S, 
 
 size_t dst_gemm_lds_bytes(int max_np, int bt) {
   const int npc = max_np == 1 ? 1 : (max_np == 3 ? 2 : 3);
-  return (size_t)bf16_nstage(npc, bt) * 2 * npc * bt * 32 * sizeof(uint16_t);
+  const size_t ring = (size_t)bf16_nstage(npc, bt) * 2 * npc * bt * 32 * sizeof(uint16_t);
+  return std::max(ring, (size_t)bt * epi_pitch(bt) * sizeof(float));  // the epilogue stages the tile
 }
 size_t dst_gemm_pair_lds_bytes(int max_np) {
   const int npc = max_np == 1 ? 1 : 2;
-  return (size_t)NSTAGE_P * npc * (128 + BNP) * 32 * sizeof(uint16_t);
+  const size_t ring = (size_t)NSTAGE_P * npc * (128 + BNP) * 32 * sizeof(uint16_t);
+  return std::max(ring, (size_t)128 * epi_pitch(BNP) * sizeof(float));
 }
 
 // Workgroup shape per instance: x1 / x3 run 16 waves of 32 x 32 (four per
@@ -838,6 +843,22 @@ struct KernelShape {
 __device__ inline int gemm_tiles(const GemmArgs& a, int bm, int bn) {
   const GemmCut cut = a.cut;
   return ((cut.am + bm - 1) / bm) * ((cut.bm + bn - 1) / bn) * a.nplanes;
+}
+
+// The arguments that a tile's first loads wait for, read from the argument segment
+// together: used where they are needed, they arrive in a dozen trips, one after the
+// other, before the first load is issued (1024^2 x 3 mixed step 793 -> 765 us with
+// the one-pass epilogue; 12 planes of 66^2, a x3 launch 7.9 -> 7.2).  The six-product
+// 64 x 64 tiles have no registers to hold them (512^2 diagnose 89.3 against 91.6 us).
+__device__ __forceinline__ void pin_args(GemmArgs& a) {
+  asm volatile("" : "+s"(a.Xb), "+s"(a.ldx), "+s"(a.x_piece), "+s"(a.x_batch), "+s"(a.xrows), "+s"(a.Sb), "+s"(a.lds),
+               "+s"(a.s_piece), "+s"(a.K), "+s"(a.trans), "+s"(a.hp), "+s"(a.hp_bits), "+s"(a.np_lo), "+s"(a.np_hi));
+  asm volatile("" : "+s"(a.fold_P), "+s"(a.s_par), "+s"(a.s_var), "+s"(a.lamA), "+s"(a.lamB), "+s"(a.lam),
+               "+s"(a.lam_var), "+s"(a.lamB_var), "+s"(a.op_lo), "+s"(a.op_hi), "+s"(a.RA), "+s"(a.RB));
+}
+// Whether mode m takes the low-precision side's products.
+__device__ __forceinline__ bool hp_mode(const GemmArgs& a, int m) {
+  return a.hp ? a.hp[m] != 0 : ((a.hp_bits >> m) & 1) != 0;
 }
 
 // Transforms of one launch: G == 1 for a single transform, else up to
@@ -873,7 +894,8 @@ void dst_gemm_bf16_kernel(GemmTable<G> g) {
   int c;
   const int lb = gemm_block<G, BT, BT>(g, c);
   if (lb < 0) return;
-  const GemmArgs& a = g.a[c];
+  GemmArgs a = g.a[c];
+  if constexpr (BT == 128 || NPMAX != 6) pin_args(a);
   const GemmCut cut = a.cut;
   const int GA = (cut.am + BT - 1) / BT, GB = (cut.bm + BT - 1) / BT;
   const int T = GA * GB * a.nplanes;
@@ -887,13 +909,13 @@ void dst_gemm_bf16_kernel(GemmTable<G> g) {
   }
   const long z = zi;
   const PlaneSel ps = select_plane(a, z);
-  const bool lo = a.hp && a.hp[ps.m];
+  const bool lo = hp_mode(a, ps.m);
   const int np = lo ? a.np_lo : a.np_hi;
   const int opieces = lo ? a.op_lo : a.op_hi;
   if (fringe) {
-    if (NPMAX == 1 || np == 1) gemm_fringe<false, 1, NT, BT == 64 ? 9 : 0>(a, z, part, cut, ps, opieces, lds16);
-    else if (NPMAX == 3 || np == 3) gemm_fringe<false, 2, NT, BT == 64 ? 9 : 0>(a, z, part, cut, ps, opieces, lds16);
-    else gemm_fringe<false, 3, NT, BT == 64 ? 5 : 0>(a, z, part, cut, ps, opieces, lds16);
+    if (NPMAX == 1 || np == 1) gemm_fringe<false, 1, NT, BT == 64 ? 9 : 0>(g.a[c], z, part, cut, ps, opieces, lds16);
+    else if (NPMAX == 3 || np == 3) gemm_fringe<false, 2, NT, BT == 64 ? 9 : 0>(g.a[c], z, part, cut, ps, opieces, lds16);
+    else gemm_fringe<false, 3, NT, BT == 64 ? 5 : 0>(g.a[c], z, part, cut, ps, opieces, lds16);
     return;
   }
   const int a0 = ta * BT;
@@ -904,6 +926,7 @@ void dst_gemm_bf16_kernel(GemmTable<G> g) {
   __shared__ float lam_tile[256];
   const bool spectral = ps.sp.lamA && opieces != 0;
   const float lam_pre = spectral ? prefetch_spectral(a, ps.sp, a0, b0) : 0.0f;
+  const float lam_z = spectral ? *ps.sp.lamz : 0.0f;
 
   floatx16 acc[TM][TN];
   double sum[TM][TN][16];
@@ -917,8 +940,8 @@ void dst_gemm_bf16_kernel(GemmTable<G> g) {
   float* stage = reinterpret_cast<float*>(lds16);
   if (spectral && threadIdx.x < 256) lam_tile[threadIdx.x] = lam_pre;  // read after store_tile's first barrier
   const float* lam = spectral ? lam_tile : nullptr;
-  if (NPMAX == 6 && np == 6 && a.acc64) store_tile<true, TM, TN, BT / 32 / TN, BT, BT>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam);
-  else store_tile<false, TM, TN, BT / 32 / TN, BT, BT>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam);
+  if (NPMAX == 6 && np == 6 && a.acc64) store_tile<true, TM, TN, BT / 32 / TN, BT, BT>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam, lam_z);
+  else store_tile<false, TM, TN, BT / 32 / TN, BT, BT>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam, lam_z);
 }
 
 
@@ -933,7 +956,8 @@ void dst_gemm_bf16_pair_kernel(GemmTable<G> g) {
   int c;
   const int lb = gemm_block<G, BM, BNP>(g, c);
   if (lb < 0) return;
-  const GemmArgs& a = g.a[c];
+  GemmArgs a = g.a[c];
+  pin_args(a);
   const GemmCut cut = a.cut;
   const int GA = (cut.am + BM - 1) / BM, GB = (cut.bm + BNP - 1) / BNP;
   const int T = GA * GB * a.nplanes;
@@ -947,12 +971,12 @@ void dst_gemm_bf16_pair_kernel(GemmTable<G> g) {
   }
   const long z = zi;
   const PlaneSel ps = select_plane(a, z);
-  const bool lo = a.hp && a.hp[ps.m];
+  const bool lo = hp_mode(a, ps.m);
   const int np = lo ? a.np_lo : a.np_hi;
   const int opieces = lo ? a.op_lo : a.op_hi;
   if (fringe) {
-    if (NPMAX == 1 || np == 1) gemm_fringe<false, 1, 512, 4>(a, z, part, cut, ps, opieces, lds16);
-    else gemm_fringe<false, 2, 512, 4>(a, z, part, cut, ps, opieces, lds16);
+    if (NPMAX == 1 || np == 1) gemm_fringe<false, 1, 512, 4>(g.a[c], z, part, cut, ps, opieces, lds16);
+    else gemm_fringe<false, 2, 512, 4>(g.a[c], z, part, cut, ps, opieces, lds16);
     return;
   }
   const int a0 = ta * BM;
@@ -963,6 +987,7 @@ void dst_gemm_bf16_pair_kernel(GemmTable<G> g) {
   __shared__ float lam_tile[256];
   const bool spectral = ps.sp.lamA && opieces != 0;
   const float lam_pre = spectral ? prefetch_spectral(a, ps.sp, a0, b0) : 0.0f;
+  const float lam_z = spectral ? *ps.sp.lamz : 0.0f;
   floatx16 acc[1][1];
   double sum[1][1][16];
   zero_acc<1, 1>(acc, sum);
@@ -971,7 +996,7 @@ void dst_gemm_bf16_pair_kernel(GemmTable<G> g) {
   float* stage = reinterpret_cast<float*>(lds16);
   if (spectral && threadIdx.x < 256) lam_tile[threadIdx.x] = lam_pre;  // read after store_tile's first barrier
   const float* lam = spectral ? lam_tile : nullptr;
-  store_tile<false, 1, 1, 2, BNP>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam);
+  store_tile<false, 1, 1, 2, BNP>(a, z, a0, b0, acc, sum, opieces, stage, ps.sp, lam, lam_z);
 }
 
 // ---------------------------------------------------------------------------
@@ -1093,8 +1118,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     }
     for (; kt < nk; ++kt) ktile(kt, acc);
   }
-  if (acc64) store_tile<true, 2, 2>(a, z, a0, b0, acc, sum, 0, lds, ps.sp);
-  else store_tile<false, 2, 2>(a, z, a0, b0, acc, sum, 0, lds, ps.sp);
+  if (acc64) store_tile<true, 2, 2, 2, 128, 128, 64>(a, z, a0, b0, acc, sum, 0, lds, ps.sp);
+  else store_tile<false, 2, 2, 2, 128, 128, 64>(a, z, a0, b0, acc, sum, 0, lds, ps.sp);
 }
 
 // 64 x 64 tiles of four 32 x 32 waves for launches of few tiles: k-tiles of 16

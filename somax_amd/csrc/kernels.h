@@ -161,9 +161,11 @@ struct GemmArgs {
   long lds, s_piece;
   int K;
   int trans;
-  // per plane precision: planes with hp[z] != 0 use np_lo products and write
-  // op_lo output pieces, the others np_hi / op_hi (pieces 0 = FP32 out)
+  // per plane precision: planes whose mode m has hp[m] != 0 use np_lo products
+  // and write op_lo output pieces, the others np_hi / op_hi (pieces 0 = FP32
+  // out).  hp null: bit m of hp_bits (launches of at most 64 modes).
   const unsigned char* hp;
+  uint64_t hp_bits;
   int np_lo, np_hi, op_lo, op_hi;
   int acc64;  // add the FP32 partial of every few k-tiles into an FP64 running sum
   // output O[ro][co], ro < RA, co < RB; columns [RB, RBpad) written as 0
