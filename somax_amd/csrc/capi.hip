@@ -48,6 +48,8 @@ struct SineSet {
   float* f32_fold = nullptr;
   uint16_t* b_fold = nullptr;
   float* lam_fold = nullptr;
+  // the bf16 operators that the y axis meets in dst_stripe, in fragment order
+  uint16_t *frag_full = nullptr, *frag_int = nullptr, *frag_fold = nullptr;
   std::vector<float> lam_host;
 };
 
@@ -151,6 +153,22 @@ static hipError_t build_fold(DeviceBlock& mem, SineSet& s) {
   if ((e = mem.upload(&s.f32_fold, ff)) != hipSuccess) return e;
   if ((e = mem.upload(&s.b_fold, bf)) != hipSuccess) return e;
   return mem.upload(&s.lam_fold, lf);
+}
+
+// Fragment-order copies of the bf16 operators (folded or plain).
+static hipError_t build_frags(DeviceBlock& mem, SineSet& s, bool fold) {
+  const long plain = 3 * s.rows * s.ld, folded = 4 * 3 * s.frows * s.fld;
+  hipError_t e = hipSuccess;
+  if (fold) {
+    if ((e = mem.alloc(&s.frag_fold, folded)) != hipSuccess) return e;
+    e = launch_fragment_order(s.b_fold, s.frag_fold, s.frows, s.fld, 12, nullptr);
+  } else {
+    if ((e = mem.alloc(&s.frag_full, plain)) != hipSuccess || (e = mem.alloc(&s.frag_int, plain)) != hipSuccess)
+      return e;
+    e = launch_fragment_order(s.b_full, s.frag_full, s.rows, s.ld, 3, nullptr);
+    if (e == hipSuccess) e = launch_fragment_order(s.b_int, s.frag_int, s.rows, s.ld, 3, nullptr);
+  }
+  return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
 }
 
 // Folded transforms halve the GEMM work; below h = 128 the four quarter
@@ -285,6 +303,10 @@ static hipError_t batch_build(Batch& b, const std::vector<const somaxhip_qg_desc
     if ((e = build_fold(b.mem, b.sy)) != hipSuccess) return e;
     b.fplane = (long)b.sx.h * b.sy.h;
   }
+  if ((b.precision == SOMAXHIP_PREC_MIXED || b.precision == SOMAXHIP_PREC_BF16X6) &&
+      std::max(b.fold ? b.sx.h : b.Nx, b.fold ? b.sy.h : b.Ny) <= STRIPE_MAX_N &&
+      (e = build_frags(b.mem, b.sy, b.fold != 0)) != hipSuccess)
+    return e;
 
   // Poisson-like modes (small lambda: the Laplacian's conditioning is not
   // capped) need the 3-piece inverse transform in the mixed solve.
@@ -390,20 +412,41 @@ static hipError_t batch_build(Batch& b, const std::vector<const somaxhip_qg_desc
     off += round_up((long)bytes, 256);
     return o;
   };
-  b.off_OP1 = take((size_t)opl * 3 * b.wpiece * sizeof(uint16_t));
-  b.off_OP2 = take((size_t)opl * 3 * b.wpiece * sizeof(uint16_t));
-  b.off_QM = take((size_t)P * b.splane * sizeof(float));
-  b.off_P0 = take((size_t)P * b.splane * sizeof(float));
-  // the direct form's scratch starts at OP1 and takes the room of these four
-  if (b.direct && off - b.off_OP1 < direct_bytes(b.Nx, b.Ny, P)) take(direct_bytes(b.Nx, b.Ny, P) - (off - b.off_OP1));
-  if (b.precision == SOMAXHIP_PREC_MIXED) b.off_D = take((size_t)P * b.splane * sizeof(float));
-  b.off_Q1 = take((size_t)P * b.splane * sizeof(float));
-  b.off_Q2 = take((size_t)P * b.splane * sizeof(float));
-  b.off_PSI = take((size_t)P * b.splane * sizeof(float));
-  b.off_DIAG = take(qg_diag_partial_doubles(b.Nx, b.Ny, P) * sizeof(double));
-  b.off_PWALL = take((size_t)P * sizeof(float));
-  b.ws_bytes = off;
-  return prepare_dst_gemm();
+  auto layout = [&] {
+    off = 0;
+    b.off_OP1 = take((size_t)opl * 3 * b.wpiece * sizeof(uint16_t));
+    b.off_OP2 = take((size_t)opl * 3 * b.wpiece * sizeof(uint16_t));
+    b.off_QM = take((size_t)P * b.splane * sizeof(float));
+    b.off_P0 = take((size_t)P * b.splane * sizeof(float));
+    // the direct form's scratch starts at OP1 and takes the room of these four
+    if (b.direct && off - b.off_OP1 < direct_bytes(b.Nx, b.Ny, P)) take(direct_bytes(b.Nx, b.Ny, P) - (off - b.off_OP1));
+    if (b.precision == SOMAXHIP_PREC_MIXED) b.off_D = take((size_t)P * b.splane * sizeof(float));
+    b.off_Q1 = take((size_t)P * b.splane * sizeof(float));
+    b.off_Q2 = take((size_t)P * b.splane * sizeof(float));
+    b.off_PSI = take((size_t)P * b.splane * sizeof(float));
+    b.off_DIAG = take(qg_diag_partial_doubles(b.Nx, b.Ny, P) * sizeof(double));
+    b.off_PWALL = take((size_t)P * sizeof(float));
+    b.ws_bytes = off;
+  };
+  // An operand in fragment order is padded to tiles of 32 in both extents.  A plan
+  // that fits the scratch of the no-allocation step only without that padding keeps
+  // the launches of single transforms.
+  const long plain = b.wpiece;
+  const bool frags = b.sy.frag_fold || b.sy.frag_full;
+  if (frags) b.wpiece = std::max(plain, round_up(b.fold ? b.sx.h : b.Nx, 32) * round_up(b.fold ? b.sy.h : b.Ny, 32));
+  layout();
+  if (const long grown = b.wpiece; grown > plain && b.ws_bytes > (size_t)SOMAXHIP_NOALLOC_SCRATCH_BYTES) {
+    b.wpiece = plain;
+    layout();
+    if (b.ws_bytes <= (size_t)SOMAXHIP_NOALLOC_SCRATCH_BYTES) {
+      b.sy.frag_fold = b.sy.frag_full = b.sy.frag_int = nullptr;
+    } else {
+      b.wpiece = grown;
+      layout();
+    }
+  }
+  e = prepare_dst_gemm();
+  return e == hipSuccess ? prepare_dst_stripe() : e;
 }
 
 static MemberParams to_member_params(const somaxhip_qg_params& p) {
@@ -637,20 +680,22 @@ void gemm(const GemmArgs& a, int batch, hipStream_t st) {
 // Products of a GEMM class: NP_F32 selects the FP32 kernels; 1, 3, 6 bf16.
 constexpr int NP_F32 = 0;
 
-// The four transforms of one solve (F1, F2, I1, I2) with their batch sizes,
-// recorded instead of launched when a merged launch will carry them.
+// The four transforms of one solve (F1, F2, I1, I2) with their batch sizes.
 struct SolveGemms {
   GemmArgs g[4];
   int batch[4];
 };
-// Launch transform k of a solve, or record it into `rec`.
-inline void emit_gemm(const GemmArgs& a, int batch, int k, SolveGemms* rec, hipStream_t st) {
-  if (rec) {
-    rec->g[k] = a;
-    rec->batch[k] = batch;
-    return;
+// The launches of a solve of one batch.
+void launch_solve(const SolveGemms& s, bool stripe, hipStream_t st) {
+  int k = 0;
+  if (stripe) {
+    double flops = 0.0;
+    for (int i = 0; i < 3; ++i) flops += 2.0 * s.g[i].RA * s.g[i].RB * s.g[i].K * s.batch[i];
+    ProfScope ps("dst_stripe", flops, 8.0 * s.batch[0] * (double)s.g[0].RA * s.g[0].RB, st);
+    launch_dst_stripe(s.g[0], s.g[1], s.g[2], s.batch[0], st);
+    k = 3;
   }
-  gemm(a, batch, st);
+  for (; k < 4; ++k) gemm(s.g[k], s.batch[k], st);
 }
 inline int pieces_for(int np) { return np == 1 ? 1 : (np == 3 ? 2 : 3); }
 
@@ -659,7 +704,7 @@ inline int pieces_for(int np) { return np == 1 ? 1 : (np == 3 ? 2 : 3); }
 // pair, last in the folded order, is zero and skipped).  Out: `out` receives
 // the parity components of the solution, 4P planes of hy x hx.
 void dst_solve_folded(const Batch& p, bool interior_input, int np_fwd, int np_inv_lo, int np_inv_hi, float* out,
-                      void* ws, hipStream_t st, bool acc64_fwd, bool acc64_inv, SolveGemms* rec) {
+                      void* ws, bool acc64_fwd, bool acc64_inv, SolveGemms& rec) {
   const int hx = p.sx.h, hy = p.sy.h, P = p.P;
   const bool f32 = np_fwd == NP_F32;
   char* OP1 = static_cast<char*>(ws) + p.off_OP1;
@@ -687,6 +732,7 @@ void dst_solve_folded(const Batch& p, bool interior_input, int np_fwd, int np_in
       g.x_piece = p.wpiece;
       g.x_batch = pb16;
       g.Sb = s.b_fold + (inverse ? 2 * 3 * var : 0);
+      g.Sfrag = s.frag_fold ? s.frag_fold + (inverse ? 2 * 3 * var : 0) : nullptr;
       g.s_piece = var;
       g.s_var = 3 * var;
     }
@@ -724,7 +770,8 @@ void dst_solve_folded(const Batch& p, bool interior_input, int np_fwd, int np_in
   g.RA = hx;
   g.RB = R0;
   g.RBpad = (int)round_up(R0, 32);
-  emit_gemm(g, 4 * P, 0, rec, st);
+  rec.g[0] = g;
+  rec.batch[0] = 4 * P;
 
   // F2: W[ix][iy] = sum_y' T[ix][y'] Sy_p[iy][y'] / (lamx_q[ix] + lamy_p[iy] - lambda)
   GemmArgs h{};
@@ -740,7 +787,8 @@ void dst_solve_folded(const Batch& p, bool interior_input, int np_fwd, int np_in
   h.lam_var = hx;
   h.lamB_var = hy;
   h.lam = p.t.lam;
-  emit_gemm(h, 4 * P, 1, rec, st);
+  rec.g[1] = h;
+  rec.batch[1] = 4 * P;
 
   // I1: V[y'][ix] = sum_iy Sy_p^T[y'][iy] W[ix][iy]
   GemmArgs u{};
@@ -751,7 +799,8 @@ void dst_solve_folded(const Batch& p, bool interior_input, int np_fwd, int np_in
   u.RA = hy;
   u.RB = hx;
   u.RBpad = (int)round_up(hx, 32);
-  emit_gemm(u, 4 * P, 2, rec, st);
+  rec.g[2] = u;
+  rec.batch[2] = 4 * P;
 
   // I2: out[y'][x'] = sum_ix V[y'][ix] Sx_q^T[x'][ix]
   GemmArgs w{};
@@ -766,7 +815,8 @@ void dst_solve_folded(const Batch& p, bool interior_input, int np_fwd, int np_in
   w.RA = hy;
   w.RB = hx;
   w.RBpad = hx;
-  emit_gemm(w, 4 * P, 3, rec, st);
+  rec.g[3] = w;
+  rec.batch[3] = 4 * P;
 }
 
 // One DST-I solve per plane of (lap_h - lambda_z) y_z = x_z, from the GEMM
@@ -776,9 +826,9 @@ void dst_solve_folded(const Batch& p, bool interior_input, int np_fwd, int np_in
 // components).  np_fwd: products of the forward transforms; np_inv_lo /
 // np_inv_hi: products of the inverse transforms of Poisson-like / other planes.
 void dst_solve(const Batch& p, bool interior_input, int np_fwd, int np_inv_lo, int np_inv_hi, float* out,
-               void* ws, hipStream_t st, bool acc64_fwd = true, bool acc64_inv = true, SolveGemms* rec = nullptr) {
+               void* ws, SolveGemms& rec, bool acc64_fwd = true, bool acc64_inv = true) {
   if (p.fold) {
-    dst_solve_folded(p, interior_input, np_fwd, np_inv_lo, np_inv_hi, out, ws, st, acc64_fwd, acc64_inv, rec);
+    dst_solve_folded(p, interior_input, np_fwd, np_inv_lo, np_inv_hi, out, ws, acc64_fwd, acc64_inv, rec);
     return;
   }
   const int Nx = p.Nx, Ny = p.Ny, P = p.P;
@@ -805,6 +855,7 @@ void dst_solve(const Batch& p, bool interior_input, int np_fwd, int np_inv_lo, i
       g.x_piece = p.wpiece;
       g.x_batch = pb16;
       g.Sb = interior_s ? s.b_int : s.b_full;
+      g.Sfrag = interior_s ? s.frag_int : s.frag_full;
       g.s_piece = s.rows * s.ld;
     }
     g.lds = s.ld;
@@ -839,7 +890,8 @@ void dst_solve(const Batch& p, bool interior_input, int np_fwd, int np_inv_lo, i
   g.RA = Nx;
   g.RB = R0;
   g.RBpad = (int)round_up(R0, 32);
-  emit_gemm(g, P, 0, rec, st);
+  rec.g[0] = g;
+  rec.batch[0] = P;
 
   // F2: W[xm][ym] = sum_y T[xm][y] Sy[ym][y] / (lamx + lamy - lambda)
   GemmArgs h{};
@@ -853,7 +905,8 @@ void dst_solve(const Batch& p, bool interior_input, int np_fwd, int np_inv_lo, i
   h.lamA = p.sx.lam;
   h.lamB = p.sy.lam;
   h.lam = p.t.lam;
-  emit_gemm(h, P, 1, rec, st);
+  rec.g[1] = h;
+  rec.batch[1] = P;
 
   // I1: V[y][xm] = sum_ym Sy[y][ym] W[xm][ym]        (S in the A slot)
   GemmArgs u{};
@@ -864,7 +917,8 @@ void dst_solve(const Batch& p, bool interior_input, int np_fwd, int np_inv_lo, i
   u.RA = Ny;
   u.RB = Nx;
   u.RBpad = (int)round_up(Nx, 32);
-  emit_gemm(u, P, 2, rec, st);
+  rec.g[2] = u;
+  rec.batch[2] = P;
 
   // I2: out[y][x] = sum_xm V[y][xm] Sx[x][xm]
   GemmArgs w{};
@@ -879,7 +933,8 @@ void dst_solve(const Batch& p, bool interior_input, int np_fwd, int np_inv_lo, i
   w.RA = Ny;
   w.RB = Nx;
   w.RBpad = Nx;
-  emit_gemm(w, P, 3, rec, st);
+  rec.g[3] = w;
+  rec.batch[3] = P;
 }
 
 // Arguments of the inversion's kernels for one batch.
@@ -999,27 +1054,41 @@ void invert(const Batch& p, Solve what, const float* q, float* psi, void* ws, hi
   const bool mixed = p.precision == SOMAXHIP_PREC_MIXED;
   const bool x6 = p.precision == SOMAXHIP_PREC_BF16X6;
   float* P0 = wsf(ws, p.off_P0);
-  {
-    const ModalArgs ma = modal_args(p, q, ws, apply_bc);
-    ProfScope ps("to_modal", 0.0, 8.0 * p.P * (double)p.splane, st);
-    launch_to_modal(ma, st);
-  }
+  SolveGemms solve{};
   if (x6) {
     // three-piece operands, six products and FP64 flushes in every transform:
     // about 2^-24 per product, accurate without a refinement pass
-    dst_solve(p, apply_bc, 6, 6, 6, P0, ws, st);
+    dst_solve(p, apply_bc, 6, 6, 6, P0, ws, solve);
   } else if (!mixed) {
-    dst_solve(p, apply_bc, NP_F32, NP_F32, NP_F32, P0, ws, st);
+    dst_solve(p, apply_bc, NP_F32, NP_F32, NP_F32, P0, ws, solve);
   } else {
     // bf16x3 forward, x6 (Poisson-like modes) / x3 inverse; FP32 per-mode
     // Helmholtz residual; correction with bf16x3 forward and bf16 inverse.
-    dst_solve(p, apply_bc, 3, 6, 3, P0, ws, st);
+    dst_solve(p, apply_bc, 3, 6, 3, P0, ws, solve);
+  }
+  {
+    // Stripes wherever they fit (dst_stripe.hip has both sides' figures); they take
+    // their operand in fragment order.  Merged ensembles launch the transforms one by
+    // one, each for all classes.
+    const bool stripe = dst_stripe_fits(solve.g[0], solve.g[1], solve.g[2]);
+    ModalArgs ma = modal_args(p, q, ws, apply_bc);
+    ma.op_frag = stripe;
     {
-      const ResidualArgs r = residual_args(p, ws);
+      ProfScope ps("to_modal", 0.0, 8.0 * p.P * (double)p.splane, st);
+      launch_to_modal(ma, st);
+    }
+    launch_solve(solve, stripe, st);
+  }
+  if (mixed) {
+    dst_solve(p, false, 3, 1, 1, wsf(ws, p.off_D), ws, solve = SolveGemms{}, true, false);
+    const bool stripe = dst_stripe_fits(solve.g[0], solve.g[1], solve.g[2]);
+    ResidualArgs r = residual_args(p, ws);
+    r.op_frag = stripe;
+    {
       ProfScope ps("residual", 0.0, 12.0 * p.P * (double)p.splane, st);
       launch_residual(r, st);
     }
-    dst_solve(p, false, 3, 1, 1, wsf(ws, p.off_D), ws, st, true, false);
+    launch_solve(solve, stripe, st);
   }
   LayerArgs la = layer_args(p, psi, ws, mixed);
   if (p.any_mass) {
@@ -1075,8 +1144,8 @@ void invert_group(const std::vector<GroupItem>& it, hipStream_t st) {
     SolveGemms rec[MAX_GROUP];
     for (int i = 0; i < n; ++i) {
       const Batch& p = *it[i].b;
-      dst_solve(p, interior, npf, npl, nph, wsf(it[i].ws, correction ? p.off_D : p.off_P0), it[i].ws, st, acc64f,
-                acc64i, &rec[i]);
+      dst_solve(p, interior, npf, npl, nph, wsf(it[i].ws, correction ? p.off_D : p.off_P0), it[i].ws, rec[i], acc64f,
+                acc64i);
     }
     for (int k = 0; k < 4; ++k) {
       GemmArgs g[MAX_GROUP];

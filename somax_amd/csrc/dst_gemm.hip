@@ -848,8 +848,7 @@ __device__ inline int gemm_tiles(const GemmArgs& a, int bm, int bn) {
 // The arguments that a tile's first loads wait for, read from the argument segment
 // together: used where they are needed, they arrive in a dozen trips, one after the
 // other, before the first load is issued (1024^2 x 3 mixed step 793 -> 765 us with
-// the one-pass epilogue; 12 planes of 66^2, a x3 launch 7.9 -> 7.2).  The six-product
-// 64 x 64 tiles have no registers to hold them (512^2 diagnose 89.3 against 91.6 us).
+// the one-pass epilogue).  The six-product 64 x 64 tiles have no registers to hold them (512^2 diagnose 89.3 against 91.6 us).
 __device__ __forceinline__ void pin_args(GemmArgs& a) {
   asm volatile("" : "+s"(a.Xb), "+s"(a.ldx), "+s"(a.x_piece), "+s"(a.x_batch), "+s"(a.xrows), "+s"(a.Sb), "+s"(a.lds),
                "+s"(a.s_piece), "+s"(a.K), "+s"(a.trans), "+s"(a.hp), "+s"(a.hp_bits), "+s"(a.np_lo), "+s"(a.np_hi));

@@ -158,6 +158,7 @@ struct GemmArgs {
   // sine operand S: rows padded to 128, k zero padded to 32
   const float* Sf;
   const uint16_t* Sb;
+  const uint16_t* Sfrag;  // Sb in fragment order (null: not kept)
   long lds, s_piece;
   int K;
   int trans;
@@ -215,6 +216,24 @@ void launch_dst_gemm_group(const GemmArgs* a, const int* batch, int n, hipStream
 // Raises the bf16 kernel's dynamic LDS limit; call before the first launch.
 hipError_t prepare_dst_gemm();
 
+// The first three transforms of a solve (F1, F2, I1 of dst_stripe.hip) in one
+// launch over `batch` planes: whether they can be, and the launch.  The same bits
+// as three launches of launch_dst_gemm.
+constexpr int STRIPE_MAX_N = 258;  // the largest extent: eight tiles of 32 rows and two rows past them
+bool dst_stripe_fits(const GemmArgs& f1, const GemmArgs& f2, const GemmArgs& i1);
+void launch_dst_stripe(const GemmArgs& f1, const GemmArgs& f2, const GemmArgs& i1, int batch, hipStream_t st);
+hipError_t prepare_dst_stripe();
+// `matrices` consecutive rows x ld bf16 matrices of src, in fragment order
+hipError_t launch_fragment_order(const uint16_t* src, uint16_t* dst, long rows, long ld, int matrices, hipStream_t st);
+
+// Fragment order of a rows x k bf16 operand (k padded to ld, a multiple of 32): 32-row
+// tiles of k16 steps, each the 64 lanes' 8 elements (row lane & 31, k half lane >> 5),
+// so that a fragment is one contiguous KiB.  Fragments of row-major rows are 32 bytes
+// of 32 lines each, and a load of one took four times as long (a stripe of 512^2 x 3,
+// six products: 54 -> 41 us).  Element (row, k) is at frag_row + frag_col.
+__host__ __device__ inline long frag_row(int row, long ld) { return (row >> 5) * (ld >> 4) * 512 + (row & 31) * 8; }
+__host__ __device__ inline int frag_col(int k) { return (k >> 4) * 512 + ((k >> 3) & 1) * 256 + (k & 7); }
+
 // Layer -> mode projection with FP64 accumulation (the stretching term makes
 // layer PV much larger than the barotropic modal PV, so an FP32 sum cancels):
 //   qm[first + p] = sum_k cl2m[p][k] * q[first + k]   (ghost ring of q read as 0 when apply_bc)
@@ -230,6 +249,7 @@ struct ModalArgs {
   Tables t;
   void* op;
   int op_pieces;
+  int op_frag;  // the operand in fragment order, k padded to op_kpad
   long op_ld, op_piece, op_batch;
   int op_kpad;
   // folded layout (fold != 0): qm and op hold, for block b = 2p + q of table
@@ -258,6 +278,7 @@ struct ResidualArgs {
   uint16_t* r;
   long op_ld, op_piece, op_batch;
   int op_kpad;
+  int op_frag;  // as ModalArgs
   long plane;
   int Nx, Ny, P;
   float idx2, idy2;

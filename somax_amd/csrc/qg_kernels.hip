@@ -705,7 +705,7 @@ __device__ __forceinline__ void residual_plain(const ResidualArgs& a, int bx, in
   const int i = bx * blockDim.x + threadIdx.x;
   const int y = i / a.op_kpad, x = i - y * a.op_kpad;
   if (y >= a.Ny) return;
-  uint16_t* o = a.r + z * a.op_batch + (long)y * a.op_ld + x;
+  uint16_t* o = a.r + z * a.op_batch + (a.op_frag ? frag_row(y, a.op_kpad) + frag_col(x) : (long)y * a.op_ld + x);
   if (x >= a.Nx) {
     store_pieces(o, a.op_piece, 2, 0.0f);
     return;
@@ -740,9 +740,10 @@ __device__ __forceinline__ void residual_fold(const ResidualArgs& a, int bx, int
   const int ky0 = (bry * 4 + wv) * RES_ROWS;
   if (kx >= a.op_kpad || ky0 >= hy) return;
   const int kend = ky0 + RES_ROWS < hy ? ky0 + RES_ROWS : hy;
-  uint16_t* o = a.r + z * a.op_batch + kx;
+  uint16_t* o = a.r + z * a.op_batch + (a.op_frag ? frag_col(kx) : kx);
+  auto row_at = [&](int k) { return a.op_frag ? frag_row(k, a.op_kpad) : (long)k * a.op_ld; };
   if (kx >= hx) {
-    for (int ky = ky0; ky < kend; ++ky) store_pieces(o + (long)ky * a.op_ld, a.op_piece, 2, 0.0f);
+    for (int ky = ky0; ky < kend; ++ky) store_pieces(o + row_at(ky), a.op_piece, 2, 0.0f);
     return;
   }
   const int blk = z / a.P, m = z - blk * a.P;
@@ -777,7 +778,7 @@ __device__ __forceinline__ void residual_fold(const ResidualArgs& a, int bx, int
     // rounding does not depend on the compiler's contraction choices
     const float lap = __builtin_fmaf(e - 2.0f * c + w, a.idx2, (n - 2.0f * c + so) * a.idy2);
     const float res = qv - 4.0f * (lap - lam * c);
-    store_pieces(o + (long)ky * a.op_ld, a.op_piece, 2, res);
+    store_pieces(o + row_at(ky), a.op_piece, 2, res);
     below = cur;
     cur = above;
   }
@@ -867,7 +868,7 @@ __device__ __forceinline__ void to_modal_plain(const ModalArgs& a, int bx, int m
     if (inside) a.qm[z * a.plane + s] = v;
     if (wop) {
       const float w = ox < cols ? v : 0.0f;  // zero padding past the operand width
-      const long o = z * a.op_batch + (long)oy * a.op_ld + ox;
+      const long o = z * a.op_batch + (a.op_frag ? frag_row(oy, a.op_kpad) + frag_col(ox) : (long)oy * a.op_ld + ox);
       if (a.op_pieces == 0) static_cast<float*>(a.op)[o] = w;
       else store_pieces(static_cast<uint16_t*>(a.op) + o, a.op_piece, a.op_pieces, w);
     }
@@ -932,7 +933,7 @@ __device__ __forceinline__ void to_modal_fold(const ModalArgs& a, int bx, int me
       if (inside) a.qm[z * fplane + (long)ky * hx + kx] = fv;
       if (wop) {
         const float w = kx < K0 ? fv : 0.0f;  // zero padding past the operand width
-        const long o = z * a.op_batch + (long)ky * a.op_ld + kx;
+        const long o = z * a.op_batch + (a.op_frag ? frag_row(ky, a.op_kpad) + frag_col(kx) : (long)ky * a.op_ld + kx);
         if (a.op_pieces == 0) static_cast<float*>(a.op)[o] = w;
         else store_pieces(static_cast<uint16_t*>(a.op) + o, a.op_piece, a.op_pieces, w);
       }
