@@ -604,10 +604,10 @@ int class_rows(const StageArgs& a) {
 // (128^2 x 3: 4.4 us against 5.2 with 8 and 7.2 with 16; WENO 256^2 x 3: 6.7, 7.9,
 // 9.9); up to four a CU, 8 (320^2 x 3: 6.1, 5.2, 7.8; 512^2 x 3: 10.0, 8.5, 8.9;
 // WENO 14.9, 12.4, 13.4); beyond, 16 (1024^2 x 3: 30.1, 21.4, 20.2; WENO 43.0,
-// 32.9, 31.7).  All heights give the same bits.  The classes of an ensemble keep
-// the height they report and let their caller set.
+// 32.9, 31.7).  All heights give the same bits.  The Arakawa classes of an ensemble
+// keep the height they report and let their caller set.
 int stage_rows(const StageArgs& a) {
-  if (a.mp) return class_rows(a);
+  if (a.mp && a.advection != 1) return class_rows(a);
   const dim3 g = stage_grid(a, 16);
   const long tiles = (long)g.x * g.y * g.z;
   return tiles <= CUS ? 4 : (tiles <= 4 * CUS ? 8 : 16);
