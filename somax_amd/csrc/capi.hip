@@ -248,13 +248,18 @@ inline bool use_direct(const Batch& p, Solve what) {
 // FP64 rate from the start.  Measured (an SSP-RK3 step of 3-layer members, us,
 // split -> direct): FP32 64^2 x 4 265 -> 114, 128^2 x 64 634 -> 483, 256^2 x 8
 // 410 -> 330, 256^2 x 32 (F = 6.6e9) 939 -> 960, 512^2 x 2 (3.3e9) 516 -> 471,
-// 512^2 x 4 (6.5e9) 575 -> 772; six products 256^2 x 8 (1.65e9) 363 -> 332,
-// 512^2 x 1 (1.63e9) 345 -> 314, 512^2 x 2 369 -> 472.
+// 512^2 x 4 (6.5e9) 575 -> 772; six products on a grid past the stripes' (F up to
+// 1.8e9) 345 -> 314.  Where six products run as stripes (stripes -> direct): 64^2 x
+// 1 129 -> 107, 128^2 x 4 (1.1e8) 157 -> 123, 256^2 x 1 (2.1e8) 160 -> 163, 64^2 x
+// 96 (3.3e8) 247 -> 261, 320^2 x 1 (4.0e8) 179 -> 193, 256^2 x 4 (8.2e8) 200 -> 219,
+// 512^2 x 1 (1.6e9) 254 -> 292.
 static bool direct_pays(int Nx, int Ny, int P, int precision) {
   if (!direct_fits(Nx, Ny)) return false;
   const double hx = (Nx + 1) / 2, hy = (Ny + 1) / 2;
   const double F = 16.0 * P * hx * hy * (hx + hy);
-  return F <= (precision == SOMAXHIP_PREC_BF16X6 ? 1.8e9 : 4.0e9);
+  if (precision != SOMAXHIP_PREC_BF16X6) return F <= 4.0e9;
+  const int fold = use_fold(Nx, Ny) ? 2 : 1;
+  return F <= (std::max(Nx, Ny) / fold <= STRIPE_MAX_N ? 3.0e8 : 1.8e9);
 }
 
 // Checks one model description; empty string when valid.
