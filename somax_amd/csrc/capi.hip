@@ -30,7 +30,9 @@ static long round_up(long v, long m) { return (v + m - 1) / m * m; }
 // tiles never read out of bounds: rows to a multiple of 128, pitch to a
 // multiple of 32 elements.  "full" is S[n][k]; "int" is S[n][k+1] (the
 // columns that meet the interior points when the ghost ring is zero).  The
-// bf16 copies hold three pieces S = s0 + s1 + s2 (piece stride rows*ld).
+// bf16 copies hold three pieces S = s0 + s1 + s2 (piece stride rows*ld).  A plan
+// holds the form that its transforms read (SineForm), once for axes of one length:
+// every form of both axes was most of a plan's creation (3 x 1024^2, 52 ms).
 struct SineSet {
   int N = 0;
   long ld = 0, rows = 0;
@@ -88,25 +90,17 @@ static void split3(double v, uint16_t* p, long stride) {
   p[2 * stride] = f32_to_bf16_bits((float)r2);
 }
 
-static hipError_t build_sines(DeviceBlock& mem, SineSet& s, int N, double d) {
+// The operators that a plan's transforms read: FP32 or bf16 pieces, plain or folded.
+struct SineForm {
+  bool f32, fold;
+};
+
+// The axis' eigenvalues and, for plain transforms, its matrices; `same`: an axis of
+// as many points, whose matrices are shared.
+static hipError_t build_sines(DeviceBlock& mem, SineSet& s, int N, double d, SineForm form, const SineSet* same) {
   s.N = N;
   s.ld = round_up(N, 32);
   s.rows = round_up(N, 128);
-  const size_t count = (size_t)s.rows * s.ld;
-  std::vector<float> ff(count, 0.0f), fi(count, 0.0f);
-  std::vector<uint16_t> bf(3 * count, 0), bi(3 * count, 0);
-  const double c = std::sqrt(2.0 / (N + 1));
-  for (int n = 0; n < N; ++n)
-    for (int k = 0; k < N; ++k) {
-      const double v = c * std::sin(M_PI * (double)(n + 1) * (double)(k + 1) / (double)(N + 1));
-      const size_t o = (size_t)n * s.ld + k;
-      ff[o] = (float)v;
-      split3(v, &bf[o], (long)count);
-      if (k >= 1 && k <= N - 2) {
-        fi[o - 1] = (float)v;
-        split3(v, &bi[o - 1], (long)count);
-      }
-    }
   std::vector<float> lam(N);
   s.lam_min = 1e300;
   s.lam_max = 0.0;
@@ -116,43 +110,85 @@ static hipError_t build_sines(DeviceBlock& mem, SineSet& s, int N, double d) {
     s.lam_min = std::fabs(l) < s.lam_min ? std::fabs(l) : s.lam_min;
     s.lam_max = std::fabs(l) > s.lam_max ? std::fabs(l) : s.lam_max;
   }
-  hipError_t e;
-  if ((e = mem.upload(&s.f32_full, ff)) != hipSuccess) return e;
-  if ((e = mem.upload(&s.f32_int, fi)) != hipSuccess) return e;
-  if ((e = mem.upload(&s.b_full, bf)) != hipSuccess) return e;
-  if ((e = mem.upload(&s.b_int, bi)) != hipSuccess) return e;
   s.lam_host = lam;
-  return mem.upload(&s.lam, lam);
+  const hipError_t up = mem.upload(&s.lam, lam);
+  if (up != hipSuccess || form.fold) return up;
+  if (same) {
+    s.f32_full = same->f32_full;
+    s.f32_int = same->f32_int;
+    s.b_full = same->b_full;
+    s.b_int = same->b_int;
+    return hipSuccess;
+  }
+  const size_t count = (size_t)s.rows * s.ld;
+  std::vector<float> ff, fi;
+  std::vector<uint16_t> bf, bi;
+  if (form.f32) {
+    ff.assign(count, 0.0f);
+    fi.assign(count, 0.0f);
+  } else {
+    bf.assign(3 * count, 0);
+    bi.assign(3 * count, 0);
+  }
+  const double c = std::sqrt(2.0 / (N + 1));
+  for (int n = 0; n < N; ++n)
+    for (int k = 0; k < N; ++k) {
+      const double v = c * std::sin(M_PI * (double)(n + 1) * (double)(k + 1) / (double)(N + 1));
+      const size_t o = (size_t)n * s.ld + k;
+      const bool in = k >= 1 && k <= N - 2;
+      if (form.f32) {
+        ff[o] = (float)v;
+        if (in) fi[o - 1] = (float)v;
+      } else {
+        split3(v, &bf[o], (long)count);
+        if (in)
+          for (int p = 0; p < 3; ++p) bi[p * count + o - 1] = bf[p * count + o];
+      }
+    }
+  hipError_t e;
+  if (form.f32) return (e = mem.upload(&s.f32_full, ff)) != hipSuccess ? e : mem.upload(&s.f32_int, fi);
+  return (e = mem.upload(&s.b_full, bf)) != hipSuccess ? e : mem.upload(&s.b_int, bi);
 }
 
 // Folded operators of an even-length axis (S[N-1-n][a] = (-1)^a S[n][a]).
-static hipError_t build_fold(DeviceBlock& mem, SineSet& s) {
+static hipError_t build_fold(DeviceBlock& mem, SineSet& s, SineForm form, const SineSet* same) {
   const int N = s.N, h = N / 2;
   s.h = h;
   s.fld = round_up(h, 32);
   s.frows = round_up(h, 128);
   const size_t var = (size_t)s.frows * s.fld;
-  std::vector<float> ff(4 * var, 0.0f), lf(2 * (size_t)h);
-  std::vector<uint16_t> bf(4 * 3 * var, 0);
+  std::vector<float> lf(2 * (size_t)h);
+  for (int p = 0; p < 2; ++p)
+    for (int i = 0; i < h; ++i) lf[(size_t)p * h + i] = s.lam_host[2 * i + p];
+  const hipError_t up = mem.upload(&s.lam_fold, lf);
+  if (up != hipSuccess) return up;
+  if (same) {
+    s.f32_fold = same->f32_fold;
+    s.b_fold = same->b_fold;
+    return hipSuccess;
+  }
+  std::vector<float> ff;
+  std::vector<uint16_t> bf;
+  if (form.f32) ff.assign(4 * var, 0.0f);
+  else bf.assign(4 * 3 * var, 0);
   const double c = std::sqrt(2.0 / (N + 1));
   auto S = [&](int a, int n) { return c * std::sin(M_PI * (double)(a + 1) * (double)(n + 1) / (double)(N + 1)); };
   for (int p = 0; p < 2; ++p)
     for (int i = 0; i < h; ++i)
       for (int k = 0; k < h; ++k) {
         const double v = S(2 * i + p, fold_phys(k, h));
-        const size_t fwd = (size_t)p * var + (size_t)i * s.fld + k;       // rows = outputs i
-        const size_t inv = (size_t)(2 + p) * var + (size_t)k * s.fld + i;  // rows = outputs k'
-        ff[fwd] = (float)v;
-        ff[inv] = (float)v;
-        split3(v, &bf[(size_t)p * 3 * var + (size_t)i * s.fld + k], (long)var);
-        split3(v, &bf[(size_t)(2 + p) * 3 * var + (size_t)k * s.fld + i], (long)var);
+        const size_t fwd = (size_t)i * s.fld + k;  // rows = outputs i
+        const size_t inv = (size_t)k * s.fld + i;  // rows = outputs k'
+        if (form.f32) {
+          ff[p * var + fwd] = (float)v;
+          ff[(2 + p) * var + inv] = (float)v;
+        } else {
+          uint16_t* f = &bf[(size_t)p * 3 * var + fwd];
+          split3(v, f, (long)var);
+          for (int q = 0; q < 3; ++q) bf[((size_t)(2 + p) * 3 + q) * var + inv] = f[q * var];
+        }
       }
-  for (int p = 0; p < 2; ++p)
-    for (int i = 0; i < h; ++i) lf[(size_t)p * h + i] = s.lam_host[2 * i + p];
-  hipError_t e;
-  if ((e = mem.upload(&s.f32_fold, ff)) != hipSuccess) return e;
-  if ((e = mem.upload(&s.b_fold, bf)) != hipSuccess) return e;
-  return mem.upload(&s.lam_fold, lf);
+  return form.f32 ? mem.upload(&s.f32_fold, ff) : mem.upload(&s.b_fold, bf);
 }
 
 // Fragment-order copies of the bf16 operators (folded or plain).
@@ -300,12 +336,14 @@ static hipError_t batch_build(Batch& b, const std::vector<const somaxhip_qg_desc
   b.precision = d0->precision;
   b.M = (int)ds.size();
   hipError_t e;
-  if ((e = build_sines(b.mem, b.sx, b.Nx, b.dx)) != hipSuccess) return e;
-  if ((e = build_sines(b.mem, b.sy, b.Ny, b.dy)) != hipSuccess) return e;
   b.fold = use_fold(b.Nx, b.Ny) ? 1 : 0;
+  const SineForm form{b.precision == SOMAXHIP_PREC_FP32, b.fold != 0};
+  const SineSet* same = b.Nx == b.Ny ? &b.sx : nullptr;
+  if ((e = build_sines(b.mem, b.sx, b.Nx, b.dx, form, nullptr)) != hipSuccess) return e;
+  if ((e = build_sines(b.mem, b.sy, b.Ny, b.dy, form, same)) != hipSuccess) return e;
   if (b.fold) {
-    if ((e = build_fold(b.mem, b.sx)) != hipSuccess) return e;
-    if ((e = build_fold(b.mem, b.sy)) != hipSuccess) return e;
+    if ((e = build_fold(b.mem, b.sx, form, nullptr)) != hipSuccess) return e;
+    if ((e = build_fold(b.mem, b.sy, form, same)) != hipSuccess) return e;
     b.fplane = (long)b.sx.h * b.sy.h;
   }
   if ((b.precision == SOMAXHIP_PREC_MIXED || b.precision == SOMAXHIP_PREC_BF16X6) &&
