@@ -12,10 +12,10 @@
 // each, not the matrix rate.  FP64 needs no split operands, no refinement
 // solve and no flushes, and three launches replace 6 (FP32, six-product) or
 // 12 (mixed).  Measured (us, one inversion; FP32 split -> direct): 64^2 x 1
-// 64 -> 16, 128^2 x 3 95 -> 23, 256^2 x 3 100 -> 34, 512^2 x 3 144 -> 86.  Per
+// 64 -> 16, 128^2 x 3 95 -> 22, 256^2 x 3 100 -> 34, 512^2 x 3 144 -> 75.  Per
 // launch at 64^2: 5 us, of which 1.5 are a launch's own and each dependent trip
 // to the Infinity Cache is 1 (the L2s start a kernel empty); at 512^2 x 3:
-// forward 23, spectral 31, inverse 30, against 5.6, 11.2 and 5.6 at the FP64
+// forward 21, spectral 30, inverse 23, against 5.6, 11.2 and 5.6 at the FP64
 // matrix rate (the 257th row of every folded extent costs a tile of 16, and 204
 // spectral workgroups leave a fifth of the chip idle).
 //
