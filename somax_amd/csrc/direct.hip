@@ -6,13 +6,14 @@
 //   forward   layer -> mode projection, both mirror folds and the x transform
 //   spectral  y transform, division by the Helmholtz symbol, y transform back
 //   inverse   x transform back, unfolding, mass correction, mode -> layer mix
+// (the first two in one launch on the smallest planes, direct_front)
 //
 // Why: below about 600 points a side the transforms are a few MFLOP to a
 // GFLOP, and what costs time is the number of launches and the chain inside
 // each, not the matrix rate.  FP64 needs no split operands, no refinement
 // solve and no flushes, and three launches replace 6 (FP32, six-product) or
 // 12 (mixed).  Measured (us, one inversion; FP32 split -> direct): 64^2 x 1
-// 64 -> 16, 128^2 x 3 95 -> 22, 256^2 x 3 100 -> 34, 512^2 x 3 144 -> 75.  Per
+// 64 -> 15, 128^2 x 3 95 -> 22, 256^2 x 3 100 -> 34, 512^2 x 3 144 -> 75.  Per
 // launch at 64^2: 5 us, of which 1.5 are a launch's own and each dependent trip
 // to the Infinity Cache is 1 (the L2s start a kernel empty); at 512^2 x 3:
 // forward 21, spectral 30, inverse 23, against 5.6, 11.2 and 5.6 at the FP64
@@ -294,6 +295,81 @@ __global__ __launch_bounds__(512) void direct_forward_kernel(DirectTable<G> g) {
   }
 }
 
+// The y products and the division of 16 x-modes of one parity block.
+struct Spectral {
+  Ring v;                     // the start of this wave's first y tile, O
+  const double *F, *Gy, *ly;  // this lane's y operators and eigenvalues
+  const double* O;
+  long zb;
+  int ns, t0;
+  bool sums;
+  double lx, cxv;
+};
+__device__ __forceinline__ void spectral_start(Spectral& s, const DirectArgs& a, int z, int py, int px, int xt) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  s.zb = (long)(z * 4 + py * 2 + px) * (256L * a.ntx * a.nty);
+  s.ns = (a.hy + 3) / 4;
+  const long ypar = py * 256L * a.nty * a.nty;
+  s.F = a.fy + ypar + lane;
+  s.Gy = a.gy + ypar + lane;
+  s.t0 = wave < a.nty ? wave : a.nty - 1;  // (waves without a tile stream the last one)
+  s.O = s.F + (long)s.t0 * 256 * a.nty;
+  ring_start(s.v, s.O, (s.ns + 3) >> 2);
+  s.lx = a.lamx[px * 16 * a.ntx + xt * 16 + (lane & 15)] - a.lam[z];
+  s.ly = a.lamy + py * 16 * a.nty + (lane >> 4);
+  s.sums = a.homsol && px == 0 && py == 0;
+  s.cxv = s.sums ? a.cx[xt * 16 + (lane & 15)] : 0.0;
+}
+// From the modes' data Ts (fragment order) to V; W: the same space for the quotient.
+template <int NW>
+__device__ __forceinline__ void spectral_run(Spectral& s, const DirectArgs& a, int z, int xt, const double* Ts,
+                                             double* W, double* red) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  double total = 0.0;
+  for (int t = wave; t < a.nty; t += NW) {
+    double4m acc = {0.0, 0.0, 0.0, 0.0};
+    double lyv[4], cyv[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      lyv[r] = s.ly[t * 16 + 4 * r];
+      cyv[r] = s.sums ? a.cy[t * 16 + (lane >> 4) + 4 * r] : 0.0;
+    }
+    product<false, 64>(s.v, s.O, Ts + lane, s.ns, acc);
+    // next: this wave's next tile, else its first tile of the way back
+    s.O = t + NW < a.nty ? s.F + (long)(t + NW) * 256 * a.nty : s.Gy + (long)s.t0 * 256 * a.nty;
+    ring_start(s.v, s.O, (s.ns + 3) >> 2);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const double w = acc[r] / (s.lx + lyv[r]);
+      W[(t * 4 + r) * 64 + lane] = w;
+      total += w * s.cxv * cyv[r];
+    }
+  }
+  if (s.sums) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o);
+    if (lane == 0) red[wave] = total;
+  }
+  __syncthreads();
+  if (s.sums && tid == 0) {
+    double w = 0.0;
+    for (int i = 0; i < NW; ++i) w += red[i];
+    a.partial[(long)z * a.ntx + xt] = w;
+  }
+  double* V = a.V + s.zb + xt * 256 + lane;
+  for (int t = wave; t < a.nty; t += NW) {
+    double4m acc = {0.0, 0.0, 0.0, 0.0};
+    product<true, 64>(s.v, s.O, W + lane, s.ns, acc);
+    if (t + NW < a.nty) {
+      s.O = s.Gy + (long)(t + NW) * 256 * a.nty;
+      ring_start(s.v, s.O, (s.ns + 3) >> 2);
+    }
+    double* o = V + (long)t * (256L * a.ntx);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r * 64] = acc[r];
+  }
+}
+
 // Spectral: workgroup = 16 x-modes of one parity block of one plane.  The y
 // transform's result stays in LDS (fragment order) between the two products.
 template <int NW, int G>
@@ -311,70 +387,120 @@ __global__ __launch_bounds__(64 * NW) void direct_spectral_kernel(DirectTable<G>
   rest >>= 1;
   const int z = rest % a.P, py = rest / a.P;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const long blk = 256L * a.ntx * a.nty;
-  const long zb = (long)(z * 4 + py * 2 + px) * blk;
-  const double* T = a.T + zb + (long)xt * (256L * a.nty);
+  const double* T = a.T + ((long)(z * 4 + py * 2 + px) * a.ntx + xt) * (256L * a.nty);
   double* W = sd;                 // [4 nty k-steps of iy][64]
   double* Ts = sd + 256 * a.nty;  // the x-modes' data, staged once for all waves
-  const int ns = (a.hy + 3) / 4;
-  const long ypar = py * 256L * a.nty * a.nty;
-  const double* F = a.fy + ypar + lane;
-  const double* Gy = a.gy + ypar + lane;
-  const int t0 = wave < a.nty ? wave : a.nty - 1;  // (waves without a tile stream the last one)
-  const double* O = F + (long)t0 * 256 * a.nty;
-  Ring v;
-  ring_start(v, O, (ns + 3) >> 2);
-  const double lx = a.lamx[px * 16 * a.ntx + xt * 16 + (lane & 15)] - a.lam[z];
-  const double* ly = a.lamy + py * 16 * a.nty + (lane >> 4);
-  const bool sums = a.homsol && px == 0 && py == 0;
-  const double cxv = sums ? a.cx[xt * 16 + (lane & 15)] : 0.0;
+  Spectral s;
+  spectral_start(s, a, z, py, px, xt);
   // straight into LDS, 1 KiB a wave and instruction
   for (int e = wave; e < 2 * a.nty; e += NW)
     __builtin_amdgcn_global_load_lds(T + e * 128 + lane * 2, Ts + e * 128, 16, 0, 0);
-  double total = 0.0;
+  __syncthreads();
+  spectral_run<NW>(s, a, z, xt, Ts, W, red);
+}
+
+// Forward and spectral in one, for planes of a few tiles: workgroup = 16 x-modes of
+// one parity block of one plane.  It projects and folds the whole plane to its
+// parity (every workgroup of a plane again: a few loads a thread), takes its 16
+// modes of the x product from LDS to LDS, and goes on as the spectral kernel.  The
+// same sums in the same order.  Bound by the chain of loads and short products, of
+// which it saves one launch and one trip through memory: at 64^2 x 1 an inversion
+// in a replayed graph 12.3 -> 11.2 us, an FP64 step of three 60.6 -> 55.9.
+template <class R, int NL>
+__global__ __launch_bounds__(512) void direct_front_kernel(DirectTable<1> g) {
+  constexpr int NW = 8;
+  extern __shared__ __attribute__((aligned(16))) double sd[];
+  __shared__ double red[NW];
+  const DirectArgs& a = g.a[0];
+  const int l = xcd_order(blockIdx.x, gridDim.x);
+  const int xt = l % a.ntx;
+  int rest = l / a.ntx;
+  const int px = rest & 1;
+  rest >>= 1;
+  const int z = rest % a.P, py = rest / a.P;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int K = direct_k(a.hx, a.apply_bc), rows = direct_k(a.hy, a.apply_bc);
+  const int pitch = direct_pitch(K), kpad = pitch - 2, nsx = (K + 3) / 4;
+  double* X = sd;  // [16 nty][pitch]
+  double* Ts = sd + 16 * a.nty * pitch;
+  double* W = Ts + 256 * a.nty;
+  const double* B = a.fx + px * 256L * a.ntx * a.ntx + (long)xt * 256 * a.ntx + lane;
+  Ring vx;
+  ring_start(vx, B, (nsx + 3) >> 2);
+  Spectral sp;
+  spectral_start(sp, a, z, py, px, xt);
+
+  int m = 0, first = 0, nl = a.P, mode = z;
+  if (a.mfirst) {
+    m = a.member[z];
+    first = a.mfirst[m];
+    nl = a.mnl[m];
+    mode = a.layer[z];
+  }
+  const double* cl = a.cl2m + m * 64 + mode * MAX_LAYERS;
+  const R* q = static_cast<const R*>(a.q) + (long)first * a.plane;
+  const int Nx = a.Nx, Ny = a.Ny;
+  // EB points of a thread at a time, all their loads before the first sum
+  constexpr int EB = NL <= 3 ? 4 : 2;
+  for (int e0 = tid; e0 < rows * kpad; e0 += 512 * EB) {
+    int x[EB], y[EB], at[EB];
+    bool live[EB];
+    double u[EB][4];
+#pragma unroll
+    for (int b = 0; b < EB; ++b) {
+      const int e = min(e0 + 512 * b, rows * kpad - 1);  // (past the end: the last point again)
+      const int jy = e / kpad, jj = e - jy * kpad;
+      live[b] = jj < K;
+      x[b] = fold_phys(live[b] ? jj : 0, a.hx);
+      y[b] = fold_phys(jy, a.hy);
+      at[b] = jy * pitch + jj;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) u[b][i] = 0.0;
+    }
+    for (int k0 = 0; k0 < nl; k0 += NL) {
+      // (layers past the last read it again and are left out of the sum)
+      R r[EB][NL][4];
+#pragma unroll
+      for (int b = 0; b < EB; ++b)
+#pragma unroll
+        for (int k = 0; k < NL; ++k) {
+          const R* p = q + (k0 + k < nl ? k0 + k : nl - 1) * a.plane;
+          const int r0 = y[b] * Nx, r1 = (Ny - 1 - y[b]) * Nx, xm = Nx - 1 - x[b];
+          r[b][k][0] = p[r0 + x[b]];
+          r[b][k][1] = p[r0 + xm];
+          r[b][k][2] = p[r1 + x[b]];
+          r[b][k][3] = p[r1 + xm];
+        }
+#pragma unroll
+      for (int k = 0; k < NL; ++k)
+        if (k0 + k < nl) {
+          const double w = cl[k0 + k];
+#pragma unroll
+          for (int b = 0; b < EB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) u[b][i] += w * (double)r[b][k][i];
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < EB; ++b) {
+      double* s = u[b];
+      if (2 * x[b] == Nx - 1) s[1] = s[3] = 0.0;  // the middle of an odd line counts once
+      if (2 * y[b] == Ny - 1) s[2] = s[3] = 0.0;
+      const double c0 = px ? s[0] - s[1] : s[0] + s[1], c1 = px ? s[2] - s[3] : s[2] + s[3];
+      X[at[b]] = live[b] ? (py ? c0 - c1 : c0 + c1) : 0.0;
+    }
+  }
+  for (int e = rows * pitch + tid; e < 16 * a.nty * pitch; e += 512) X[e] = 0.0;
   __syncthreads();
   for (int t = wave; t < a.nty; t += NW) {
     double4m acc = {0.0, 0.0, 0.0, 0.0};
-    double lyv[4], cyv[4];
+    product<true, 4>(vx, B, X + (t * 16 + (lane & 15)) * pitch + (lane >> 4), nsx, acc);
+    if (t + NW < a.nty) ring_start(vx, B, (nsx + 3) >> 2);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      lyv[r] = ly[t * 16 + 4 * r];
-      cyv[r] = sums ? a.cy[t * 16 + (lane >> 4) + 4 * r] : 0.0;
-    }
-    product<false, 64>(v, O, Ts + lane, ns, acc);
-    // next: this wave's next tile, else its first tile of the way back
-    O = t + NW < a.nty ? F + (long)(t + NW) * 256 * a.nty : Gy + (long)t0 * 256 * a.nty;
-    ring_start(v, O, (ns + 3) >> 2);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const double w = acc[r] / (lx + lyv[r]);
-      W[(t * 4 + r) * 64 + lane] = w;
-      total += w * cxv * cyv[r];
-    }
-  }
-  if (sums) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o);
-    if (lane == 0) red[wave] = total;
+    for (int r = 0; r < 4; ++r) Ts[t * 256 + r * 64 + lane] = acc[r];
   }
   __syncthreads();
-  if (sums && tid == 0) {
-    double w = 0.0;
-    for (int i = 0; i < NW; ++i) w += red[i];
-    a.partial[(long)z * a.ntx + xt] = w;
-  }
-  double* V = a.V + zb + xt * 256 + lane;
-  for (int t = wave; t < a.nty; t += NW) {
-    double4m acc = {0.0, 0.0, 0.0, 0.0};
-    product<true, 64>(v, O, W + lane, ns, acc);
-    if (t + NW < a.nty) {
-      O = Gy + (long)(t + NW) * 256 * a.nty;
-      ring_start(v, O, (ns + 3) >> 2);
-    }
-    double* o = V + (long)t * (256L * a.ntx);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[r * 64] = acc[r];
-  }
+  spectral_run<NW>(sp, a, z, xt, Ts, W, red);
 }
 
 // Inverse: workgroup = 16 x 16 XT folded points (four mirror images of each) of
@@ -533,8 +659,27 @@ __global__ __launch_bounds__(256 * NMODE) void direct_inverse_kernel(DirectTable
     }
 }
 
+constexpr int DIRECT_LDS = 157 * 1024;
 size_t forward_lds(const DirectArgs& a) {
   return (size_t)64 * direct_pitch(direct_k(a.hx, a.apply_bc)) * sizeof(double);
+}
+size_t front_lds(const DirectArgs& a) {
+  return (size_t)a.nty * (16 * direct_pitch(direct_k(a.hx, a.apply_bc)) + 512) * sizeof(double);
+}
+// The forward and spectral kernels in one launch (direct_front_kernel) while that
+// saves more than its repeated folds cost.  A workgroup loads rows x row x layers
+// points four times (lines of at least 32 points: shorter rows cost as much):
+// us of an inversion in a replayed graph, two launches -> one: 16^2 x 1 10.5 -> 9.2,
+// 64^2 x 1 12.3 -> 11.2, 64^2 x 5 18.4 -> 17.2, 128^2 x 1 15.5 -> 15.1, but 110^2 x 2
+// (7040) 15.3 -> 15.35, 20 x 120 x 3 (5760) 14.9 -> 15.0, 128^2 x 3 (12288) 18.7 -> 19.7;
+// 160^2 x 1 (five tiles of rows on eight waves, two rings of the x product) 16.8
+// -> 18.2.  And one workgroup per CU, as a full chip pays for every repeat (steps
+// of ensembles: 64^2, 240 workgroups 98 -> 93, 288 108 -> 120; 32^2, 192 103 -> 95,
+// 384 104 -> 112).
+bool direct_front(const DirectArgs& a) {
+  const int K = direct_k(a.hx, a.apply_bc), rows = direct_k(a.hy, a.apply_bc);
+  return K <= 64 && rows <= 64 && rows * std::max(direct_pitch(K) - 2, 32) * a.nlmax <= 5120 &&
+         a.P * 4 * a.ntx <= 256;
 }
 size_t spectral_lds(const DirectArgs& a) { return (size_t)512 * a.nty * sizeof(double); }
 // Column tiles per workgroup of the inverse kernel: two where a fold has more
@@ -547,10 +692,15 @@ template <class K>
 hipError_t raise_lds(K kernel, int bytes) {
   return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
-constexpr int DIRECT_LDS = 157 * 1024;
 template <class R, int G>
 hipError_t prepare_kernels() {
   hipError_t e = raise_lds(direct_forward_kernel<R, 1, G>, DIRECT_LDS);
+  if (G == 1) {
+    if (e == hipSuccess) e = raise_lds(direct_front_kernel<R, 1>, DIRECT_LDS);
+    if (e == hipSuccess) e = raise_lds(direct_front_kernel<R, 2>, DIRECT_LDS);
+    if (e == hipSuccess) e = raise_lds(direct_front_kernel<R, 3>, DIRECT_LDS);
+    if (e == hipSuccess) e = raise_lds(direct_front_kernel<R, 4>, DIRECT_LDS);
+  }
   if (e == hipSuccess) e = raise_lds(direct_forward_kernel<R, 2, G>, DIRECT_LDS);
   if (e == hipSuccess) e = raise_lds(direct_forward_kernel<R, 3, G>, DIRECT_LDS);
   if (e == hipSuccess) e = raise_lds(direct_forward_kernel<R, 4, G>, DIRECT_LDS);
@@ -581,6 +731,16 @@ void launch_forward(DirectTable<G>& g, int blocks, size_t lds, int nlmax, hipStr
   else if (nlmax == 2) hipLaunchKernelGGL((direct_forward_kernel<R, 2, G>), dim3(blocks), dim3(512), lds, st, g);
   else if (nlmax == 3) hipLaunchKernelGGL((direct_forward_kernel<R, 3, G>), dim3(blocks), dim3(512), lds, st, g);
   else hipLaunchKernelGGL((direct_forward_kernel<R, 4, G>), dim3(blocks), dim3(512), lds, st, g);
+}
+template <class R>
+void launch_front(DirectTable<1>& g, hipStream_t st) {
+  const DirectArgs& a = g.a[0];
+  const dim3 blocks(a.P * 4 * a.ntx), threads(512);
+  const size_t lds = front_lds(a);
+  if (a.nlmax == 1) hipLaunchKernelGGL((direct_front_kernel<R, 1>), blocks, threads, lds, st, g);
+  else if (a.nlmax == 2) hipLaunchKernelGGL((direct_front_kernel<R, 2>), blocks, threads, lds, st, g);
+  else if (a.nlmax == 3) hipLaunchKernelGGL((direct_front_kernel<R, 3>), blocks, threads, lds, st, g);
+  else hipLaunchKernelGGL((direct_front_kernel<R, 4>), blocks, threads, lds, st, g);
 }
 template <int G>
 void launch_spectral(DirectTable<G>& g, int blocks, size_t lds, int nty, hipStream_t st) {
@@ -775,14 +935,21 @@ void run(const DirectCall* c, int n, hipStream_t st, const DirectPhase& phase) {
       lds[k] = std::max(lds[k], need[k]);
     }
   }
-  phase(0, [&] {
-    g.t = t[0];
-    launch_forward<R, G>(g, blocks[0], lds[0], nlmax, st);
-  });
-  phase(1, [&] {
-    g.t = t[1];
-    launch_spectral<G>(g, blocks[1], lds[1], nty, st);
-  });
+  bool front = false;
+  if constexpr (G == 1) {
+    front = direct_front(g.a[0]);
+    if (front) phase(3, [&] { launch_front<R>(g, st); });
+  }
+  if (!front) {
+    phase(0, [&] {
+      g.t = t[0];
+      launch_forward<R, G>(g, blocks[0], lds[0], nlmax, st);
+    });
+    phase(1, [&] {
+      g.t = t[1];
+      launch_spectral<G>(g, blocks[1], lds[1], nty, st);
+    });
+  }
   phase(2, [&] {
     g.t = t[2];
     if (xt == 2) launch_inverse<R, 2, G>(g, blocks[2], lds[2], nlmax, st);

@@ -499,7 +499,8 @@ struct DirectCall {
   float* psi_wall;     // nullable: wall psi per plane
   double* alpha;       // nullable: multiplier per plane
 };
-// phase(k, launch) calls launch() for kernel k of the three (timing hooks).
+// phase(k, launch) calls launch() for kernel k of the three, 3 for the first two
+// in one (timing hooks).
 using DirectPhase = std::function<void(int, const std::function<void()>&)>;
 void launch_direct(const DirectCall& c, hipStream_t st, const DirectPhase& phase);
 void launch_direct_group(const DirectCall* c, int n, hipStream_t st, const DirectPhase& phase);  // n <= MAX_GROUP

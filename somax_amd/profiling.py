@@ -63,7 +63,7 @@ _BENCH_NAMES = (("dst_gemm_bf16_kernel<1", "dst_gemm_bf16x1"), ("dst_gemm_bf16_k
                 ("dst_gemm_bf16_kernel<6", "dst_gemm_bf16x6"), ("dst_gemm_f32_kernel", "dst_gemm_fp32"),
                 ("dst_gemm_f32_small_kernel", "dst_gemm_fp32"), ("dst_stripe_kernel", "dst_stripe"),
                 ("direct_forward_kernel", "direct_forward"), ("direct_spectral_kernel", "direct_spectral"),
-                ("direct_inverse_kernel", "direct_inverse"),
+                ("direct_inverse_kernel", "direct_inverse"), ("direct_front_kernel", "direct_front"),
                 ("qg_stage_", "qg_stage"), ("residual", "residual"), ("to_modal", "to_modal"),
                 ("to_layer", "to_layer"), ("swm_stage_kernel", "swm_stage"))
 
