@@ -13,8 +13,8 @@
 // each, not the matrix rate.  FP64 needs no split operands, no refinement
 // solve and no flushes, and three launches replace 6 (FP32, six-product) or
 // 12 (mixed).  Measured (us, one inversion; FP32 split -> direct): 64^2 x 1
-// 64 -> 15, 128^2 x 3 95 -> 22, 256^2 x 3 100 -> 34, 512^2 x 3 144 -> 75.  Per
-// launch at 64^2: 5 us, of which 1.5 are a launch's own and each dependent trip
+// 64 -> 12, 128^2 x 3 95 -> 19, 256^2 x 3 100 -> 34, 512^2 x 3 144 -> 72.  Per
+// launch at 64^2: 5 to 7 us, of which 1.5 are a launch's own and each dependent trip
 // to the Infinity Cache is 1 (the L2s start a kernel empty); at 512^2 x 3:
 // forward 21, spectral 30, inverse 23, against 5.6, 11.2 and 5.6 at the FP64
 // matrix rate (the 257th row of every folded extent costs a tile of 16, and 204
@@ -202,10 +202,9 @@ __global__ __launch_bounds__(512) void direct_forward_kernel(DirectTable<G> g) {
   const double* Bx = a.fx + px * 256L * a.ntx * a.ntx + lane;
   const int ns = (K + 3) / 4;
   int t = part + a.split * (wave >> 2);
-  // (waves without a tile stream the last one, so the loads are unconditional)
-  const double* B = Bx + (long)(t < a.ntx ? t : a.ntx - 1) * 256 * a.ntx;
+  const double* B = Bx + (long)t * 256 * a.ntx;
   Ring v;
-  ring_start(v, B, (ns + 3) >> 2);
+  if (t < a.ntx) ring_start(v, B, (ns + 3) >> 2);
 
   int m = 0, first = 0, nl = a.P, mode = z;
   if (a.mfirst) {
@@ -298,13 +297,22 @@ __global__ __launch_bounds__(512) void direct_forward_kernel(DirectTable<G> g) {
 // The y products and the division of 16 x-modes of one parity block.
 struct Spectral {
   Ring v;                     // the start of this wave's first y tile, O
-  const double *F, *Gy, *ly;  // this lane's y operators and eigenvalues
+  Ring g;                     // and of its first tile of the way back
+  const double *F, *Gy, *ly, *cy;  // this lane's y operators, eigenvalues and column sums
+  double lyv[4], cyv[4];           // the latter two of the next tile
   const double* O;
   long zb;
   int ns, t0;
   bool sums;
   double lx, cxv;
 };
+__device__ __forceinline__ void spectral_tile(Spectral& s, int t) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    s.lyv[r] = s.ly[t * 16 + 4 * r];
+    s.cyv[r] = s.sums ? s.cy[t * 16 + 4 * r] : 0.0;
+  }
+}
 __device__ __forceinline__ void spectral_start(Spectral& s, const DirectArgs& a, int z, int py, int px, int xt) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   s.zb = (long)(z * 4 + py * 2 + px) * (256L * a.ntx * a.nty);
@@ -312,37 +320,41 @@ __device__ __forceinline__ void spectral_start(Spectral& s, const DirectArgs& a,
   const long ypar = py * 256L * a.nty * a.nty;
   s.F = a.fy + ypar + lane;
   s.Gy = a.gy + ypar + lane;
-  s.t0 = wave < a.nty ? wave : a.nty - 1;  // (waves without a tile stream the last one)
+  s.t0 = wave < a.nty ? wave : a.nty - 1;
   s.O = s.F + (long)s.t0 * 256 * a.nty;
-  ring_start(s.v, s.O, (s.ns + 3) >> 2);
+  // (waves without a tile load nothing: their streams would cost L1 time, 64 KB a
+  // ring and workgroup; measured 128^2 x 3 two Tsit5 steps 308 -> 301 us)
+  if (wave < a.nty) ring_start(s.v, s.O, (s.ns + 3) >> 2);
   s.lx = a.lamx[px * 16 * a.ntx + xt * 16 + (lane & 15)] - a.lam[z];
   s.ly = a.lamy + py * 16 * a.nty + (lane >> 4);
   s.sums = a.homsol && px == 0 && py == 0;
   s.cxv = s.sums ? a.cx[xt * 16 + (lane & 15)] : 0.0;
+  s.cy = a.cy + (lane >> 4);
 }
 // From the modes' data Ts (fragment order) to V; W: the same space for the quotient.
-template <int NW>
+// EARLY: at most one tile a wave, its eigenvalues read before (spectral_tile) and
+// the ring of its way back started before the first product.
+template <int NW, bool EARLY>
 __device__ __forceinline__ void spectral_run(Spectral& s, const DirectArgs& a, int z, int xt, const double* Ts,
                                              double* W, double* red) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   double total = 0.0;
+  Ring& g = EARLY ? s.g : s.v;
+  if (EARLY && wave < a.nty) ring_start(s.g, s.Gy + (long)s.t0 * 256 * a.nty, (s.ns + 3) >> 2);
   for (int t = wave; t < a.nty; t += NW) {
     double4m acc = {0.0, 0.0, 0.0, 0.0};
-    double lyv[4], cyv[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      lyv[r] = s.ly[t * 16 + 4 * r];
-      cyv[r] = s.sums ? a.cy[t * 16 + (lane >> 4) + 4 * r] : 0.0;
-    }
+    if (!EARLY) spectral_tile(s, t);
     product<false, 64>(s.v, s.O, Ts + lane, s.ns, acc);
     // next: this wave's next tile, else its first tile of the way back
-    s.O = t + NW < a.nty ? s.F + (long)(t + NW) * 256 * a.nty : s.Gy + (long)s.t0 * 256 * a.nty;
-    ring_start(s.v, s.O, (s.ns + 3) >> 2);
+    if (!EARLY) {
+      s.O = t + NW < a.nty ? s.F + (long)(t + NW) * 256 * a.nty : s.Gy + (long)s.t0 * 256 * a.nty;
+      ring_start(s.v, s.O, (s.ns + 3) >> 2);
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const double w = acc[r] / (s.lx + lyv[r]);
+      const double w = acc[r] / (s.lx + s.lyv[r]);
       W[(t * 4 + r) * 64 + lane] = w;
-      total += w * s.cxv * cyv[r];
+      total += w * s.cxv * s.cyv[r];
     }
   }
   if (s.sums) {
@@ -357,12 +369,13 @@ __device__ __forceinline__ void spectral_run(Spectral& s, const DirectArgs& a, i
     a.partial[(long)z * a.ntx + xt] = w;
   }
   double* V = a.V + s.zb + xt * 256 + lane;
+  if (EARLY) s.O = s.Gy + (long)s.t0 * 256 * a.nty;
   for (int t = wave; t < a.nty; t += NW) {
     double4m acc = {0.0, 0.0, 0.0, 0.0};
-    product<true, 64>(s.v, s.O, W + lane, s.ns, acc);
+    product<true, 64>(g, s.O, W + lane, s.ns, acc);
     if (t + NW < a.nty) {
       s.O = s.Gy + (long)(t + NW) * 256 * a.nty;
-      ring_start(s.v, s.O, (s.ns + 3) >> 2);
+      ring_start(g, s.O, (s.ns + 3) >> 2);
     }
     double* o = V + (long)t * (256L * a.ntx);
 #pragma unroll
@@ -396,7 +409,7 @@ __global__ __launch_bounds__(64 * NW) void direct_spectral_kernel(DirectTable<G>
   for (int e = wave; e < 2 * a.nty; e += NW)
     __builtin_amdgcn_global_load_lds(T + e * 128 + lane * 2, Ts + e * 128, 16, 0, 0);
   __syncthreads();
-  spectral_run<NW>(s, a, z, xt, Ts, W, red);
+  spectral_run<NW, false>(s, a, z, xt, Ts, W, red);
 }
 
 // Forward and spectral in one, for planes of a few tiles: workgroup = 16 x-modes of
@@ -405,7 +418,8 @@ __global__ __launch_bounds__(64 * NW) void direct_spectral_kernel(DirectTable<G>
 // modes of the x product from LDS to LDS, and goes on as the spectral kernel.  The
 // same sums in the same order.  Bound by the chain of loads and short products, of
 // which it saves one launch and one trip through memory: at 64^2 x 1 an inversion
-// in a replayed graph 12.3 -> 11.2 us, an FP64 step of three 60.6 -> 55.9.
+// in a replayed graph 12.3 -> 10.5 us, an FP64 step of three 60.6 -> 52.5 (with the
+// ring of the way back started late, by waves without a tile too: 11.3, 55.9).
 template <class R, int NL>
 __global__ __launch_bounds__(512) void direct_front_kernel(DirectTable<1> g) {
   constexpr int NW = 8;
@@ -426,9 +440,10 @@ __global__ __launch_bounds__(512) void direct_front_kernel(DirectTable<1> g) {
   double* W = Ts + 256 * a.nty;
   const double* B = a.fx + px * 256L * a.ntx * a.ntx + (long)xt * 256 * a.ntx + lane;
   Ring vx;
-  ring_start(vx, B, (nsx + 3) >> 2);
+  if (wave < a.nty) ring_start(vx, B, (nsx + 3) >> 2);
   Spectral sp;
   spectral_start(sp, a, z, py, px, xt);
+  spectral_tile(sp, sp.t0);
 
   int m = 0, first = 0, nl = a.P, mode = z;
   if (a.mfirst) {
@@ -441,7 +456,7 @@ __global__ __launch_bounds__(512) void direct_front_kernel(DirectTable<1> g) {
   const R* q = static_cast<const R*>(a.q) + (long)first * a.plane;
   const int Nx = a.Nx, Ny = a.Ny;
   // EB points of a thread at a time, all their loads before the first sum
-  constexpr int EB = NL <= 3 ? 4 : 2;
+  constexpr int EB = NL <= 2 ? 4 : 2;
   for (int e0 = tid; e0 < rows * kpad; e0 += 512 * EB) {
     int x[EB], y[EB], at[EB];
     bool live[EB];
@@ -492,15 +507,14 @@ __global__ __launch_bounds__(512) void direct_front_kernel(DirectTable<1> g) {
   }
   for (int e = rows * pitch + tid; e < 16 * a.nty * pitch; e += 512) X[e] = 0.0;
   __syncthreads();
-  for (int t = wave; t < a.nty; t += NW) {
+  if (wave < a.nty) {  // one tile a wave: at most 65 folded points (direct_front)
     double4m acc = {0.0, 0.0, 0.0, 0.0};
-    product<true, 4>(vx, B, X + (t * 16 + (lane & 15)) * pitch + (lane >> 4), nsx, acc);
-    if (t + NW < a.nty) ring_start(vx, B, (nsx + 3) >> 2);
+    product<true, 4>(vx, B, X + (wave * 16 + (lane & 15)) * pitch + (lane >> 4), nsx, acc);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) Ts[t * 256 + r * 64 + lane] = acc[r];
+    for (int r = 0; r < 4; ++r) Ts[wave * 256 + r * 64 + lane] = acc[r];
   }
   __syncthreads();
-  spectral_run<NW>(sp, a, z, xt, Ts, W, red);
+  spectral_run<NW, true>(sp, a, z, xt, Ts, W, red);
 }
 
 // Inverse: workgroup = 16 x 16 XT folded points (four mirror images of each) of
@@ -668,17 +682,17 @@ size_t front_lds(const DirectArgs& a) {
 }
 // The forward and spectral kernels in one launch (direct_front_kernel) while that
 // saves more than its repeated folds cost.  A workgroup loads rows x row x layers
-// points four times (lines of at least 32 points: shorter rows cost as much):
-// us of an inversion in a replayed graph, two launches -> one: 16^2 x 1 10.5 -> 9.2,
-// 64^2 x 1 12.3 -> 11.2, 64^2 x 5 18.4 -> 17.2, 128^2 x 1 15.5 -> 15.1, but 110^2 x 2
-// (7040) 15.3 -> 15.35, 20 x 120 x 3 (5760) 14.9 -> 15.0, 128^2 x 3 (12288) 18.7 -> 19.7;
-// 160^2 x 1 (five tiles of rows on eight waves, two rings of the x product) 16.8
-// -> 18.2.  And one workgroup per CU, as a full chip pays for every repeat (steps
-// of ensembles: 64^2, 240 workgroups 98 -> 93, 288 108 -> 120; 32^2, 192 103 -> 95,
-// 384 104 -> 112).
+// points four times (rows of at least 32 points: shorter ones cost as much).
+// us of an inversion in a replayed graph, two launches -> one: 16^2 x 1 10.5 -> 8.3,
+// 64^2 x 1 12.3 -> 10.5, 64^2 x 7 21.4 -> 19.9, 128^2 x 2 (8064) 14.9 -> 14.3; but 128^2 x 3
+// (12096) 16.0 -> 17.3, 30 x 120 x 6 (11520) 19.2 -> 19.6.  Up to 64 points a side
+// every wave has at most one tile and its ring holds the tile's whole stream (160^2
+// x 1: 16.8 -> 18.2).  And one workgroup per CU, as a full chip pays for every
+// repeat (steps of ensembles: 64^2, 240 workgroups 98 -> 93, 288 108 -> 120; 32^2, 192
+// 103 -> 95, 384 104 -> 112).
 bool direct_front(const DirectArgs& a) {
   const int K = direct_k(a.hx, a.apply_bc), rows = direct_k(a.hy, a.apply_bc);
-  return K <= 64 && rows <= 64 && rows * std::max(direct_pitch(K) - 2, 32) * a.nlmax <= 5120 &&
+  return K <= 64 && rows <= 64 && rows * std::max(direct_pitch(K) - 2, 32) * a.nlmax <= 8192 &&
          a.P * 4 * a.ntx <= 256;
 }
 size_t spectral_lds(const DirectArgs& a) { return (size_t)512 * a.nty * sizeof(double); }

@@ -45,10 +45,11 @@ def test_direct_inversion_matches_oracle(gpu, nx, ny, nl, mass):
         assert r < BAR
 
 
-# around the limits of the one-launch front (rows and row at most 64, 5120 points
-# over the layers): on it 126 x 126, 127 x 125, 64 x 64 x 5 and 30 x 78 x 2 (one
-# tile of columns, three of rows); past it 129 x 126, 126 x 129, 64 x 64 x 6
-FRONT = [(126, 126, 1), (127, 125, 1), (129, 126, 1), (126, 129, 1), (64, 64, 5), (64, 64, 6), (30, 78, 2)]
+# around the limits of the one-launch front (rows and row at most 64, 8192 points
+# over the layers): on it 126 x 126 x 2, 127 x 125, 64 x 64 x 8 and 30 x 78 x 2 (one
+# tile of columns, three of rows); past it 129 x 126, 126 x 129, 126 x 126 x 3
+FRONT = [(126, 126, 1), (127, 125, 1), (129, 126, 1), (126, 129, 1), (64, 64, 5), (64, 64, 6), (64, 64, 8), (30, 78, 2), (126, 126, 2),
+         (126, 126, 3)]
 
 
 @pytest.mark.parametrize("nx,ny,nl", FRONT)
