@@ -292,15 +292,16 @@ __device__ inline double lap64(const Stage64& s, F f, int jj, int ii) {
 // the boundary condition (Q), of the streamfunction (P), of the total PV
 // q + beta (y - y0) (QT) and of the Laplacian of Q with a zero ghost ring
 // (L, read by the biharmonic term); pw is the layer's wall value of psi
-// (WENO-Z).
-template <class QF, class PF, class QTF, class LF>
-__device__ inline double rhs_point(const Stage64& s, QF Q, PF P, QTF QT, LF L, int l, int j, int i, double pw) {
+// (WENO-Z), wind the row's forcing.
+template <bool WENO, class QF, class PF, class QTF, class LF>
+__device__ inline double rhs_point(const Stage64& s, QF Q, PF P, QTF QT, LF L, int l, int j, int i, double pw,
+                                 double wind) {
   const int Nx = s.Nx, Ny = s.Ny;
   auto ghost = [&](int jj, int ii) { return jj == 0 || jj == Ny - 1 || ii == 0 || ii == Nx - 1; };
   auto lap = [&](auto F, int jj, int ii) { return lap64(s, F, jj, ii); };
   double r = 0.0;
   if (!ghost(j, i)) {
-    if (s.advection == SOMAXHIP_ADV_WENO) {
+    if constexpr (WENO) {
       const int n_x = Nx - 2, n_y = Ny - 2;
       // corner streamfunction: corner (b, a) at T-index (a + 1/2, b + 1/2)
       auto CS = [&](int b, int a) {
@@ -331,7 +332,7 @@ __device__ inline double rhs_point(const Stage64& s, QF Q, PF P, QTF QT, LF L, i
       r = -((jpp + jpx + jxp) / (12.0 * s.dx * s.dy));
     }
   }
-  r = r + (s.tau0 * s.wind_scale[l]) * s.wind_row[j];
+  r = r + wind;
   if (!ghost(j, i)) {
     if (s.kappa != 0.0 && l == s.nl - 1) r = r + -s.kappa * lap(P, j, i);
     if (s.nu != 0.0) r = r + s.nu * lap(Q, j, i);
@@ -347,7 +348,10 @@ __device__ inline double combine(const Stage64& s, double x, double qn, double r
   return s.qn ? s.a * qn / s.adiv + o : o;
 }
 
-__global__ __launch_bounds__(256) void stage64_kernel(Stage64 s) {
+// One Arakawa stage, a thread per cell that reads its stencil from memory (all loads
+// together): of a plane that leaves the chip idle, a tile's barrier and LDS trip
+// cost more than they save (a step of 64^2 x 1 52.3 us against 53.9).
+__global__ __launch_bounds__(256) void stage64_point_kernel(Stage64 s) {
   const long c = blockIdx.x * 256L + threadIdx.x;
   const int l = blockIdx.y;
   if (c >= s.plane) return;
@@ -362,17 +366,12 @@ __global__ __launch_bounds__(256) void stage64_kernel(Stage64 s) {
   };
   auto QT = [&](int jj, int ii) { return Q(jj, ii) + s.beta_row[jj]; };
   auto P = [&](int jj, int ii) { return psi[(long)jj * Nx + ii]; };
-  double pw = 0.0;
-  if (s.alpha && s.advection == SOMAXHIP_ADV_WENO) {
-    pw = s.cm2l[l * s.nl] * s.alpha[0];
-    for (int m = 1; m < s.nl; ++m) pw = pw + s.cm2l[l * s.nl + m] * s.alpha[m];
-  }
   // the inner Laplacian of the biharmonic term, recomputed at each neighbour
   auto L = [&](int jj, int ii) {
     const bool g = jj == 0 || jj == Ny - 1 || ii == 0 || ii == Nx - 1;
     return g ? 0.0 : lap64(s, Q, jj, ii);
   };
-  const double r = rhs_point(s, Q, P, QT, L, l, j, i, pw);
+  const double r = rhs_point<false>(s, Q, P, QT, L, l, j, i, 0.0, (s.tau0 * s.wind_scale[l]) * s.wind_row[j]);
   const long e = l * s.plane + c;
   const double o = combine(s, in[c], s.qn ? s.qn[e] : 0.0, r);
   if (s.out) s.out[e] = o;
@@ -386,6 +385,79 @@ __global__ __launch_bounds__(256) void stage64_kernel(Stage64 s) {
       t = t + s.next.wl * o;
     }
     s.next.out[e] = s.next.y[e] + s.nh * t;
+  }
+}
+
+// One stage of a 16 x 16 tile.  The state (boundary condition applied), psi and the
+// beta rows are staged in LDS with the widest stencil's ring of 3, every load of
+// a thread before the first wait.  WENO-Z from memory waits once per branch of its
+// faces; Arakawa on larger planes reads every line nine times through L1.  A step,
+// us: WENO-Z 64^2 x 1 72.6 -> 68.0, 128^2 x 3 102 -> 92, 512^2 x 3 387 -> 362; Arakawa
+// 128^2 x 3 77.1 -> 76.1, 512^2 x 3 271 -> 257.
+constexpr int S64_TILE = 16, S64_HALO = 3, S64_PITCH = S64_TILE + 2 * S64_HALO;
+template <bool WENO>
+__global__ __launch_bounds__(256) void stage64_kernel(Stage64 s) {
+  __shared__ double stq[S64_PITCH * S64_PITCH], stp[S64_PITCH * S64_PITCH], stb[S64_PITCH];
+  const int l = blockIdx.y, Nx = s.Nx, Ny = s.Ny;
+  const int ntx = (Nx + S64_TILE - 1) / S64_TILE;
+  const int by = (int)blockIdx.x / ntx, bx = (int)blockIdx.x - by * ntx;
+  const int i0 = bx * S64_TILE - S64_HALO, j0 = by * S64_TILE - S64_HALO;
+  const int i = i0 + S64_HALO + (threadIdx.x & 15), j = j0 + S64_HALO + (threadIdx.x >> 4);
+  const bool live = i < Nx && j < Ny;
+  const long c = live ? (long)j * Nx + i : 0, e = l * s.plane + c;
+  const double* in = s.in + l * s.plane;
+  const double* psi = s.psi + l * s.plane;
+  double q[2], p[2];
+  int k[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    // (past the plane: its nearest cell, never read)
+    k[b] = min((int)threadIdx.x + 256 * b, S64_PITCH * S64_PITCH - 1);
+    const int y = min(max(j0 + k[b] / S64_PITCH, 0), Ny - 1), x = min(max(i0 + k[b] % S64_PITCH, 0), Nx - 1);
+    const bool g = y == 0 || y == Ny - 1 || x == 0 || x == Nx - 1;
+    q[b] = in[(long)y * Nx + x];
+    p[b] = psi[(long)y * Nx + x];
+    if (s.apply_bc && g) q[b] = 0.0;
+  }
+  const double beta = s.beta_row[min(max(j0 + min((int)threadIdx.x, S64_PITCH - 1), 0), Ny - 1)];
+  const double wind = (s.tau0 * s.wind_scale[l]) * s.wind_row[live ? j : 0];
+  const double inc = in[c], qnc = s.qn ? s.qn[e] : 0.0;
+  double t = 0.0, yc = 0.0;
+  if (s.next.out) {
+    yc = s.next.y[e];
+    if (s.next.nk) {
+      t = s.next.w[0] * s.next.k[0][e];
+      for (int m = 1; m < s.next.nk; ++m) t = t + s.next.w[m] * s.next.k[m][e];
+    }
+  }
+  double pw = 0.0;
+  if (WENO && s.alpha) {
+    pw = s.cm2l[l * s.nl] * s.alpha[0];
+    for (int m = 1; m < s.nl; ++m) pw = pw + s.cm2l[l * s.nl + m] * s.alpha[m];
+  }
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    stq[k[b]] = q[b];
+    stp[k[b]] = p[b];
+  }
+  if (threadIdx.x < S64_PITCH) stb[threadIdx.x] = beta;
+  __syncthreads();
+  if (!live) return;
+  // q with the boundary condition, and q + beta (y - y0) (total PV)
+  auto Q = [&](int jj, int ii) { return stq[(jj - j0) * S64_PITCH + ii - i0]; };
+  auto QT = [&](int jj, int ii) { return Q(jj, ii) + stb[jj - j0]; };
+  auto P = [&](int jj, int ii) { return stp[(jj - j0) * S64_PITCH + ii - i0]; };
+  // the inner Laplacian of the biharmonic term, recomputed at each neighbour
+  auto L = [&](int jj, int ii) {
+    const bool g = jj == 0 || jj == Ny - 1 || ii == 0 || ii == Nx - 1;
+    return g ? 0.0 : lap64(s, Q, jj, ii);
+  };
+  const double r = rhs_point<WENO>(s, Q, P, QT, L, l, j, i, pw, wind);
+  const double o = combine(s, inc, qnc, r);
+  if (s.out) s.out[e] = o;
+  if (s.next.out) {
+    t = s.next.nk ? t + s.next.wl * o : s.next.wl * o;
+    s.next.out[e] = yc + s.nh * t;
   }
 }
 
@@ -535,7 +607,11 @@ Stage64 stage_args(const Qg64& p, const double* in, const double* psi, const dou
 }
 
 void launch_stage(const Qg64& p, const Stage64& s, hipStream_t st) {
-  stage64_kernel<<<dim3(blocks(p.plane), p.nl), 256, 0, st>>>(s);
+  // Arakawa by tiles from 2^15 cells on: 64^2 x 3 (13068) loses 1-2%, 128^2 x 3 (50700) gains 1-2%
+  const unsigned tiles = (unsigned)(((p.Nx + S64_TILE - 1) / S64_TILE) * (long)((p.Ny + S64_TILE - 1) / S64_TILE));
+  if (s.advection == SOMAXHIP_ADV_WENO) stage64_kernel<true><<<dim3(tiles, p.nl), 256, 0, st>>>(s);
+  else if (p.plane * p.nl >= 32768) stage64_kernel<false><<<dim3(tiles, p.nl), 256, 0, st>>>(s);
+  else stage64_point_kernel<<<dim3(blocks(p.plane), p.nl), 256, 0, st>>>(s);
 }
 
 // dq = RHS of the BC-applied q (apply_bc) or of q as given

@@ -127,6 +127,28 @@ def test_fp64_rhs(gpu, advection, mass, nu):
     assert r < 1e-10 and r_raw < 1e-10
 
 
+# lines (n + 2) of 16, 17, 15 and 33 cells around the stage's 16 x 16 tiles and a
+# line shorter than the stencil; Arakawa on either side of 2^15 cells (32760 by
+# cells, 33072 and 33672 by tiles)
+@pytest.mark.parametrize("n,ny,nl,advection", [(14, 15, 2, "weno"), (13, 31, 1, "weno"), (47, 14, 3, "weno"),
+                                               (2, 20, 1, "weno"), (103, 102, 3, "arakawa"),
+                                               (104, 102, 3, "arakawa"), (181, 182, 1, "arakawa")])
+def test_fp64_stage_tiles(gpu, n, ny, nl, advection):
+    """RHS with and without the boundary condition and one step, bars as above."""
+    from somax_amd import BaroclinicQGState
+
+    _log(f"[fp64 stage tiles] {n}x{ny}x{nl} {advection}")
+    model, setup = _pair(n, nl=nl, ny=ny, advection=advection, mass_correction=True, lateral_viscosity=50.0)
+    q, qd = _state(model, seed=n, ghost_noise=True)
+    r = rel(model.build_terms()(0.0, BaroclinicQGState(q=qd)).q.cpu().numpy(), oqg.rhs(setup, oqg.apply_bc(q)))
+    r_raw = rel(model.vector_field(0.0, BaroclinicQGState(q=qd)).q.cpu().numpy(), oqg.rhs(setup, q))
+    q1 = qd.clone()
+    model._step_inplace(q1, 600.0, 1)
+    r1 = rel(q1.cpu().numpy(), oqg.ssprk3_step(setup, q, 600.0))
+    _log(f"  rel-L2 rhs {r:.3e}, without BC {r_raw:.3e}, step {r1:.3e}")
+    assert r < 1e-10 and r_raw < 1e-10 and r1 < 1e-12
+
+
 @pytest.mark.parametrize("advection,mass", [("arakawa", False), ("weno", True)])
 def test_fp64_ssprk3(gpu, advection, mass):
     """One and 100 SSP-RK3 steps of 1200 s at 64^2, three layers."""
