@@ -38,6 +38,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <limits>
 #include <memory>
 #include <new>
 #include <type_traits>
@@ -778,7 +779,9 @@ AxisTables axis_tables(int N, double d) {
   AxisTables t;
   t.f.assign(2 * (size_t)hp * hp, 0.0);
   t.g.assign(2 * (size_t)hp * hp, 0.0);
-  t.lam.assign(2 * (size_t)hp, -1.0 / (d * d));  // padded modes: any value that keeps the symbol away from 0
+  // padded modes: a symbol that no Helmholtz parameter, of either sign, brings to 0 (0 / 0
+  // there would reach every point through the next product)
+  t.lam.assign(2 * (size_t)hp, -std::numeric_limits<double>::infinity());
   t.c.assign(hp, 0.0);
   // S[n][k] = sqrt(2/(N+1)) sin(pi (n+1)(k+1)/(N+1)); angles reduced in
   // integers to [0, 2(N+1)), one sine per residue
