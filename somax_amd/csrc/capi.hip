@@ -248,47 +248,72 @@ struct Batch {
   int any_mass = 0;
   float* homsol = nullptr;
   double* hmean = nullptr;
-  // direct FP64 inversion (null: it does not pay, or a mixed ensemble class,
-  // which only ever takes SSP-RK3 steps)
+  // direct FP64 inversion (null: no call of the batch takes it)
   struct DirectDelete {
     void operator()(Direct* d) const { direct_destroy(d); }
   };
   std::unique_ptr<Direct, DirectDelete> direct;
+  bool direct_step = false, direct_state = false;  // which calls take it (use_direct)
 };
 
 // What an inversion is for decides its form (`use_direct`).
 enum class Solve {
-  STEP,   // a stage of an SSP-RK3 step
-  STATE,  // psi itself, a Tsit5 stage, a projection
+  STEP,   // a stage of an SSP-RK3 step: a model's or an ensemble member's
+  STATE,  // a model's psi itself, a Tsit5 stage, a projection
   FIELD,  // derivatives of psi are the result (tendency, diagnostics)
 };
 
-// Whether an inversion of batch `p` runs in its direct form: wherever the
-// batch has one (direct_pays), except
-//   * SSP-RK3 steps of the mixed form.  Ensembles take those in merged launch
-//     groups whose phases are the split-operand transforms, and a member's
-//     step equals its single model's bit for bit, so both keep them;
-//   * results that are derivatives of psi.  They carry psi's last bits
-//     amplified (1e-5 in a tendency, 1e-3 in a vorticity at 512^2), so any
-//     other order of sums moves them by that much; they keep the arithmetic
-//     that their stored references were made with.
+// Whether an inversion of batch `p` runs in its direct form.  Not the
+// derivatives of psi: they carry psi's last bits amplified (1e-5 of a
+// tendency, 1e-3 of a vorticity at 512^2), so the direct form's other order of
+// sums, though nearer to FP64, would move stored results of `rhs` and `diagnose`
+// by that much; and six products at 512^2 take 121 us by it, 84 by the stripes.
+// Their psi is therefore that of the split-operand transforms: within their
+// 1e-6 of the direct form's, not its bits.
 inline bool use_direct(const Batch& p, Solve what) {
-  return p.direct && what != Solve::FIELD && !(what == Solve::STEP && p.precision == SOMAXHIP_PREC_MIXED);
+  return p.direct && ((what == Solve::STEP && p.direct_step) || (what == Solve::STATE && p.direct_state));
 }
 
-// Whether the direct FP64 form is the faster inversion of P planes: the grid
-// has to fit, and its operations F (four products of the folded transforms)
-// have to stay below what the split-operand launches do in the time they take
-// at least.  Those cost 4 launches of one round of tiles each, whatever the
-// number of planes, until the tiles fill the chip; the direct form runs at the
-// FP64 rate from the start.  Measured (an SSP-RK3 step of 3-layer members, us,
-// split -> direct): FP32 64^2 x 4 265 -> 114, 128^2 x 64 634 -> 483, 256^2 x 8
-// 410 -> 330, 256^2 x 32 (F = 6.6e9) 939 -> 960, 512^2 x 2 (3.3e9) 516 -> 471,
-// 512^2 x 4 (6.5e9) 575 -> 772; six products on a grid past the stripes' (F up to
-// 1.8e9) 345 -> 314.  Where six products run as stripes (stripes -> direct): 64^2 x
-// 1 129 -> 107, 128^2 x 4 (1.1e8) 157 -> 123, 256^2 x 1 (2.1e8) 160 -> 163, 64^2 x
-// 96 (3.3e8) 247 -> 261, 320^2 x 1 (4.0e8) 179 -> 193, 256^2 x 4 (8.2e8) 200 -> 219,
-// 512^2 x 1 (1.6e9) 254 -> 292.
+// Whether the steps of a grid invert in the direct form: a rule of the grid and
+// the precision alone, so that a member's bits do not depend on what steps beside
+// it and equal its single model's.  Mixed steps never do: merged ensembles take
+// them by split-operand transforms.
+//
+// FP32.  The direct form runs at the FP64 rate, half of FP32's, and pays where it
+// does fewer operations (extents padded to 16) than the 128-wide tiles (folded
+// from 256 points on; past 128, one or two rows cost nothing), or where what counts is
+// the passes over the planes, below 2e8 operations a plane.  An SSP-RK3 step of
+// 3-layer members, us, transforms -> direct: 64^2 x 1 148 -> 74, x 256 672 -> 456;
+// 256^2 x 1 184 -> 137, x 45 1262 -> 1101; 400^2 (0.68 of the tiles' operations) x 1
+// 223 -> 202, x 18 1561 -> 1279; 430^2 (0.79) x 1 229 -> 217, x 16 1304 -> 1405; 512^2
+// (1.2) x 1 255 -> 252, x 11 1396 -> 1577; 511^2 (0.6) x 11 2034 -> 1580; 600^2 (0.63)
+// x 1 337 -> 296, x 8 1828 -> 1578; 512 x 256 (1.3) x 1 220 -> 186, x 22 1328 -> 1412.
+//
+// Six products.  Up to 1.25e7 operations a plane (144^2), stripes -> direct: 64^2 x 1
+// 102 -> 74, x 16 108 -> 97, x 300 445 -> 530; 96^2 x 1 109 -> 84, x 90 312 -> 338; 128^2 x 1
+// 128 -> 91, x 183 1149 -> 1108; 144^2 x 144 1088 -> 995; 20 x 500 x 83 951 -> 544. Past it
+// 160^2 x 117 1051 -> 1126, 192^2 x 1 139 -> 110, x 81 970 -> 1127; 256^2 x 1 135 -> 135,
+// x 12 329 -> 420.
+static bool direct_steps(int Nx, int Ny, int precision) {
+  if (!direct_fits(Nx, Ny) || precision == SOMAXHIP_PREC_MIXED) return false;
+  const int hx = (Nx + 1) / 2, hy = (Ny + 1) / 2;
+  auto operations = [](double x, double y, double k) { return 16.0 * x * y * k; };
+  if (precision == SOMAXHIP_PREC_BF16X6) return operations(hx, hy, hx + hy) <= 1.25e7;
+  const double px = round_up(hx, 16), py = round_up(hy, 16), direct = operations(px, py, px + py);
+  if (direct <= 2.0e8) return true;
+  const bool fold = use_fold(Nx, Ny);
+  const int ex = fold ? hx : Nx, ey = fold ? hy : Ny;
+  const GemmCut c = gemm_cut(ex, ey, std::max(ex, ey), 256);
+  const double tiles = operations(round_up(c.am, 128), round_up(c.bm, 128), ex + ey) * (fold ? 1.0 : 0.25);
+  return direct <= 0.75 * tiles;
+}
+
+// Whether the direct form is the faster inversion of a single model's P planes
+// (Solve::STATE; ensembles only step).  Its operations F have to stay below what
+// the split-operand launches do in the time they take at least: 4 launches of one
+// round of tiles each, whatever the number of planes, until the tiles fill the
+// chip.  Six products where the stripes fit, stripes -> direct as above: 256^2 x 3
+// (2.1e8) equal, 320^2 x 3 (4.0e8) 179 -> 193.
 static bool direct_pays(int Nx, int Ny, int P, int precision) {
   if (!direct_fits(Nx, Ny)) return false;
   const double hx = (Nx + 1) / 2, hy = (Ny + 1) / 2;
@@ -404,7 +429,9 @@ static hipError_t batch_build(Batch& b, const std::vector<const somaxhip_qg_desc
       (e = b.mem.upload(&dhp, hp)) != hipSuccess || (e = b.mem.upload(&dws, wscale)) != hipSuccess ||
       (e = b.mem.upload(&b.dbeta_rows, dbeta)) != hipSuccess || (e = b.mem.upload(&b.wind_rows, wind)) != hipSuccess)
     return e;
-  if (direct_pays(b.Nx, b.Ny, P, b.precision) && !(ensemble && b.precision == SOMAXHIP_PREC_MIXED)) {
+  b.direct_step = direct_steps(b.Nx, b.Ny, b.precision);
+  b.direct_state = !ensemble && direct_pays(b.Nx, b.Ny, P, b.precision);
+  if (b.direct_step || b.direct_state) {
     DirectDesc dd;
     dd.Nx = b.Nx;
     dd.Ny = b.Ny;

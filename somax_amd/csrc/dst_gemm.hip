@@ -1295,9 +1295,11 @@ int cu_count() {
 // FP32 one is not.  Measured, a right-hand side (us, 128 x 128 -> 64 x 64): FP32
 // 64^2 x 3 74 -> 43, 301^2 x 3 152 -> 74, 512^2 x 3 152 -> 80, 640^2 x 3 175 ->
 // 117; six products 301^2 x 3 96 -> 56, 512^2 x 3 102 -> 76; mixed 256^2 x 3
-// 105 -> 85, 512^2 x 3 140 -> 114.  Launches that share the chip with others
-// (classes of a concurrent ensemble) keep the denser tiles: a 32-member
-// ensemble's step took 743 against 654 us on small ones.
+// 105 -> 85, 512^2 x 3 140 -> 114.  bf16 launches that share the chip with others
+// (classes of a concurrent ensemble) keep the denser tiles: a 32-member mixed
+// ensemble's step took 743 against 654 us on small ones.  FP32 ones do not: beside
+// the direct form's launches, an FP32 class of two 512^2 members was the whole
+// ensemble's critical path (32 members 569 -> 397 us).
 //
 // The x1 / x3 transforms run on pair tiles when their 128 x 128 workgroups
 // (tiles and fringe) would take more than one round of the CUs: measured, the
@@ -1316,7 +1318,7 @@ Tiles pick_tiles(GemmArgs* a, int n, int max_np) {
     return b;
   };
   // (the FP32 small kernel always sums its windows in FP64)
-  if (a[0].alone && (!f32 || a[0].acc64))
+  if (f32 ? a[0].acc64 != 0 : a[0].alone != 0)
     for (int fdots = 64; fdots <= (f32 ? 256 : 128); fdots *= 2)
       if (total(Tiles::SMALL, fdots) <= 2 * cus) return Tiles::SMALL;
   return total(Tiles::WHOLE, 256) > cus && !f32 && max_np <= 3 ? Tiles::PAIR : Tiles::WHOLE;

@@ -7,12 +7,11 @@ counts and parameters -- steps as one ensemble: members sharing a grid,
 advection and precision form a class whose planes every kernel of the step
 covers in one launch; classes run concurrently on their own streams, and the
 step is captured as a hipGraph and replayed.  The arithmetic per member is
-that of ``model.step`` (FP32 and six-product classes of so many planes that
-their inversion leaves the direct FP64 form round differently, at 1e-8).
+that of ``model.step``, bit for bit, whatever steps beside it.
 
 With ``merged=True`` the classes are packed into launch groups (those
-sharing precision, advection, biharmonic flag and stage tile height, up to
-eight classes each): every kernel phase of a Runge-Kutta stage is then one
+sharing precision, the form of their inversion, advection, biharmonic flag and
+stage tile height, up to eight classes each): every kernel phase of a Runge-Kutta stage is then one
 launch over the whole group, whose blocks a work table assigns to the
 classes, instead of one launch per class.
 

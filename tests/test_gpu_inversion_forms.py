@@ -84,3 +84,63 @@ def test_negative_helmholtz_parameter(gpu, precision):
         r = rel(psi[p], dst.helmholtz_dst(q[p].astype(np.float64), d, d, lams[p]))
         print(f"[forms] lambda {lams[p] * d * d:+.0f} / dx^2, {precision}: rel-L2 {r:.2e}", flush=True)
         assert r < (1e-11 if plan.f64 else 1e-7)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "mixed", "bf16x6", "fp64"])
+@pytest.mark.parametrize("Nx,Ny", [(5, 4), (23, 50), (46, 33), (66, 67), (131, 67), (257, 40), (130, 130), (260, 262),
+                                   (303, 218), (514, 258)])
+def test_workspace_contents_do_not_matter(gpu, Nx, Ny, precision):
+    """An inversion and a right-hand side from a workspace of NaN equal those from one of
+    zeros, bit for bit: no form reads what it has not written."""
+    import torch
+
+    from somax_amd import _lib
+
+    lams = np.array([0.0, 3e-10])
+    plan = _Plan(Nx, Ny, 2e4, 3e4, lams, precision)
+    q = plan.tensor((np.random.default_rng(Nx + Ny).standard_normal((2, Ny, Nx)) * 1e-10).astype(np.float32))
+    prm = _lib.QGParams(15.0, 1e9, 3.6e-8, 0.0)
+    rhs = plan.lib.somaxhip_qg_rhs_f64 if plan.f64 else plan.lib.somaxhip_qg_rhs
+    outs = []
+    for byte in (0, 255):
+        ws = torch.full((plan.ws_bytes,), byte, dtype=torch.uint8, device="cuda")
+        psi, psi2, dq = (torch.empty_like(q) for _ in range(3))
+        inv = plan.lib.somaxhip_qg_invert_f64 if plan.f64 else plan.lib.somaxhip_qg_invert
+        for bc in (1, 0):
+            ws.fill_(byte)
+            _lib.check(inv(plan.plan, q.data_ptr(), psi.data_ptr(), bc, ws.data_ptr(), None), "invert")
+            ws.fill_(byte)
+            _lib.check(rhs(plan.plan, q.data_ptr(), dq.data_ptr(), psi2.data_ptr(), ctypes.byref(prm), bc,
+                           ws.data_ptr(), None), "rhs")
+            outs.append([psi.clone(), psi2.clone(), dq.clone()])
+    for a, b in zip(outs[:2], outs[2:]):
+        assert all(torch.isfinite(x).all() and torch.equal(x, y) for x, y in zip(a, b))
+
+
+# (precision, n, layers, members): grids whose steps invert in the direct form (256^2 FP32,
+# 64^2 and 144^2 six products, 511^2) and by the transforms (512^2, 192^2), with members
+# enough that the class leaves the launch shapes of a single model
+SIBLINGS = [("fp32", 256, 3, 33), ("fp32", 512, 3, 3), ("fp32", 511, 2, 5), ("fp32", 430, 1, 8), ("bf16x6", 64, 3, 30),
+            ("bf16x6", 144, 2, 14), ("bf16x6", 192, 3, 4), ("mixed", 200, 3, 5)]
+
+
+@pytest.mark.parametrize("merged", [False, True])
+@pytest.mark.parametrize("precision,n,nl,members", SIBLINGS)
+def test_member_bits_do_not_depend_on_siblings(gpu, precision, n, nl, members, merged):
+    """A member steps as its single model does, bit for bit, in a class of many planes
+    and beside a class of another grid."""
+    import torch
+
+    from somax_amd import QGEnsemble
+    from somax_amd import testcases as tc
+
+    models = [_member(n, n, nl, precision=precision)] * members + [_member(48, 40, 2, precision=precision)]
+    pv = [tc.random_pv(m, 7 + i).astype(np.float32) for i, m in enumerate((models[0], models[-1]))]
+    qs = [pv[0] * np.float32(1.0 + 0.01 * i) for i in range(members)] + [pv[1]]
+    ens = QGEnsemble(models, merged=merged)
+    packed = ens.pack(qs)
+    ens.step(packed, 600.0, 2)
+    for i in (0, members // 2, members - 1, members):
+        one = torch.from_numpy(qs[i]).cuda()
+        models[i]._step_inplace(one, 600.0, 2)
+        assert torch.equal(ens.member(packed, i), one.view(ens.shapes[i])), i
