@@ -6,6 +6,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <string>
 
 namespace somax {
@@ -19,6 +20,28 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 // Thread-local last error text for somaxhip_last_error().
 void set_error(const std::string& msg);
+
+// Host work that each device needs once (a kernel's attributes belong to the device
+// they are set on), from any number of threads; repeated until it succeeds.
+class OncePerDevice {
+ public:
+  template <class F>
+  hipError_t operator()(F prepare) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const std::lock_guard<std::mutex> lock(mu_);
+    const uint64_t bit = dev < 64 ? (uint64_t)1 << dev : 0;
+    if (done_ & bit) return hipSuccess;
+    e = prepare();
+    if (e == hipSuccess) done_ |= bit;
+    return e;
+  }
+
+ private:
+  std::mutex mu_;
+  uint64_t done_ = 0;
+};
 
 // Round-to-nearest-even float -> bf16 bits (finite inputs; NaN kept quiet).
 __host__ __device__ inline uint16_t f32_to_bf16_bits(float x) {

@@ -731,13 +731,13 @@ hipError_t prepare_kernels() {
   return e;
 }
 hipError_t prepare_direct() {
-  static hipError_t status = [] {
+  static OncePerDevice once;
+  return once([] {
     hipError_t e = prepare_kernels<float, 1>();
     if (e == hipSuccess) e = prepare_kernels<float, MAX_GROUP>();
     if (e == hipSuccess) e = prepare_kernels<double, 1>();
     return e;
-  }();
-  return status;
+  });
 }
 
 template <class R, int G>

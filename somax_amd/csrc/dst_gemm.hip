@@ -1246,7 +1246,8 @@ hipError_t prepare_np() {
 hipError_t prepare_dst_gemm() {
   // up to 144 KiB of the 160 KiB LDS of a gfx950 CU; set outside any stream
   // capture, before the first launch
-  static hipError_t status = [] {
+  static OncePerDevice once;
+  return once([] {
     hipError_t e = prepare_np<1, 1>();
     if (e == hipSuccess) e = prepare_np<3, 1>();
     if (e == hipSuccess) e = prepare_np<6, 1>();
@@ -1256,8 +1257,7 @@ hipError_t prepare_dst_gemm() {
     if (e == hipSuccess) e = raise(reinterpret_cast<const void*>(dst_gemm_f32_small_kernel<1>), F32_SMALL_LDS);
     if (e == hipSuccess) e = raise(reinterpret_cast<const void*>(dst_gemm_f32_small_kernel<MAX_GROUP>), F32_SMALL_LDS);
     return e;
-  }();
-  return status;
+  });
 }
 
 namespace {

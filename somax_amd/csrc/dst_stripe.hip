@@ -633,13 +633,13 @@ hipError_t launch_fragment_order(const uint16_t* src, uint16_t* dst, long rows, 
 }
 
 hipError_t prepare_dst_stripe() {
-  static hipError_t status = [] {
+  static OncePerDevice once;
+  return once([] {
     hipError_t e = raise<3, 1>();
     if (e == hipSuccess) e = raise<3, 6>();
     if (e == hipSuccess) e = raise<6, 6>();
     return e;
-  }();
-  return status;
+  });
 }
 
 bool dst_stripe_fits(const GemmArgs& f1, const GemmArgs& f2, const GemmArgs& i1) {
