@@ -116,7 +116,8 @@ typedef struct {
 int somaxhip_qg_plan_create(const somaxhip_qg_desc* desc, somaxhip_qg_plan* plan);
 int somaxhip_qg_plan_destroy(somaxhip_qg_plan plan);
 
-/* Bytes of caller-provided device workspace that the calls below need. */
+/* Bytes of caller-provided device workspace that the calls below need.  A
+ * workspace is aligned to 16 bytes; 8 do for a plan of precision FP32 or FP64. */
 size_t somaxhip_qg_workspace_bytes(somaxhip_qg_plan plan);
 
 /* psi = _invert_pv(q), or _invert_pv(apply_boundary_conditions(q)) when

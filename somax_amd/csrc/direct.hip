@@ -675,6 +675,9 @@ __global__ __launch_bounds__(256 * NMODE) void direct_inverse_kernel(DirectTable
 }
 
 constexpr int DIRECT_LDS = 157 * 1024;
+// The spectral kernel's loads into LDS take 16 bytes a lane; a caller's workspace
+// need not be aligned to more than a double.
+constexpr size_t DIRECT_ALIGN = 16;
 size_t forward_lds(const DirectArgs& a) {
   return (size_t)64 * direct_pitch(direct_k(a.hx, a.apply_bc)) * sizeof(double);
 }
@@ -835,7 +838,7 @@ bool direct_fits(int Nx, int Ny) {
 
 size_t direct_bytes(int Nx, int Ny, int P) {
   const size_t ntx = ((Nx + 1) / 2 + 15) / 16, nty = ((Ny + 1) / 2 + 15) / 16;
-  return ((size_t)P * 2 * 4 * 256 * ntx * nty + (size_t)P * ntx) * sizeof(double);
+  return ((size_t)P * 2 * 4 * 256 * ntx * nty + (size_t)P * ntx) * sizeof(double) + DIRECT_ALIGN;
 }
 
 void direct_destroy(Direct* d) { delete d; }
@@ -919,7 +922,8 @@ DirectArgs call_args(const DirectCall& c) {
   a.psi = c.psi;
   a.apply_bc = c.apply_bc ? 1 : 0;
   const size_t blocks = (size_t)a.P * 4 * 256 * a.ntx * a.nty;
-  a.T = static_cast<double*>(c.buf);
+  const uintptr_t at = reinterpret_cast<uintptr_t>(c.buf);
+  a.T = reinterpret_cast<double*>((at + DIRECT_ALIGN - 1) / DIRECT_ALIGN * DIRECT_ALIGN);
   a.V = a.T + blocks;
   a.partial = a.V + blocks;
   a.homsol = c.homsol;

@@ -1317,8 +1317,12 @@ Tiles pick_tiles(GemmArgs* a, int n, int max_np) {
     }
     return b;
   };
-  // (the FP32 small kernel always sums its windows in FP64)
-  if (f32 ? a[0].acc64 != 0 : a[0].alone != 0)
+  // (the FP32 small kernel always sums its windows in FP64, and loads 16 bytes a lane
+  // into LDS: from a workspace aligned to less the wide tiles, whose loads need 4)
+  bool small = f32 ? a[0].acc64 != 0 : a[0].alone != 0;
+  if (f32)
+    for (int i = 0; i < n; ++i) small = small && reinterpret_cast<uintptr_t>(a[i].Xf) % 16 == 0;
+  if (small)
     for (int fdots = 64; fdots <= (f32 ? 256 : 128); fdots *= 2)
       if (total(Tiles::SMALL, fdots) <= 2 * cus) return Tiles::SMALL;
   return total(Tiles::WHOLE, 256) > cus && !f32 && max_np <= 3 ? Tiles::PAIR : Tiles::WHOLE;

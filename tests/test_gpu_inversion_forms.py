@@ -117,6 +117,30 @@ def test_workspace_contents_do_not_matter(gpu, Nx, Ny, precision):
         assert all(torch.isfinite(x).all() and torch.equal(x, y) for x, y in zip(a, b))
 
 
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("Nx,Ny", [(34, 40), (131, 67), (258, 258), (303, 218), (514, 100)])
+def test_workspace_aligned_to_eight_bytes(gpu, Nx, Ny, precision):
+    """A workspace that starts 8 bytes past an allocation's start gives the bits of an
+    aligned one, in inversions and right-hand sides."""
+    import torch
+
+    from somax_amd import _lib
+
+    plan = _Plan(Nx, Ny, 2e4, 3e4, np.array([0.0, 3e-10]), precision)
+    q = plan.tensor((np.random.default_rng(Nx + Ny).standard_normal((2, Ny, Nx)) * 1e-10).astype(np.float32))
+    rhs = plan.lib.somaxhip_qg_rhs_f64 if plan.f64 else plan.lib.somaxhip_qg_rhs
+    prm = _lib.QGParams(15.0, 1e9, 3.6e-8, 0.0)
+    outs = []
+    for offset in (0, 8):
+        ws = torch.empty(plan.ws_bytes + 256, dtype=torch.uint8, device="cuda")
+        dq = torch.empty_like(q)
+        _lib.check(rhs(plan.plan, q.data_ptr(), dq.data_ptr(), None, ctypes.byref(prm), 1, ws.data_ptr() + offset,
+                       None), "rhs")
+        torch.cuda.synchronize()
+        outs.append((plan.invert(q, offset), dq))
+    assert all(torch.equal(x, y) for x, y in zip(*outs))
+
+
 # (precision, n, layers, members): grids whose steps invert in the direct form (256^2 FP32,
 # 64^2 and 144^2 six products, 511^2) and by the transforms (512^2, 192^2), with members
 # enough that the class leaves the launch shapes of a single model
