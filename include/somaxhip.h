@@ -47,7 +47,9 @@ enum {
 
 /* Arithmetic of the DST-I Helmholtz inversion. */
 enum {
-  SOMAXHIP_PREC_FP32 = 0,   /* plain: FP32 MFMA sine-transform GEMMs */
+  SOMAXHIP_PREC_FP32 = 0,   /* plain: FP32 MFMA sine-transform GEMMs with FP64 windows, or, in the
+                               inversions of steps, Tsit5, projections and somaxhip_qg_invert on
+                               grids where it is faster, FP64 throughout (the direct form) */
   SOMAXHIP_PREC_MIXED = 1,  /* BF16 hi/lo 3-product MFMA, FP32 accumulate, one
                                iterative-refinement pass on the Helmholtz residual */
   SOMAXHIP_PREC_BF16X6 = 2, /* extension: BF16 hi/mid/lo three-piece operands, six
@@ -141,7 +143,14 @@ int somaxhip_qg_rhs(somaxhip_qg_plan plan, const float* q, float* dq, float* psi
  * laplacian(psi) (u, v, zeta nullable); ke_enstrophy (device, 2*nl doubles)
  * receives per layer the kinetic energy 0.5 sum (uT^2 + vT^2) dx dy and the
  * enstrophy 0.5 sum q^2 dx dy over the interior, summed in FP64 in a fixed
- * order. */
+ * order.
+ *
+ * The inversions of somaxhip_qg_rhs and _diagnose are the transforms of the
+ * plan's precision on every grid; those of somaxhip_qg_invert and the steps may
+ * take the direct FP64 form instead.  Both are within 1e-6 of the FP64 result
+ * (2-norm; the direct form 1e-7), and psi of the same q may differ by as much
+ * between them; a tendency or a vorticity amplifies that to about 1e-5 and 1e-3
+ * at 512 x 512.  FP64 plans have one form. */
 int somaxhip_qg_diagnose(somaxhip_qg_plan plan, const float* q, float* psi, float* u, float* v, float* zeta,
                          double* ke_enstrophy, void* workspace, somaxhip_stream_t stream);
 
@@ -149,9 +158,10 @@ int somaxhip_qg_diagnose(somaxhip_qg_plan plan, const float* q, float* psi, floa
  * (core/model.py:75, diffrax.Tsit5 with ConstantStepSize).  Advances q in
  * place by nsteps steps of dt with the boundary condition applied before
  * every RHS; six RHS evaluations per step (first same as last), each an
- * inversion plus the fused RHS kernel.  tsit5_workspace: a second caller
- * buffer of somaxhip_qg_tsit5_workspace_bytes (stage state and the seven
- * stage derivatives). */
+ * inversion plus the fused RHS kernel, which also forms the next stage's
+ * state.  tsit5_workspace: a second caller buffer of
+ * somaxhip_qg_tsit5_workspace_bytes (eight states, of which five stage
+ * derivatives and two stage states are used). */
 size_t somaxhip_qg_tsit5_workspace_bytes(somaxhip_qg_plan plan);
 int somaxhip_qg_step_tsit5(somaxhip_qg_plan plan, float* q, int nsteps, double dt, const somaxhip_qg_params* params,
                            void* workspace, void* tsit5_workspace, somaxhip_stream_t stream);

@@ -9,7 +9,8 @@ field names, ``create()`` keyword arguments and defaults, and the
 
 Extensions beyond the reference (keyword-only, defaults reproduce the
 reference): ``biharmonic_viscosity``, ``advection="weno"``,
-``precision`` (``"fp32"``: FP32 MFMA transforms; ``"mixed"``: bf16 hi/lo
+``precision`` (``"fp32"``: FP32 MFMA transforms, or an FP64 inversion on grids
+where that is faster; ``"mixed"``: bf16 hi/lo
 three-product transforms plus one refinement pass on the Helmholtz residual;
 ``"bf16x6"``: bf16 hi/mid/lo six-product transforms with FP64 accumulation,
 one direct solve; ``"fp64"``: the whole step in FP64 on float64 state, as the
@@ -362,7 +363,9 @@ class _QGBase(SomaxModel):
         return self._state_cls(q=self._zero_ghost(state.q).reshape(state.q.shape))
 
     def vector_field(self, t: float, state, args=None):
-        """``dq/dt`` on the given state as is (baroclinic.py:161-190)."""
+        """``dq/dt`` on the given state as is (baroclinic.py:161-190), from the transforms
+        of the model's precision; a step may invert in the direct FP64 form, whose
+        tendency differs by the transforms' rounding."""
         return self._state_cls(q=self._rhs(state.q, apply_bc=False).reshape(state.q.shape))
 
     def build_terms(self):
@@ -475,7 +478,9 @@ class BaroclinicQG(_QGBase):
 
     def diagnose(self, state) -> BaroclinicQGDiagnostics:
         """baroclinic.py:197-228: psi, geostrophic velocities on V / U faces,
-        kinetic energy and enstrophy per layer (FP64 sums), relative vorticity."""
+        kinetic energy and enstrophy per layer (FP64 sums), relative vorticity.
+        psi is within 1e-6 of the FP64 inversion, as ``_invert_pv``'s, which may come
+        from the direct FP64 form and then differs from it by as much."""
         torch = _torch()
         psi, u, v, zeta, ke, ens = self._diagnose(state.q)
         shape = (self._nl, self.grid.Ny, self.grid.Nx)
