@@ -12,11 +12,12 @@
 // GFLOP, and what costs time is the number of launches and the chain inside
 // each, not the matrix rate.  FP64 needs no split operands, no refinement
 // solve and no flushes, and three launches replace 6 (FP32, six-product) or
-// 12 (mixed).  Measured (us, one inversion; FP32 split -> direct): 64^2 x 1
-// 64 -> 12, 128^2 x 3 95 -> 19, 256^2 x 3 100 -> 34, 512^2 x 3 144 -> 72.  Per
+// 12 (mixed).  Measured (us, one inversion in a replayed graph; FP32 transforms of
+// 128 x 128 tiles -> direct): 64^2 x 1 62 -> 10.7, 128^2 x 3 93 -> 18.2, 256^2 x 3
+// 98 -> 33.5, 512^2 x 3 143 -> 72 (64 x 64 tiles: about as fast).  Per
 // launch at 64^2: 5 to 7 us, of which 1.5 are a launch's own and each dependent trip
 // to the Infinity Cache is 1 (the L2s start a kernel empty); at 512^2 x 3:
-// forward 21, spectral 30, inverse 23, against 5.6, 11.2 and 5.6 at the FP64
+// forward 21, spectral 30, inverse 24, against 5.6, 11.2 and 5.6 at the FP64
 // matrix rate (the 257th row of every folded extent costs a tile of 16, and 204
 // spectral workgroups leave a fifth of the chip idle).
 //
@@ -688,10 +689,10 @@ size_t front_lds(const DirectArgs& a) {
 // saves more than its repeated folds cost.  A workgroup loads rows x row x layers
 // points four times (rows of at least 32 points: shorter ones cost as much).
 // us of an inversion in a replayed graph, two launches -> one: 16^2 x 1 10.5 -> 8.3,
-// 64^2 x 1 12.3 -> 10.5, 64^2 x 7 21.4 -> 19.9, 128^2 x 2 (8064) 14.9 -> 14.3; but 128^2 x 3
-// (12096) 16.0 -> 17.3, 30 x 120 x 6 (11520) 19.2 -> 19.6.  Up to 64 points a side
-// every wave has at most one tile and its ring holds the tile's whole stream (160^2
-// x 1: 16.8 -> 18.2).  And one workgroup per CU, as a full chip pays for every
+// 64^2 x 1 12.3 -> 10.5, 64^2 x 7 21.4 -> 19.9, 126^2 x 2 (8064) 14.9 -> 14.3; but 126^2 x 3
+// (12096) 16.0 -> 17.3, 30 x 120 x 6 (11520) 19.2 -> 19.6.  Up to 64 points a side every wave has at most one
+// tile, and its ring holds the tile's whole stream or, at 65 folded points, all but
+// the last step (160^2 x 1: 16.8 -> 18.2).  And one workgroup per CU, as a full chip pays for every
 // repeat (steps of ensembles: 64^2, 240 workgroups 98 -> 93, 288 108 -> 120; 32^2, 192
 // 103 -> 95, 384 104 -> 112).
 bool direct_front(const DirectArgs& a) {

@@ -473,7 +473,7 @@ namespace somax {
 // Direct FP64 inversion of one batch (direct.hip): psi = Cm2l (lap_h -
 // lambda)^-1 Cl2m q with every sum and intermediate in FP64, three launches.
 // Folded extents up to DIRECT_MAX_H: the forward kernel's four parity rows
-// (64 rows of LDS, one double per folded point) end at 157 KiB of the 160.
+// (64 rows of LDS, one double per folded point) take 153 KiB of the 160 there.
 constexpr int DIRECT_MAX_H = 304;
 struct Direct;
 struct DirectDesc {
