@@ -1107,8 +1107,8 @@ DirectCall direct_call(const Batch& p, const float* q, float* psi, void* ws, boo
 
 // Phases of the direct inversion as the profile names them; `folded` is the
 // number of points of all planes, mults the products of one 1-D transform.
-DirectPhase direct_phases(double points, double mults, hipStream_t st) {
-  return [=](int k, const std::function<void()>& launch) {
+auto direct_phases(double points, double mults, hipStream_t st) {
+  return [=](int k, FunctionRef<void()> launch) {
     static const char* const names[4] = {"direct_forward", "direct_spectral", "direct_inverse", "direct_front"};
     static const double products[4] = {1.0, 2.0, 1.0, 3.0}, bytes[4] = {12.0, 16.0, 12.0, 12.0};
     ProfScope ps(names[k], 2.0 * mults * products[k], bytes[k] * points, st);

@@ -6,7 +6,7 @@
 // the member and plane tables below.  A single model is the one-member batch.
 #pragma once
 
-#include <functional>
+#include <type_traits>
 #include <vector>
 
 #include "somaxhip.h"
@@ -499,9 +499,25 @@ struct DirectCall {
   float* psi_wall;     // nullable: wall psi per plane
   double* alpha;       // nullable: multiplier per plane
 };
+// A callable passed down a call, by reference (a std::function would copy it to the
+// heap on every inversion).
+template <class S>
+class FunctionRef;
+template <class... A>
+class FunctionRef<void(A...)> {
+ public:
+  template <class F, class = std::enable_if_t<!std::is_same<std::decay_t<F>, FunctionRef>::value>>
+  FunctionRef(const F& f)
+      : f_(&f), call_([](const void* g, A... a) { (*static_cast<const F*>(g))(a...); }) {}
+  void operator()(A... a) const { call_(f_, a...); }
+
+ private:
+  const void* f_;
+  void (*call_)(const void*, A...);
+};
 // phase(k, launch) calls launch() for kernel k of the three, 3 for the first two
 // in one (timing hooks).
-using DirectPhase = std::function<void(int, const std::function<void()>&)>;
+using DirectPhase = FunctionRef<void(int, FunctionRef<void()>)>;
 void launch_direct(const DirectCall& c, hipStream_t st, const DirectPhase& phase);
 void launch_direct_group(const DirectCall* c, int n, hipStream_t st, const DirectPhase& phase);  // n <= MAX_GROUP
 

@@ -567,7 +567,7 @@ void invert(const Qg64& p, const double* q, double* psi, void* ws, bool apply_bc
       c.hmean = p.hmean;
       c.alpha = alpha;
     }
-    launch_direct(c, st, [](int, const std::function<void()>& launch) { launch(); });
+    launch_direct(c, st, [](int, FunctionRef<void()> launch) { launch(); });
     return;
   }
   const unsigned nb = blocks(p.plane);

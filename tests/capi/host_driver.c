@@ -6,9 +6,10 @@
  *   host_driver LIB nx ny nl precision
  *
  * creates a plan on device 0 and one on device 1, runs an inversion, a right-hand side
- * and a step on device 1, and prints "workspace BYTES", "launches N" and "refused N":
- * the launches on a device that ask for more than the 64 KiB of dynamic LDS that a
- * kernel has unless hipFuncSetAttribute raised it there. */
+ * and a step on device 1, and prints "workspace BYTES", "launches N", "refused N" (the
+ * launches on a device that ask for more than the 64 KiB of dynamic LDS that a
+ * kernel has unless hipFuncSetAttribute raised it there) and "allocations N" (C++
+ * allocations of the three calls). */
 #include <dlfcn.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -20,7 +21,7 @@ typedef struct {
   unsigned x, y, z;
 } grid3;
 
-static int device, launches, refused;
+static int device, launches, refused, allocations;
 static struct {
   const void* f;
   int device, bytes;
@@ -89,6 +90,13 @@ int hipGetSymbolAddress(void** p, const void* s) {
   *p = scratch;
   return 0;
 }
+/* operator new and delete */
+void* _Znwm(size_t n) {
+  ++allocations;
+  return malloc(n);
+}
+void _ZdlPv(void* p) { free(p); }
+void _ZdlPvm(void* p, size_t n) { free(p); }
 int hipGetLastError(void) { return 0; }
 const char* hipGetErrorString(int e) { return "error"; }
 int hipStreamSynchronize(void* s) { return 0; }
@@ -127,12 +135,13 @@ int main(int argc, char** argv) {
   for (device = 0; device < 2; ++device)
     if (create(&d, &plan[device])) return 3;
   device = 1;
-  launches = refused = 0;
+  launches = refused = allocations = 0;
   const somaxhip_qg_params prm = {1.0, 0.0, 0.0, 0.0};
   static double q[1];  /* no launch reads memory */
   if (invert(plan[1], q, q + 1, 0, q, NULL) || rhs(plan[1], q, q + 1, NULL, &prm, 1, q, NULL) ||
       step(plan[1], q, NULL, 1, 1.0, &prm, q, NULL))
     return 4;
-  printf("workspace %zu\nlaunches %d\nrefused %d\n", bytes(plan[1]), launches, refused);
+  printf("workspace %zu\nlaunches %d\nrefused %d\nallocations %d\n", bytes(plan[1]), launches, refused,
+         allocations);
   return 0;
 }

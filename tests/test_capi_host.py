@@ -38,3 +38,10 @@ def test_second_device_has_its_lds_limits_raised(driver, n, precision):
     out = driver(n, n, 3, precision)
     assert out["launches"] >= 14
     assert out["refused"] == 0
+
+
+@pytest.mark.parametrize("precision", sorted(PRECISION))
+@pytest.mark.parametrize("n", [30, 130, 512])
+def test_calls_allocate_no_host_memory(driver, n, precision):
+    """An inversion, a right-hand side and a step allocate nothing on the host."""
+    assert driver(n, n, 3, precision)["allocations"] == 0
